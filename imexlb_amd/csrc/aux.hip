@@ -20,11 +20,12 @@ __device__ __forceinline__ double feq_f64(int i, double p, double u, double v, d
 }
 
 // Population f of direction i (weight class of slot `slot`, which is i or
-// bb(i)) in the stored convention, g = f - s with s the direction's shift.
+// bb(i)) of cell p of plane z in the stored convention, g = f - s with s the
+// direction's shift.
 template <typename S>
-__device__ __forceinline__ void put(S *lat, uint64_t ps, int slot, uint32_t c, double f, double s)
+__device__ __forceinline__ void put(S *lat, const LatGeom &g, int slot, uint32_t z, uint32_t c, double f, double s)
 {
-    S *p = lat + (uint64_t)slot * ps + c;
+    S *p = lat + g.off(slot, z, c);
     if constexpr (std::is_same<S, double>::value)
         *p = f;
     else if constexpr (std::is_same<S, float>::value)
@@ -34,9 +35,9 @@ __device__ __forceinline__ void put(S *lat, uint64_t ps, int slot, uint32_t c, d
 }
 
 template <typename S>
-__device__ __forceinline__ double get(const S *lat, uint64_t ps, int slot, uint32_t c, double s)
+__device__ __forceinline__ double get(const S *lat, const LatGeom &g, int slot, uint32_t z, uint32_t c, double s)
 {
-    const S *p = lat + (uint64_t)slot * ps + c;
+    const S *p = lat + g.off(slot, z, c);
     if constexpr (std::is_same<S, double>::value)
         return *p;
     else if constexpr (std::is_same<S, float>::value)
@@ -95,7 +96,7 @@ __global__ void k_init(const InitParams P)
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
         const double f = feq_f64(i, p, u, v, w);
-        put<S>(lat, P.pstride, P.layout == 1 ? BB[i] : i, c, f, P.sh[i]);
+        put<S>(lat, P.geom, P.layout == 1 ? BB[i] : i, z, y * P.nx + x, f, P.sh[i]);
     }
     // the fields themselves are the moments of step 0, as the reference's
     // Initialize leaves them in p, ua, va, wa; a solid cell reports a fluid at
@@ -118,31 +119,22 @@ hipError_t launch_init(int dtype, const InitParams &P, hipStream_t st)
     return hipGetLastError();
 }
 
-// Lattice slot holding f*_i(x) for each storage layout.
-__device__ __forceinline__ void slot_of(const XferParams &P, int i, uint32_t c, int &slot, uint32_t &cell)
+// Lattice slot and cell (plane, cell of the plane) holding f*_i of cell
+// (x, y, z) for each storage layout.
+__device__ __forceinline__ void slot_of(const XferParams &P, int i, int x, int y, int z, int &slot, uint32_t &plane,
+                                        uint32_t &cell)
 {
     const uint32_t nx = P.nx, ny = P.ny, nz = P.nz;
-    if (P.layout == 0) {
-        slot = i;
-        cell = c;
-        return;
-    }
-    if (P.layout == 1) {
-        slot = BB[i];
-        cell = c;
-        return;
-    }
+    slot = P.layout == 1 ? BB[i] : i;
+    plane = (uint32_t)z;
+    cell = (uint32_t)y * nx + (uint32_t)x;
+    if (P.layout < 2) return;
     // streamed (AA after an odd step): f*_i(x) sits at x + e_i in slot i, or
     // at x in slot bb(i) when x + e_i is a cavity wall
-    const uint32_t t = P.divx.div(c);
-    int x = (int)(c - t * nx);
-    const uint32_t zz = P.divy.div(t);
-    int y = (int)(t - zz * ny), z = (int)zz;
     int xd = x + EX[i], yd = y + EY[i], zd = z + EZ[i];
     if (P.bc == BC_CAVITY) {
         if (xd < 0 || xd >= (int)nx || yd < 0 || yd >= (int)ny || zd < 0 || zd >= (int)nz) {
             slot = BB[i];
-            cell = c;
             return;
         }
     } else {
@@ -150,8 +142,8 @@ __device__ __forceinline__ void slot_of(const XferParams &P, int i, uint32_t c, 
         yd = yd < 0 ? yd + (int)ny : (yd >= (int)ny ? yd - (int)ny : yd);
         zd = zd < 0 ? zd + (int)nz : (zd >= (int)nz ? zd - (int)nz : zd);
     }
-    slot = i;
-    cell = ((uint32_t)zd * ny + (uint32_t)yd) * nx + (uint32_t)xd;
+    plane = (uint32_t)zd;
+    cell = (uint32_t)yd * nx + (uint32_t)xd;
 }
 
 template <typename S>
@@ -159,16 +151,18 @@ __global__ void k_get_f(const XferParams P)
 {
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= P.ncell) return;
+    const uint32_t t = P.divx.div(c), z = P.divy.div(t);
+    const int x = (int)(c - t * P.nx), y = (int)(t - z * P.ny);
     const S *lat = (const S *)P.lat;
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
         int slot;
-        uint32_t cell;
-        slot_of(P, i, c, slot, cell);
+        uint32_t plane, cell;
+        slot_of(P, i, x, y, (int)z, slot, plane, cell);
         double v = 0.0;
         // slot is i or bb(i); both share the weight class of i
-        if (slot == i) v = get<S>(lat, P.pstride, i, cell, P.sh[i]);
-        else v = get<S>(lat, P.pstride, BB[i], cell, P.sh[i]);
+        if (slot == i) v = get<S>(lat, P.geom, i, plane, cell, P.sh[i]);
+        else v = get<S>(lat, P.geom, BB[i], plane, cell, P.sh[i]);
         P.buf[(uint64_t)i * P.ncell + c] = v;
     }
 }
@@ -178,15 +172,17 @@ __global__ void k_set_f(const XferParams P)
 {
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= P.ncell) return;
+    const uint32_t t = P.divx.div(c), z = P.divy.div(t);
+    const int x = (int)(c - t * P.nx), y = (int)(t - z * P.ny);
     S *lat = (S *)P.lat;
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
         int slot;
-        uint32_t cell;
-        slot_of(P, i, c, slot, cell);
+        uint32_t plane, cell;
+        slot_of(P, i, x, y, (int)z, slot, plane, cell);
         const double v = P.buf[(uint64_t)i * P.ncell + c];
-        if (slot == i) put<S>(lat, P.pstride, i, cell, v, P.sh[i]);
-        else put<S>(lat, P.pstride, BB[i], cell, v, P.sh[i]);
+        if (slot == i) put<S>(lat, P.geom, i, plane, cell, v, P.sh[i]);
+        else put<S>(lat, P.geom, BB[i], plane, cell, v, P.sh[i]);
     }
 }
 
@@ -301,7 +297,7 @@ __global__ void __launch_bounds__(256) k_force_pass1(const FusedParams P, double
             zd = zd < 0 ? zd + P.nz : (zd >= P.nz ? zd - P.nz : zd);
             const uint32_t cd = ((uint32_t)zd * P.ny + (uint32_t)yd) * P.nx + (uint32_t)xd;
             if (P.mask[cd] != 1) continue;
-            const double f = 2.0 * get<S>(lat, P.pstride, i, c, P.sh[i]);
+            const double f = 2.0 * get<S>(lat, P.geom, i, zz, (uint32_t)y * P.nx + (uint32_t)x, P.sh[i]);
             acc[0] += f * (double)EX[i];
             acc[1] += f * (double)EY[i];
             acc[2] += f * (double)EZ[i];
@@ -512,8 +508,8 @@ __device__ __forceinline__ GhostSrc faithful_src(const FusedParams &P, int q, in
     g.is_deep = r == -1;
     g.deep = 0.0;
     if (g.is_deep && P.faithful_sphere) g.deep = faithful_sphere_f0(P, P.seed, q, i, j, k);
-    const uint64_t in_cell = r == -2 ? ((uint64_t)k * P.ny + j) * P.nx + i : 0;
-    g.p = r == -2 ? (const double *)P.src + (uint64_t)q * P.pstride + in_cell
+    const uint64_t in_cell = r == -2 ? P.geom.off(q, (uint32_t)k, (uint32_t)j * P.nx + i) : 0;
+    g.p = r == -2 ? (const double *)P.src + in_cell
                   : P.ring + (uint64_t)q * P.ring_n + (uint64_t)(r < 0 ? 0 : r);
     return g;
 }
@@ -664,7 +660,8 @@ __global__ void k_faithful_stage_fill(const FusedParams P)
         q = side == 0 ? nth_dir<0, -1>(r) : nth_dir<0, 1>(r);
         x = side == 0 ? 1u : (uint32_t)P.nx - 2u;
     }
-    P.stage[t] = ((const double *)P.src)[(uint64_t)q * P.pstride + yz * P.nx + x];
+    const uint32_t z = (uint32_t)(yz / P.ny), y = (uint32_t)(yz - (uint64_t)z * P.ny);
+    P.stage[t] = ((const double *)P.src)[P.geom.off(q, z, y * P.nx + x)];
 }
 
 hipError_t launch_faithful_stage_fill(const FusedParams &P, hipStream_t st)
@@ -758,7 +755,7 @@ __global__ void k_faithful_usr(const FusedParams P, int lo, int n)
     v = g.is_deep ? g.deep : v;
     const bool solid = valid & (mc == 1);
     const bool nb_solid = in ? m == 1 : faithful_sphere_solid(P.nx, xi, yi, zi);
-    if (solid & !nb_solid) ((double *)P.src)[(uint64_t)q * P.pstride + c] = v;
+    if (solid & !nb_solid) ((double *)P.src)[P.geom.off(q, (uint32_t)z, (uint32_t)y * P.nx + x)] = v;
 }
 
 hipError_t launch_faithful_boundaries(const FusedParams &P, hipStream_t st)

@@ -35,7 +35,9 @@ struct imexlb_handle {
     double *partials = nullptr;
     double *result = nullptr;  // device scratch for reductions (4 doubles)
     int nparts = 1024;
-    uint64_t pstride = 0;
+    uint64_t pstride = 0;    // structure of arrays: elements between populations
+    LatGeom geom{};          // the lattices' layout
+    size_t lat_bytes = 0;    // one lattice
     uint32_t ncell = 0;
     size_t elem = 8;
     double shift = 0.0;      // S: FP32/FP16 lattices store f - s_i with sum_i s_i = S
@@ -194,6 +196,7 @@ static void fill_fused_params(imexlb_handle *h, FusedParams &P, int src, int dst
     P.nz = c.nz;
     P.ncell = h->ncell;
     P.pstride = h->pstride;
+    P.geom = h->geom;
     P.src = h->lat[src];
     P.dst = h->lat[dst];
     P.mask = h->mask;
@@ -379,7 +382,11 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
         const int pad = c.stride_pad < 0 ? IMEXLB_DEFAULT_PAD : c.stride_pad;
         h->pstride = ((uint64_t)h->ncell + per - 1) / per * per + (uint64_t)pad / h->elem;
     }
-    h->block = c.block ? c.block : 256;
+    // plane tiles unless the caller asks for a stride or an address mode of the
+    // structure of arrays (imexlb_config.stride_pad, addr_mode)
+    h->geom = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
+    if (c.stride_pad < 0 && c.addr_mode < 0) tile_geom((uint32_t)c.nx, (uint32_t)c.ny, h->elem, h->geom);
+    h->block = c.block ? c.block : (h->geom.tl == 31 ? 256 : tile_block((uint64_t)c.nx * c.ny));
     h->cpt = c.cells_per_thread ? c.cells_per_thread : 1;
     h->xcd = c.xcd_remap < 0 ? 1 : c.xcd_remap;
     h->ntl = c.nt_loads < 0 ? 1 : (c.nt_loads ? 1 : 0);
@@ -390,13 +397,27 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
         if (c.case_id == IMEXLB_CASE_SPHERE && c.mode == IMEXLB_MODE_CONFIG) h->ush = c.u0;
         storage_shift(h->shift, h->ush, h->sh);
     }
-    const size_t lat_bytes = (size_t)Q * h->pstride * h->elem;
     const int nlat = c.storage == IMEXLB_PULL ? 2 : 1;
-    for (int k = 0; k < nlat; ++k) {
-        if (hipMalloc(&h->lat[k], lat_bytes) != hipSuccess)
-            return bail(fail(h, IMEXLB_ENOMEM, "lattice of %zu bytes", lat_bytes));
-        h->device_bytes += lat_bytes;
+    auto alloc_lattices = [&]() {
+        h->lat_bytes = (size_t)(lattice_elems(h->geom, (uint32_t)c.nz) * h->elem);
+        for (int k = 0; k < nlat; ++k)
+            if (hipMalloc(&h->lat[k], h->lat_bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                for (auto &p : h->lat)
+                    if (p) hipFree(p);
+                h->lat[0] = h->lat[1] = nullptr;
+                return false;
+            }
+        return true;
+    };
+    bool have = alloc_lattices();
+    if (!have && h->geom.tl != 31) {  // tiles round the planes up: arrays may still fit
+        h->geom = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
+        h->block = c.block ? c.block : 256;
+        have = alloc_lattices();
     }
+    if (!have) return bail(fail(h, IMEXLB_ENOMEM, "lattice of %zu bytes", h->lat_bytes));
+    h->device_bytes += (int64_t)nlat * (int64_t)h->lat_bytes;
     for (int k = 0; k < 4; ++k) {
         if (hipMalloc(&h->mom[k], (size_t)h->ncell * 8) != hipSuccess)
             return bail(fail(h, IMEXLB_ENOMEM, "moments"));
@@ -545,7 +566,7 @@ int imexlb_initialize(imexlb_handle *h)
     P.ny = c.ny;
     P.nz = c.nz;
     P.ncell = h->ncell;
-    P.pstride = h->pstride;
+    P.geom = h->geom;
     P.dst = h->lat[0];
     P.layout = c.storage == IMEXLB_AA ? 1 : 0;
     P.kind = c.case_id == IMEXLB_CASE_TGV ? 0 : (bc_of(c) == BC_FAITHFUL && c.case_id == IMEXLB_CASE_SPHERE ? 2 : 1);
@@ -572,8 +593,7 @@ int imexlb_initialize(imexlb_handle *h)
     if (c.storage == IMEXLB_PULL && c.case_id == IMEXLB_CASE_SPHERE) {
         // solid cells are never written by the step; give both lattices the
         // same initial contents
-        HIPCHK(h, hipMemcpyAsync(h->lat[1], h->lat[0], (size_t)Q * h->pstride * h->elem, hipMemcpyDeviceToDevice,
-                                 h->stream));
+        HIPCHK(h, hipMemcpyAsync(h->lat[1], h->lat[0], h->lat_bytes, hipMemcpyDeviceToDevice, h->stream));
     }
     h->steps = 0;
     h->mom_step = 0;  // k_init wrote the initial fields
@@ -736,7 +756,7 @@ static int xfer(imexlb_handle *h, double *host, bool get)
     P.ny = c.ny;
     P.nz = c.nz;
     P.ncell = h->ncell;
-    P.pstride = h->pstride;
+    P.geom = h->geom;
     std::memcpy(P.sh, h->sh, sizeof P.sh);
     P.bc = bc_of(c);
     std::memcpy(P.corr, h->corr, sizeof P.corr);
@@ -948,7 +968,9 @@ int imexlb_get_info(imexlb_handle *h, imexlb_info *info)
     info->xcd_remap = h->xcd;
     info->nt_loads = h->ntl;
     info->addr_mode = h->ph ? -1 : fused_addr_mode(h->elem, h->pstride, c.addr_mode < 0 ? 2 : c.addr_mode);
-    info->cells_per_thread = h->ph ? h->cpt : fused_cells_per_thread(h->cpt, bc_of(c), (uint32_t)c.nx, info->addr_mode);
+    info->cells_per_thread = h->ph                  ? h->cpt
+                             : h->geom.tl != 31 ? (h->cpt == 2 ? 2 : 1)
+                                                : fused_cells_per_thread(h->cpt, bc_of(c), (uint32_t)c.nx, info->addr_mode);
     return IMEXLB_OK;
 }
 
@@ -982,7 +1004,8 @@ int imexlb_autotune(imexlb_handle *h, const char *cache_path, int steps, int32_t
         // grouped bases: address mode 2); elsewhere they would time the
         // one-cell kernel again
         const int am = fused_addr_mode(h->elem, h->pstride, c.addr_mode < 0 ? 2 : c.addr_mode);
-        const int max_cpt = fused_cells_per_thread(3, bc_of(c), (uint32_t)c.nx, am) == 3 ? 3 : 2;
+        const int max_cpt =
+            h->geom.tl == 31 && fused_cells_per_thread(3, bc_of(c), (uint32_t)c.nx, am) == 3 ? 3 : 2;
         for (int b : blocks)
             for (int cpt = 1; cpt <= max_cpt; ++cpt)
                 for (int xcd = 0; xcd <= 1; ++xcd)
@@ -1045,7 +1068,7 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
     if (rc) return rc;
     if (steps < 2) steps = 2;
     steps += steps & 1;  // whole AA periods
-    const size_t lat_bytes = (size_t)Q * h->pstride * h->elem;
+    const size_t lat_bytes = h->lat_bytes;
     const int nlat = h->cfg.storage == IMEXLB_PULL ? 2 : 1;
     // candidate 0 is the current lattice, which may lie in a window
     imx::ChunkedWindow win0 = std::move(h->win);
@@ -1119,7 +1142,7 @@ int imexlb_tune_placement_window(imexlb_handle *h, int64_t slack_bytes, int64_t 
     if (rc) return rc;
     if (steps < 2) steps = 2;
     steps += steps & 1;  // whole AA periods
-    const size_t lat_bytes = (size_t)Q * h->pstride * h->elem;
+    const size_t lat_bytes = h->lat_bytes;
     const int nlat = h->cfg.storage == IMEXLB_PULL ? 2 : 1;
     const size_t total = (size_t)nlat * lat_bytes + (size_t)slack_bytes;
     size_t free_b = 0, total_b = 0;

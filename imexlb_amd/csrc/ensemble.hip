@@ -433,6 +433,7 @@ int imexlb_ensemble_create(const imexlb_domain *doms, int n, int dtype, int stor
             P.nz = D.nz;
             P.ncell = nc;
             P.pstride = pstride[d];
+            P.geom = soa_geom((uint32_t)P.nx, (uint32_t)P.ny, pstride[d]);
             if (storage == IMEXLB_PULL) {
                 P.src = e->lat[2 * d + par];
                 P.dst = e->lat[2 * d + 1 - par];
@@ -490,7 +491,7 @@ int imexlb_ensemble_initialize(imexlb_ensemble *e)
         P.ny = D.ny;
         P.nz = D.nz;
         P.ncell = F.ncell;
-        P.pstride = F.pstride;
+        P.geom = F.geom;
         P.dst = e->lat[2 * d];
         P.layout = e->storage == IMEXLB_AA ? 1 : 0;
         P.kind = D.case_id == IMEXLB_CASE_TGV ? 0 : 1;

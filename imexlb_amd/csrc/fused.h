@@ -312,6 +312,8 @@ __device__ __forceinline__ void collide_lp_stream(float (&g)[Q], double pd, floa
     }
 }
 
+__device__ __forceinline__ bool wave_any(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; }
+
 // Where a cell's populations come from and go to.
 struct CellCtx {
     uint32_t c;
@@ -395,6 +397,19 @@ __device__ __forceinline__ bool src_out(const CellCtx &k, int i)
 __device__ __forceinline__ uint32_t src_off(const CellCtx &k, int i)
 {
     return k.rowb[1 - EZ[i]][1 - EY[i]] + k.xv[1 - EX[i]];
+}
+
+// Reduced precision: what a link bounced off the channel's ball takes on the
+// way, v - 6 w_i e_x U.  The roundings are written out, so that every kernel
+// variant does the same: one fused multiply-add in FP32, the product rounded
+// first in FP16.
+template <typename S>
+__device__ __forceinline__ float ball_link(const FusedParams &P, int i, float v)
+{
+#pragma clang fp contract(off)
+    const float c = (float)(WVAL[WCLASS[i]] * EX[i]), u = 6.f * (float)P.ush;
+    if constexpr (std::is_same<S, float>::value) return __builtin_fmaf(-c, u, v);
+    else return v - c * u;
 }
 
 // AA storage reads and writes the same 27 addresses per cell: direction i is
@@ -489,10 +504,7 @@ __device__ __forceinline__ void cell_gather(const FusedParams &P, const CellCtx 
                     // g_i = g*_bb(i) + s_bb(i) - s_i = g*_bb(i) - 6 w_i e_x U (the
                     // inflow equilibrium's stream U runs along x: nothing to add
                     // where e_x = 0)
-                    if (EX[i] != 0) {
-                        const R b = v - (float)(WVAL[WCLASS[i]] * EX[i]) * (6.f * (float)P.ush);
-                        v = solid ? b : v;
-                    }
+                    if (EX[i] != 0) v = solid ? ball_link<S>(P, i, v) : v;
                 }
                 if (EX[i] > 0) {
                     R in;
@@ -570,6 +582,31 @@ __device__ __forceinline__ void cell_collide(const FusedParams &P, const CellCtx
     }
 }
 
+// What the next step's x-face boundary kernels read, each row's nine together
+// (FusedParams::stage): the cavity's walls x = 1 (e_x = -1) and x = nx - 2
+// (e_x = +1), the sphere's inlet x = 0 (e_x = +1) and outlet x = nx - 1
+// (e_x = -1).  The register array f is indexed with compile-time constants
+// only (XDIR_P / XDIR_M), the two cases chosen by selects: an index computed
+// at run time would move f to private memory (64 more bytes written per
+// cell).
+__device__ __forceinline__ void stage_rows(const FusedParams &P, const CellCtx &k, const double (&f)[Q])
+{
+    if (P.stage == nullptr) return;
+    const uint64_t plane = (uint64_t)P.ny * P.nz, yz = (uint64_t)k.z * P.ny + k.y;
+    const uint32_t x = k.xv[1];
+    const bool sph = P.faithful_sphere != 0;
+    if (x == (sph ? 0u : 1u)) {
+        auto *p0 = glb(P.stage + yz * STAGE_ROW);
+#pragma unroll
+        for (int r = 0; r < 9; ++r) p0[r] = sph ? f[XDIR_P[r]] : f[XDIR_M[r]];
+    }
+    if (x == (sph ? P.nx - 1u : P.nx - 2u)) {
+        auto *p1 = glb(P.stage + (plane + yz) * STAGE_ROW);
+#pragma unroll
+        for (int r = 0; r < 9; ++r) p1[r] = sph ? f[XDIR_M[r]] : f[XDIR_P[r]];
+    }
+}
+
 // REUSE: the AA odd step stores through the gather's addresses (see
 // cell_gather); otherwise the store addresses are formed again from the
 // cell, which is cheaper in registers when the addresses of two cells per
@@ -582,31 +619,7 @@ __device__ __forceinline__ void cell_scatter(const FusedParams &P, const CellCtx
     const uint64_t ps = P.pstride;
     const uint32_t c = k.c;
     if constexpr (PAT == PAT_PULL) {
-        if constexpr (BC == BC_FAITHFUL) {
-            // what the next step's x-face boundary kernels read, each row's
-            // nine together (FusedParams::stage): the cavity's walls x = 1
-            // (e_x = -1) and x = nx - 2 (e_x = +1), the sphere's inlet x = 0
-            // (e_x = +1) and outlet x = nx - 1 (e_x = -1)
-            // The register array f is indexed with compile-time constants
-            // only (XDIR_P / XDIR_M), the two cases chosen by selects: an index
-            // computed at run time would move f to private memory (64 more
-            // bytes written per cell).
-            if (P.stage != nullptr) {
-                const uint64_t plane = (uint64_t)P.ny * P.nz, yz = (uint64_t)k.z * P.ny + k.y;
-                const uint32_t x = k.xv[1];
-                const bool sph = P.faithful_sphere != 0;
-                if (x == (sph ? 0u : 1u)) {
-                    auto *p0 = glb(P.stage + yz * STAGE_ROW);
-#pragma unroll
-                    for (int r = 0; r < 9; ++r) p0[r] = sph ? f[XDIR_P[r]] : f[XDIR_M[r]];
-                }
-                if (x == (sph ? P.nx - 1u : P.nx - 2u)) {
-                    auto *p1 = glb(P.stage + (plane + yz) * STAGE_ROW);
-#pragma unroll
-                    for (int r = 0; r < 9; ++r) p1[r] = sph ? f[XDIR_M[r]] : f[XDIR_P[r]];
-                }
-            }
-        }
+        if constexpr (BC == BC_FAITHFUL) stage_rows(P, k, f);
 #pragma unroll
         for (int i = 0; i < Q; ++i) st_pop<S, true, AM, true>(dst, ps, i, c, f[i]);
     } else if constexpr (PAT == PAT_AA_EVEN) {
@@ -708,8 +721,6 @@ __device__ __forceinline__ void st_pair(S *ptr, int cls, typename RealOf<S>::typ
     if constexpr (NT && IMX_STORE_POLICY != 1) __builtin_nontemporal_store(v, p);
     else *p = v;
 }
-
-__device__ __forceinline__ bool wave_any(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; }
 
 template <typename S, int PAT, bool NTL>
 __global__ void __launch_bounds__(512) k_fused_pair(const FusedParams P)

@@ -86,10 +86,91 @@ inline int fused_cells_per_thread(int cpt, int bc, uint32_t nx, int am)
     return cpt == 2 ? 2 : 1;
 }
 
+// Where population i of cell (z, p), p = y nx + x, lies in a lattice, in
+// elements: z zs + i is + (p >> tl) ts + p, i.e. within a z plane the cells
+// come in tiles of 2^tl, and a tile holds its populations one after the other.
+//
+// Two layouts:
+// - structure of arrays: one tile per lattice (tl = 31), is = the population
+//   stride, zs = nx ny.
+// - plane tiles: each z plane is a row of tiles of T = 2^tl cells, is = T,
+//   zs = 27 T tiles.  One population of a tile is at most 32 KiB, so the 27
+//   accesses of a wavefront fall into neighbouring DRAM rows of the same
+//   channels, where 27 arrays a gigabyte apart open 27 rows in banks that the
+//   lattice's place in HBM decides.  In-place 27-stream pass over 512^3 FP64,
+//   no arithmetic, TB/s (arrays / tiles of 4 / 8 / 16 / 32 / 64 / 128 KiB per
+//   population): 5.5 / 6.0 / 6.3 / 6.5 / 6.5 / 6.3 / 5.7, at every offset in 200 GiB
+//   for the tiles (6.5), 5.5 or 6.4 by offset for the arrays; a pull pass 5.3 / 5.9 / 6.0 /
+//   6.1 / 6.2 / 6.0 / 5.5.  Tiles that are not a power of two, or padded
+//   between populations, were slower (6.0).
+struct LatGeom {
+    uint64_t zs, is;
+    uint32_t ts, tl;
+#if defined(__HIPCC__)
+    __host__ __device__ __forceinline__ uint64_t off(int slot, uint32_t z, uint32_t p) const
+    {
+        return (uint64_t)z * zs + (uint64_t)slot * is + (uint64_t)(p >> tl) * ts + p;
+    }
+#endif
+};
+
+inline LatGeom soa_geom(uint32_t nx, uint32_t ny, uint64_t pstride)
+{
+    return LatGeom{(uint64_t)nx * ny, pstride, 0, 31};
+}
+
+// Elements of a lattice of nz planes.
+inline uint64_t lattice_elems(const LatGeom &g, uint32_t nz)
+{
+    return g.tl == 31 ? (uint64_t)Q * g.is : (uint64_t)nz * g.zs;
+}
+
+// Plane tiles for a lattice, where they serve: the largest tile of at most
+// 32 KiB per population (at least 64 cells) whose last tile leaves at most a
+// sixteenth of the plane unused.  Not for planes below 512 cells, whose
+// workgroups would be mostly idle (a workgroup never spans two planes), nor
+// where three planes exceed the 4 GiB that the kernels' 32-bit offsets reach.
+inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, LatGeom &g)
+{
+    const uint64_t plane = (uint64_t)nx * ny;
+    if (plane < 512) return false;
+    uint32_t tl = 6;
+    for (uint32_t t = 6; (elem << t) <= 32768; ++t) {
+        const uint64_t n = ((plane - 1) >> t) + 1;
+        if (((n << t) - plane) * 16 <= plane) tl = t;
+    }
+    const uint64_t tiles = ((plane - 1) >> tl) + 1;
+    const uint64_t zs = (tiles * Q) << tl;
+    if (3 * zs * elem > (uint64_t(1) << 32)) return false;
+    g = LatGeom{zs, uint64_t(1) << tl, (uint32_t)(Q - 1) << tl, tl};
+    return true;
+}
+
+// Threads per workgroup of the plane-tile kernels where the caller names
+// none: the largest of 256, 192, 128 and 64 that leaves at most a sixteenth of
+// the plane's threads idle, else the one that leaves the fewest.
+inline int tile_block(uint64_t plane)
+{
+    int best = 256;
+    uint64_t idle_best = ~uint64_t(0);
+    for (int b = 256; b >= 64; b -= 64) {
+        const uint64_t idle = (plane + b - 1) / b * b - plane;
+        if (idle * 16 <= plane) return b;
+        if (idle < idle_best) {
+            idle_best = idle;
+            best = b;
+        }
+    }
+    return best;
+}
+
 struct FusedParams {
     int nx, ny, nz;
     uint32_t ncell;          // nx * ny * nz
-    uint64_t pstride;        // elements between consecutive populations
+    uint64_t pstride;        // elements between consecutive populations (structure of arrays)
+    LatGeom geom;            // the lattice's layout
+    uint32_t bpp;            // plane tiles: workgroups per z plane
+    FastDiv divb;            // division by bpp
     const void *src;         // pull: lattice read; AA: the single lattice
     void *dst;               // pull: lattice written; AA: same as src
     double *mom_p, *mom_u, *mom_v, *mom_w;  // written when mom_p != nullptr
@@ -189,7 +270,7 @@ hipError_t launch_fused(int dtype, int bc, int pattern, const FusedParams &P, in
 struct InitParams {
     int nx, ny, nz;
     uint32_t ncell;
-    uint64_t pstride;
+    LatGeom geom;
     void *dst;               // lattice written (stored convention)
     int layout;              // 0 natural (pull), 1 swapped (AA after an even step)
     int kind;                // 0 TGV from the per-axis tables, 1 uniform (u0,0,0)/p0, masked,
@@ -210,7 +291,7 @@ hipError_t launch_init(int dtype, const InitParams &P, hipStream_t st);
 struct XferParams {
     int nx, ny, nz;
     uint32_t ncell;
-    uint64_t pstride;
+    LatGeom geom;
     void *lat;
     double *buf;             // [Q][nz][ny][nx]
     int layout;              // 0 natural, 1 swapped (AA even), 2 streamed (AA odd)

@@ -1,0 +1,67 @@
+"""The plane-tile layout (kernels.h LatGeom, tile.h) against the structure of
+arrays, which an explicit addr_mode selects and the oracle checks: the same
+populations and moments, bit for bit, in every case, storage and launch shape,
+on planes that end inside a tile, a workgroup or a wavefront."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (32, 16): the smallest tiled plane; (45, 37), (129, 33): ragged rows and
+# tiles; (64, 64), (128, 32): whole tiles; (700, 2) and (2, 300): one and many
+# rows per workgroup
+PLANES = [(32, 16, 3), (45, 37, 5), (64, 64, 4), (128, 32, 3), (129, 33, 4), (700, 2, 3), (2, 300, 2)]
+SHAPES = [None, (64, 1, 0, 0), (512, 2, 1, 1), (192, 3, 1, 1)]
+
+
+def state(n, steps, shape=None, addr_mode=-1, tau=0.06, **kw):
+    from imexlb_amd import LBM
+    g = LBM(*n, tau, u0=0.05, addr_mode=addr_mode, **kw)
+    if shape is not None:
+        g.set_launch(*shape)
+    g.Initialize()
+    g.step(steps, 3)
+    f, m = g.get_f(), g.moments()
+    info = g.info()
+    g.close()
+    return f, m, info
+
+
+def same(a, b, what):
+    assert np.array_equal(a[0], b[0]), f"populations: {what}"
+    for name, x, y in zip("puvw", a[1], b[1]):
+        assert np.array_equal(x, y), f"moment {name}: {what}"
+
+
+@pytest.mark.parametrize("n", PLANES)
+@pytest.mark.parametrize("case,mode", [("tgv", "faithful"), ("cavity", "config")])
+@pytest.mark.parametrize("dtype,storage", [("f64", "pull"), ("f64", "aa"), ("f32", "aa"), ("f16", "pull"), ("f16", "aa")])
+def test_tiles_equal_arrays(n, case, mode, dtype, storage):
+    print(f"[case] tiles {case} {n} {dtype} {storage}", flush=True)
+    kw = dict(case=case, mode=mode, dtype=dtype, storage=storage)
+    for steps in (6, 7):
+        want = state(n, steps, addr_mode=2, **kw)
+        for shape in SHAPES:
+            got = state(n, steps, shape, **kw)
+            same(got, want, f"{steps} steps, launch {shape}")
+            assert got[2]["cells_per_thread"] == (2 if shape and shape[1] == 2 else 1)
+
+
+BOUNDED = [
+    ("cavity", "faithful", (24, 30, 5), "f64", None),
+    ("cavity", "faithful", (100, 41, 6), "f64", None),
+    ("sphere", "faithful", (72, 20, 18), "f64", None),
+    ("sphere", "faithful", (130, 37, 40), "f64", None),
+    ("sphere", "config", (40, 24, 24), "f64", (12.0, 11.0, 12.0, 4.5)),
+    ("sphere", "config", (67, 33, 30), "f16", (20.0, 16.0, 15.0, 5.0)),
+    ("sphere", "config", (64, 32, 30), "f32", (20.0, 16.0, 15.0, 12.0)),
+]
+
+
+@pytest.mark.parametrize("case,mode,n,dtype,ball", BOUNDED)
+def test_tiles_equal_arrays_at_boundaries(case, mode, n, dtype, ball):
+    print(f"[case] tiles {case} {mode} {n} {dtype}", flush=True)
+    kw = dict(case=case, mode=mode, dtype=dtype, sphere=ball, tau=0.1)
+    want = state(n, 7, addr_mode=2, **kw)
+    for shape in SHAPES:
+        same(state(n, 7, shape, **kw), want, f"launch {shape}")
