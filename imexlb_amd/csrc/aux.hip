@@ -25,7 +25,7 @@ __device__ __forceinline__ double feq_f64(int i, double p, double u, double v, d
 template <typename S>
 __device__ __forceinline__ void put(S *lat, const LatGeom &g, int slot, uint32_t z, uint32_t c, double f, double s)
 {
-    S *p = lat + g.off(slot, z, c);
+    S *p = lat + g.off(g.pos(slot), z, c);
     if constexpr (std::is_same<S, double>::value)
         *p = f;
     else if constexpr (std::is_same<S, float>::value)
@@ -37,7 +37,7 @@ __device__ __forceinline__ void put(S *lat, const LatGeom &g, int slot, uint32_t
 template <typename S>
 __device__ __forceinline__ double get(const S *lat, const LatGeom &g, int slot, uint32_t z, uint32_t c, double s)
 {
-    const S *p = lat + g.off(slot, z, c);
+    const S *p = lat + g.off(g.pos(slot), z, c);
     if constexpr (std::is_same<S, double>::value)
         return *p;
     else if constexpr (std::is_same<S, float>::value)

@@ -87,7 +87,7 @@ inline int fused_cells_per_thread(int cpt, int bc, uint32_t nx, int am)
 }
 
 // Where population i of cell (z, p), p = y nx + x, lies in a lattice, in
-// elements: z zs + i is + (p >> tl) ts + p, i.e. within a z plane the cells
+// elements: z zs + pos(i) is + (p >> tl) ts + p, i.e. within a z plane the cells
 // come in tiles of 2^tl, and a tile holds its populations one after the other.
 //
 // Two layouts:
@@ -103,20 +103,29 @@ inline int fused_cells_per_thread(int cpt, int bc, uint32_t nx, int am)
 //   for the tiles (6.5), 5.5 or 6.4 by offset for the arrays; a pull pass 5.3 / 5.9 / 6.0 /
 //   6.1 / 6.2 / 6.0 / 5.5.  Tiles that are not a power of two, or padded
 //   between populations, were slower (6.0).
+//
+// AA lattices in tiles keep the populations sorted by e_z (by_ez): the odd step
+// reads and writes nine of them in each of three planes, and those nine are
+// then neighbours.  TGV 512^3 passes without arithmetic, TB/s, index order /
+// by e_z: odd step FP64 5.7 / 6.0, FP32 5.7 / 5.9, even step 6.6 / 6.5, 6.5 / 6.4;
+// pull 6.3 / 6.2, so pull lattices keep the index order.
 struct LatGeom {
     uint64_t zs, is;
     uint32_t ts, tl;
+    int by_ez;
 #if defined(__HIPCC__)
-    __host__ __device__ __forceinline__ uint64_t off(int slot, uint32_t z, uint32_t p) const
+    // the place of population i among a tile's 27 (i: a compile-time constant)
+    __host__ __device__ __forceinline__ int pos(int i) const { return by_ez ? EZ_POS.v[i] : i; }
+    __host__ __device__ __forceinline__ uint64_t off(int place, uint32_t z, uint32_t p) const
     {
-        return (uint64_t)z * zs + (uint64_t)slot * is + (uint64_t)(p >> tl) * ts + p;
+        return (uint64_t)z * zs + (uint64_t)place * is + (uint64_t)(p >> tl) * ts + p;
     }
 #endif
 };
 
 inline LatGeom soa_geom(uint32_t nx, uint32_t ny, uint64_t pstride)
 {
-    return LatGeom{(uint64_t)nx * ny, pstride, 0, 31};
+    return LatGeom{(uint64_t)nx * ny, pstride, 0, 31, 0};
 }
 
 // Elements of a lattice of nz planes.
@@ -130,7 +139,7 @@ inline uint64_t lattice_elems(const LatGeom &g, uint32_t nz)
 // sixteenth of the plane unused.  Not for planes below 512 cells, whose
 // workgroups would be mostly idle (a workgroup never spans two planes), nor
 // where three planes exceed the 4 GiB that the kernels' 32-bit offsets reach.
-inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, LatGeom &g)
+inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, bool aa, LatGeom &g)
 {
     const uint64_t plane = (uint64_t)nx * ny;
     if (plane < 512) return false;
@@ -142,7 +151,7 @@ inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, LatGeom &g)
     const uint64_t tiles = ((plane - 1) >> tl) + 1;
     const uint64_t zs = (tiles * Q) << tl;
     if (3 * zs * elem > (uint64_t(1) << 32)) return false;
-    g = LatGeom{zs, uint64_t(1) << tl, (uint32_t)(Q - 1) << tl, tl};
+    g = LatGeom{zs, uint64_t(1) << tl, (uint32_t)(Q - 1) << tl, tl, aa ? 1 : 0};
     return true;
 }
 
@@ -162,6 +171,25 @@ inline int tile_block(uint64_t plane)
         }
     }
     return best;
+}
+
+// Rows per workgroup of the AA odd step's row kernel (tile.h k_tiled_rows)
+// for a requested block: as many whole rows as fit it, at least one; 0 where
+// the shifted form (k_tiled) serves better:
+// - rows that are not a whole number of wavefronts or exceed 512 threads;
+// - rows of one wavefront (64x256x256 FP32: 146 us with rows, 140 without);
+// - lattices that the 256 MB last-level cache holds a good part of, where the
+//   shifted form's second access to a line is cheap (us per AA step, rows /
+//   shifted: cavity 128^3 FP64 148 / 146, FP32 78 / 66, TGV 192x80x80 FP64 93 / 85; above
+//   512 MiB TGV 512^3 FP64 9580 / 10430, 448x256x256 FP64 2105 / 2355, FP16 513 / 536,
+//   cavity 256^3 FP64 1179 / 1327, FP32 594 / 617);
+// - the FP16 cavity, whose x walls split the rows' 128-byte lines (320x192x192:
+//   257 / 208).
+inline uint32_t tile_rows(int nx, int block, uint64_t lattice_bytes, int bc, uint64_t elem)
+{
+    if (nx % 64 != 0 || nx == 64 || nx > 512) return 0;
+    if (lattice_bytes < (uint64_t(512) << 20) || (bc != BC_PERIODIC && elem == 2)) return 0;
+    return block > nx ? (uint32_t)(block / nx) : 1u;
 }
 
 struct FusedParams {

@@ -37,6 +37,23 @@ IMX_HD constexpr double w(int i) { return WVAL[WCLASS[i]]; }
 constexpr float H_SCALE[4] = {4.0f, 16.0f, 64.0f, 256.0f};
 constexpr float H_INV_SCALE[4] = {0.25f, 0.0625f, 0.015625f, 0.00390625f};
 
+// The directions' places when they are sorted by e_z: those with e_z = -1
+// first, then 0, then +1, each in index order.
+struct EzPos {
+    int v[Q];
+};
+constexpr EzPos ez_pos()
+{
+    EzPos p{};
+    for (int i = 0; i < Q; ++i) {
+        int n = 0;
+        for (int k = 0; k < Q; ++k) n += EZ[k] < EZ[i] || (EZ[k] == EZ[i] && k < i) ? 1 : 0;
+        p.v[i] = n;
+    }
+    return p;
+}
+constexpr EzPos EZ_POS = ez_pos();
+
 // The d-th direction, in index order, of the nine with e_AXIS * SIGN > 0
 // (d < 9), and a direction's velocity and opposite, for kernels that give each
 // direction its own row of workgroups.

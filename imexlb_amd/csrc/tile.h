@@ -66,12 +66,20 @@ __device__ __forceinline__ void tile_setup(const FusedParams &P, uint32_t z, uin
     }
 }
 
-// Population `slot` of a plane at byte offset `o`: the plane's first element
+// The place of population i in a tile (LatGeom::pos).
+template <int PAT>
+__device__ __forceinline__ constexpr int tile_slot(int i)
+{
+    return PAT == PAT_PULL ? i : EZ_POS.v[i];
+}
+
+// Population i of a plane at byte offset `o`: the plane's first element
 // is the same for all lanes, the population's place is added to the 32-bit
 // offset.
-template <typename S>
-__device__ __forceinline__ S *tile_ptr(S *plane, const FusedParams &P, int slot, uint32_t o)
+template <int PAT, typename S>
+__device__ __forceinline__ S *tile_ptr(S *plane, const FusedParams &P, int i, uint32_t o)
 {
+    const int slot = tile_slot<PAT>(i);
     using B = typename std::conditional<std::is_const<S>::value, const char, char>::type;
     return (S *)((B *)plane + (uint32_t)(o + (uint32_t)slot * (uint32_t)(P.geom.is * sizeof(S))));
 }
@@ -110,7 +118,7 @@ __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx 
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
         if constexpr (PAT == PAT_AA_EVEN) {
-            f[i] = ld_ptr<S, NTL>(tile_ptr(pl[1], P, i, t.o[1][1]), WCLASS[i]);
+            f[i] = ld_ptr<S, NTL>(tile_ptr<PAT>(pl[1], P, i, t.o[1][1]), WCLASS[i]);
             if constexpr (BC == BC_CAVITY) {
                 if (EZ[i] < 0) {
                     R lid;
@@ -126,7 +134,7 @@ __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx 
             // lines that no other wavefront reads are not kept
             const bool nt = NTL && EX[i] == 0;
             if constexpr (BC == BC_PERIODIC) {
-                const S *p = tile_ptr(from, P, s, o);
+                const S *p = tile_ptr<PAT>(from, P, s, o);
                 f[i] = nt ? ld_ptr<S, true>(p, WCLASS[i]) : ld_ptr<S, false>(p, WCLASS[i]);
             } else if constexpr (BC == BC_CAVITY) {
                 // One base (the plane below), two offsets: where x - e_i is
@@ -134,8 +142,8 @@ __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx 
                 const bool out = src_out(k, i);
                 const uint32_t zb = (uint32_t)((pl[1] - pl[0]) * (int64_t)sizeof(S));
                 const uint32_t is = (uint32_t)(P.geom.is * sizeof(S));
-                const uint32_t in = (uint32_t)((from - pl[0]) * (int64_t)sizeof(S)) + (uint32_t)s * is + o;
-                const uint32_t own = zb + (uint32_t)BB[s] * is + t.o[1][1];
+                const uint32_t in = (uint32_t)((from - pl[0]) * (int64_t)sizeof(S)) + (uint32_t)tile_slot<PAT>(s) * is + o;
+                const uint32_t own = zb + (uint32_t)tile_slot<PAT>(BB[s]) * is + t.o[1][1];
                 const S *p = (const S *)((const char *)pl[0] + (out ? own : in));
                 R v = nt ? ld_ptr<S, true>(p, WCLASS[i]) : ld_ptr<S, false>(p, WCLASS[i]);
                 if (EZ[i] < 0) {
@@ -155,7 +163,7 @@ __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx 
                 const uint32_t rzi =
                     2 * (P.ring_a + P.ring_b) + (EZ[i] < 0 ? P.ring_c : 0u) + k.rz0 - EY[i] * nx - EX[i];
                 const uint32_t r = ox ? rxi : (oy ? ryi : rzi);
-                const S *p = tile_ptr(from, P, s, o);
+                const S *p = tile_ptr<PAT>(from, P, s, o);
                 if (i != 0) {
                     const S *g = (const S *)P.ring + (uint64_t)i * P.ring_n + r;
                     p = ox || oy || oz ? g : p;
@@ -163,7 +171,7 @@ __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx 
                 f[i] = nt ? ld_ptr<S, true>(p, WCLASS[i]) : ld_ptr<S, false>(p, WCLASS[i]);
             } else {  // channel, pull only
                 bool solid = false;
-                const S *p = tile_ptr(from, P, s, o);
+                const S *p = tile_ptr<PAT>(from, P, s, o);
                 if constexpr (!CLEAR) {
                     if (i != 0 && k.m == 2) {
                         const uint32_t nz = P.nz, z = P.divy.div(P.divx.div(k.c));
@@ -174,7 +182,7 @@ __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx 
                                                         : y;
                         solid = *glb(P.mask + ((uint64_t)zs * P.ny + ys) * P.nx + k.xv[1 - EX[i]]) == 1;
                     }
-                    const S *own = tile_ptr(pl[1], P, BB[i], t.o[1][1]);
+                    const S *own = tile_ptr<PAT>(pl[1], P, BB[i], t.o[1][1]);
                     p = solid ? own : p;
                 }
                 R v = ld_ptr<S, false>(p, WCLASS[i]);
@@ -215,7 +223,7 @@ __device__ __forceinline__ void tile_scatter(const FusedParams &P, const TileCtx
         if constexpr (BC == BC_FAITHFUL) stage_rows(P, k, f);
 #pragma unroll
         for (int i = 0; i < Q; ++i)
-            st_ptr<S>(tile_ptr(pl[1], P, PAT == PAT_PULL ? i : BB[i], o9[1][1]), WCLASS[i], f[i]);
+            st_ptr<S>(tile_ptr<PAT>(pl[1], P, PAT == PAT_PULL ? i : BB[i], o9[1][1]), WCLASS[i], f[i]);
     } else {
         // to slot i of x + e_i, or bounced back into slot bb(i) at x
 #pragma unroll
@@ -226,11 +234,11 @@ __device__ __forceinline__ void tile_scatter(const FusedParams &P, const TileCtx
             if constexpr (BC == BC_CAVITY) {
                 const uint32_t zb = (uint32_t)((pl[1] - pl[0]) * (int64_t)sizeof(S));
                 const uint32_t is = (uint32_t)(P.geom.is * sizeof(S));
-                const uint32_t in = (uint32_t)((to - pl[0]) * (int64_t)sizeof(S)) + (uint32_t)i * is + o;
-                const uint32_t own = zb + (uint32_t)BB[i] * is + o9[1][1];
+                const uint32_t in = (uint32_t)((to - pl[0]) * (int64_t)sizeof(S)) + (uint32_t)tile_slot<PAT>(i) * is + o;
+                const uint32_t own = zb + (uint32_t)tile_slot<PAT>(BB[i]) * is + o9[1][1];
                 p = (S *)((char *)pl[0] + (src_out(k, BB[i]) ? own : in));
             } else {
-                p = tile_ptr(to, P, i, o);
+                p = tile_ptr<PAT>(to, P, i, o);
             }
             if (IMX_TILE_ODD_NT || EX[i] == 0) st_ptr<S, true>(p, WCLASS[i], f[i]);
             else st_ptr<S, false>(p, WCLASS[i], f[i]);
@@ -245,11 +253,14 @@ __device__ __forceinline__ void tile_scatter(const FusedParams &P, const TileCtx
 // / one run per XCD / runs of 8, block 256 (pull unless said): TGV 256^3 FP64 1292 /
 // 1218 / 1209, FP32 605 / 621 / 603, FP16 310 / 310 / 297, 301x203x157 FP32 337 / 367 / 342,
 // channel 512x256x256 FP16 640 / 702 / 637, cavity 128^3 FP64 AA 149.6 / 149.6 / 146.0.
+// Grids that the chip holds at once stay linear (cavity 64^3 AA, 1024
+// workgroups, linear / runs of 8: FP64 22.3 / 23.4, FP32 10.8 / 12.4, FP16 8.0 / 9.2;
+// 96^3, 3456 workgroups: 67.8 / 67.5, 33.8 / 33.2, 23.5 / 22.7).
 __device__ __forceinline__ uint32_t xcd_run(uint32_t b, uint32_t nb)
 {
     constexpr uint32_t RUN = 8, ALL = 8 * RUN;
     const uint32_t g = b / ALL, r = b % ALL;
-    return (g + 1) * ALL <= nb ? g * ALL + (r & 7u) * RUN + (r >> 3) : b;
+    return nb > 2048 && (g + 1) * ALL <= nb ? g * ALL + (r & 7u) * RUN + (r >> 3) : b;
 }
 
 // Before (structure of arrays, k_fused) and after, us per step, first
@@ -303,6 +314,166 @@ __global__ void __launch_bounds__(512) k_tiled(const FusedParams P)
     }
 }
 
+// The value of the lane before (EXP 1) or after (EXP -1); the first (last)
+// lane takes `edge`.
+template <int EXP>
+__device__ __forceinline__ float lane_shift(float v, float edge)
+{
+    constexpr int CTRL = EXP > 0 ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, edge), __builtin_bit_cast(int, v),
+                                                                 CTRL, 0xf, 0xf, false));
+}
+template <int EXP>
+__device__ __forceinline__ double lane_shift(double v, double edge)
+{
+    constexpr int CTRL = EXP > 0 ? 0x138 : 0x130;
+    const uint64_t a = __builtin_bit_cast(uint64_t, v), e = __builtin_bit_cast(uint64_t, edge);
+    const uint32_t lo = __builtin_amdgcn_update_dpp((int)(uint32_t)e, (int)(uint32_t)a, CTRL, 0xf, 0xf, false);
+    const uint32_t hi = __builtin_amdgcn_update_dpp((int)(uint32_t)(e >> 32), (int)(uint32_t)(a >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+
+// The AA odd step on rows that are whole wavefronts (nx a multiple of 64, at
+// most 512): a workgroup is one or more whole rows, every population moves in
+// x-aligned lines, loaded and stored non-temporally, and what crosses into a
+// neighbouring cell in x crosses between lanes (DPP; LDS between wavefronts)
+// instead of through shifted lines.  The shifted form loads a line twice and
+// stores it in two parts, through L2: 5.2 TB/s against 5.9-6.1 for this
+// pattern without arithmetic (TGV 512^3, FP64).  As every row is one
+// wavefront's, its addresses are scalars and one lane offset serves all 27.
+template <typename R>
+struct RowEdges {
+    // [wavefront][0: its last lane, e_x = 1; 1: its first lane, e_x = -1][XDIR_P / XDIR_M rank]
+    R v[8][2][10];
+};
+
+template <typename S, int BC, bool NTL>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k_tiled_rows(const FusedParams P)
+{
+    using R = typename RealOf<S>::type;
+    constexpr bool F64 = std::is_same<S, double>::value;
+    constexpr bool WALLS = BC == BC_CAVITY;
+    __shared__ RowEdges<R> in, out;
+    uint32_t b = blockIdx.x;
+    if (P.xcd_remap) b = xcd_run(b, P.nblocks);
+    const uint32_t nx = P.nx, ny = P.ny, nz = P.nz, plane = nx * ny;
+    const uint32_t z = P.divb.div(b), lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), per_row = nx >> 6;
+    const uint32_t row = wave / per_row, seg = wave - row * per_row;
+    const uint32_t y0 = (b - z * P.bpp) * (blockDim.x / nx) + row;
+    // a last workgroup's rows beyond the plane work on the last row and store
+    // nothing
+    const bool live = y0 < ny;
+    const uint32_t y = live ? y0 : ny - 1, x = seg * 64u + lane;
+    const uint32_t first = row * per_row;
+    const uint32_t prev = seg == 0 ? first + per_row - 1 : wave - 1, next = seg + 1 == per_row ? first : wave + 1;
+
+    const uint32_t zv[3] = {z == 0 ? (WALLS ? 0 : nz - 1) : z - 1, z, z == nz - 1 ? (WALLS ? z : 0) : z + 1};
+    const uint32_t yv[3] = {y == 0 ? (WALLS ? 0 : ny - 1) : y - 1, y, y == ny - 1 ? (WALLS ? y : 0) : y + 1};
+    const bool zo[3] = {WALLS && z == 0, false, WALLS && z == nz - 1};
+    const bool yo[3] = {WALLS && y == 0, false, WALLS && y == ny - 1};
+    S *const lat = (S *)P.dst;
+    S *seg_of[3][3];  // this wavefront's cells in rows (z + a - 1, y + b - 1), population 0
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) seg_of[a][c] = uniform_ptr(lat + P.geom.off(0, zv[a], yv[c] * nx + seg * 64u));
+    // population `slot` of lane `l` of row (z + a - 1, y + c - 1)
+    auto at = [&](int a, int c, int slot, uint32_t l) {
+        return (S *)((char *)seg_of[a][c] + (uint32_t)(l * (uint32_t)sizeof(S) + (uint32_t)tile_slot<PAT_AA_ODD>(slot) * (uint32_t)(P.geom.is * sizeof(S))));
+    };
+
+    R f[Q];
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+        // from slot bb(i) of x - e_i; where that row lies outside the cavity,
+        // the cell's own slot i, not shifted
+        const bool o = zo[1 - EZ[i]] || yo[1 - EY[i]];
+        f[i] = ld_ptr<S, NTL>(o ? at(1, 1, i, lane) : at(1 - EZ[i], 1 - EY[i], BB[i], lane), WCLASS[i]);
+    }
+    // cells at an x wall take their own slot i
+    R wall[9];
+    const bool xw_lo = WALLS && seg == 0, xw_hi = WALLS && seg + 1 == per_row;
+    R wall2[9];
+    if (xw_lo) {
+#pragma unroll
+        for (int r = 0; r < 9; ++r) wall[r] = ld_ptr<S>(at(1, 1, XDIR_P[r], 0), WCLASS[XDIR_P[r]]);
+    }
+    if (xw_hi) {
+#pragma unroll
+        for (int r = 0; r < 9; ++r) wall2[r] = ld_ptr<S>(at(1, 1, XDIR_M[r], 63), WCLASS[XDIR_M[r]]);
+    }
+    auto exchange = [&](RowEdges<R> &e, bool gather) {
+        if (lane == 0 || lane == 63) {
+#pragma unroll
+            for (int r = 0; r < 9; ++r) e.v[wave][lane == 0][r] = lane == 0 ? f[XDIR_M[r]] : f[XDIR_P[r]];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 9; ++r) {
+            const int p = XDIR_P[r], m = XDIR_M[r];
+            R ep = e.v[prev][0][r], em = e.v[next][1][r];
+            if (gather && xw_lo) ep = wall[r];
+            if (gather && xw_hi) em = wall2[r];
+            const R sp = lane_shift<1>(f[p], ep), sm = lane_shift<-1>(f[m], em);
+            if constexpr (WALLS) {
+                const bool op = gather ? zo[1 - EZ[p]] || yo[1 - EY[p]] : zo[1 + EZ[p]] || yo[1 + EY[p]];
+                const bool om = gather ? zo[1 - EZ[m]] || yo[1 - EY[m]] : zo[1 + EZ[m]] || yo[1 + EY[m]];
+                f[p] = op ? f[p] : sp;
+                f[m] = om ? f[m] : sm;
+            } else {
+                f[p] = sp;
+                f[m] = sm;
+            }
+        }
+    };
+    exchange(in, true);
+    // FP64: 127 registers (four wavefronts per SIMD) instead of 129
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (WALLS) {
+#pragma unroll
+        for (int i = 0; i < Q; ++i)
+            if (EZ[i] < 0) {
+                R lid;
+                if constexpr (F64) lid = f[i] + P.corr[i];
+                else lid = f[i] + (float)P.corr[i];
+                f[i] = z == nz - 1 ? lid : f[i];
+            }
+    }
+
+    CellCtx k;
+    k.c = z * plane + y * nx + x;
+    cell_collide<S, BC>(P, k, f, P.mom_p != nullptr && live);
+
+    if constexpr (WALLS) {
+        // what leaves through an x wall comes back into slot bb(i) of the cell
+        if (live && xw_hi && lane == 63) {
+#pragma unroll
+            for (int r = 0; r < 9; ++r) st_ptr<S, false>(at(1, 1, XDIR_M[r], lane), WCLASS[XDIR_M[r]], f[BB[XDIR_M[r]]]);
+        }
+        if (live && xw_lo && lane == 0) {
+#pragma unroll
+            for (int r = 0; r < 9; ++r) st_ptr<S, false>(at(1, 1, XDIR_P[r], lane), WCLASS[XDIR_P[r]], f[BB[XDIR_P[r]]]);
+        }
+    }
+    exchange(out, false);
+    if (!live) return;
+    uint32_t to = lane;  // see tile_scatter
+    asm("" : "+v"(to));
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+        // to slot i of x + e_i, or back into the cell's own slot bb(i)
+        const bool o = zo[1 + EZ[i]] || yo[1 + EY[i]];
+        S *const p = o ? at(1, 1, BB[i], to) : at(1 + EZ[i], 1 + EY[i], i, to);
+        if constexpr (WALLS) {
+            // nothing arrives at an x wall from beyond it
+            if (EX[i] > 0 && xw_lo && !o && lane == 0) continue;
+            if (EX[i] < 0 && xw_hi && !o && lane == 63) continue;
+        }
+        st_ptr<S, true>(p, WCLASS[i], f[i]);
+    }
+}
+
 template <typename S, int CPT, bool NTL>
 hipError_t launch_tiled_cpt(int bc, int pattern, const FusedParams &P, int block, hipStream_t st)
 {
@@ -333,6 +504,23 @@ template <typename S>
 hipError_t launch_tiled(int bc, int pattern, const FusedParams &P0, int block, hipStream_t st)
 {
     FusedParams P = P0;
+    const uint32_t rows = tile_rows(P.nx, block, lattice_elems(P.geom, (uint32_t)P.nz) * sizeof(S), bc, sizeof(S));
+    if (pattern == PAT_AA_ODD && rows > 0) {
+        P.bpp = ((uint32_t)P.ny + rows - 1) / rows;
+        P.divb.init(P.bpp);
+        P.nblocks = P.bpp * (uint32_t)P.nz;
+        const dim3 grid(P.nblocks), blk(rows * (uint32_t)P.nx);
+#define IMX_L(B)                                                                                  \
+    do {                                                                                          \
+        if (P.ntl) hipLaunchKernelGGL((k_tiled_rows<S, B, true>), grid, blk, 0, st, P);           \
+        else hipLaunchKernelGGL((k_tiled_rows<S, B, false>), grid, blk, 0, st, P);                \
+    } while (0)
+        if (bc == BC_PERIODIC) IMX_L(BC_PERIODIC);
+        else if (bc == BC_CAVITY) IMX_L(BC_CAVITY);
+        else return hipErrorInvalidValue;
+#undef IMX_L
+        return hipGetLastError();
+    }
     const int cpt = P.cpt == 2 ? 2 : 1;
     const uint32_t plane = (uint32_t)P.nx * (uint32_t)P.ny, per = (uint32_t)block * (uint32_t)cpt;
     P.bpp = (plane + per - 1) / per;

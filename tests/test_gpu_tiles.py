@@ -9,8 +9,10 @@ pytestmark = pytest.mark.gpu
 
 # (32, 16): the smallest tiled plane; (45, 37), (129, 33): ragged rows and
 # tiles; (64, 64), (128, 32): whole tiles; (700, 2) and (2, 300): one and many
-# rows per workgroup
-PLANES = [(32, 16, 3), (45, 37, 5), (64, 64, 4), (128, 32, 3), (129, 33, 4), (700, 2, 3), (2, 300, 2)]
+# rows per workgroup; (64, 9), (192, 7), (512, 3): rows of one, three and eight
+# wavefronts, with rows left over in the last workgroup
+PLANES = [(32, 16, 3), (45, 37, 5), (64, 64, 4), (128, 32, 3), (129, 33, 4), (700, 2, 3), (2, 300, 2),
+          (64, 9, 4), (192, 7, 3), (512, 3, 2)]
 SHAPES = [None, (64, 1, 0, 0), (512, 2, 1, 1), (192, 3, 1, 1)]
 
 
@@ -65,3 +67,19 @@ def test_tiles_equal_arrays_at_boundaries(case, mode, n, dtype, ball):
     want = state(n, 7, addr_mode=2, **kw)
     for shape in SHAPES:
         same(state(n, 7, shape, **kw), want, f"launch {shape}")
+
+
+# The AA odd step's row kernel runs on lattices above 512 MiB: rows of two,
+# three and eight wavefronts, rows left over in the last workgroup of a plane
+ROWS = [("tgv", "faithful", (512, 131, 40), "f64"), ("tgv", "faithful", (192, 201, 131), "f32"),
+        ("tgv", "faithful", (128, 515, 160), "f16"), ("cavity", "config", (192, 101, 140), "f64"),
+        ("cavity", "config", (128, 203, 201), "f32"), ("cavity", "config", (512, 67, 79), "f64")]
+
+
+@pytest.mark.parametrize("case,mode,n,dtype", ROWS)
+def test_row_kernel_equals_arrays(case, mode, n, dtype):
+    print(f"[case] rows {case} {n} {dtype}", flush=True)
+    kw = dict(case=case, mode=mode, dtype=dtype, storage="aa")
+    want = state(n, 5, addr_mode=2, **kw)
+    for shape in (None, (512, 1, 0, 0)):
+        same(state(n, 5, shape, **kw), want, f"launch {shape}")
