@@ -16,6 +16,7 @@
 #include "window.h"
 #include "kernels.h"
 #include "phased.h"
+#include "readback.h"
 
 using namespace imx;
 
@@ -59,6 +60,7 @@ struct imexlb_handle {
     // valid for the lattices, start state and launch shape in gkey
     hipGraphExec_t gexec = nullptr;
     uint64_t gkey[8] = {};
+    imx::ReadBack back;      // reads of fields and populations into host memory
     // phased engine
     PhasedState *ph = nullptr;
     std::string err;
@@ -732,9 +734,11 @@ int imexlb_get_moments(imexlb_handle *h, double *p, double *u, double *v, double
         return fail(h, IMEXLB_ESTATE, "no moments for step %lld (last written at %lld)", (long long)h->steps,
                     (long long)h->mom_step);
     double *out[4] = {p, u, v, w};
+    imx::ReadBack::Part part[4];
+    int n = 0;
     for (int k = 0; k < 4; ++k)
-        if (out[k]) HIPCHK(h, hipMemcpyAsync(out[k], h->mom[k], (size_t)h->ncell * 8, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+        if (out[k]) part[n++] = {out[k], h->mom[k], (size_t)h->ncell * 8};
+    HIPCHK(h, h->back.copy(part, n, h->device, h->stream));
     return IMEXLB_OK;
 }
 
@@ -776,7 +780,8 @@ static int xfer(imexlb_handle *h, double *host, bool get)
     hipError_t e = hipSuccess;
     if (get) {
         e = launch_get_f(c.dtype, P, h->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(host, d, bytes, hipMemcpyDeviceToHost, h->stream);
+        const imx::ReadBack::Part part{host, d, bytes};
+        if (e == hipSuccess) e = h->back.copy(&part, 1, h->device, h->stream);
     } else {
         e = hipMemcpyAsync(d, host, bytes, hipMemcpyHostToDevice, h->stream);
         if (e == hipSuccess) e = launch_set_f(c.dtype, P, h->stream);
@@ -838,8 +843,8 @@ int imexlb_checkpoint_write(imexlb_handle *h, const char *path)
     rc = h->ph ? phased_get_state(h->ph, f.data(), h->err) : imexlb_get_f(h, f.data());
     if (rc) return rc;
     if (h->ring) {
-        HIPCHK(h, hipMemcpyAsync(f.data() + nf, h->ring, ring_doubles(h) * 8, hipMemcpyDeviceToHost, h->stream));
-        HIPCHK(h, hipStreamSynchronize(h->stream));
+        const imx::ReadBack::Part part{f.data() + nf, h->ring, ring_doubles(h) * 8};
+        HIPCHK(h, h->back.copy(&part, 1, h->device, h->stream));
     }
     FILE *fp = std::fopen(path, "wb");
     if (!fp) return fail(h, IMEXLB_EIO, "cannot open %s", path);
@@ -932,8 +937,8 @@ int imexlb_diagnostics(imexlb_handle *h, double *ke, double *mass)
     HIPCHK(h, launch_diag(h->mom[0], h->mom[1], h->mom[2], h->mom[3], h->mask, h->ncell, h->partials, h->nparts,
                           h->result, h->stream));
     double out[2];
-    HIPCHK(h, hipMemcpyAsync(out, h->result, sizeof out, hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    const imx::ReadBack::Part part{out, h->result, sizeof out};
+    HIPCHK(h, h->back.copy(&part, 1, h->device, h->stream));
     *ke = out[0];
     *mass = out[1];
     return IMEXLB_OK;
@@ -949,8 +954,8 @@ int imexlb_sphere_force(imexlb_handle *h, double *force3)
     FusedParams P;
     fill_fused_params(h, P, h->cur, h->cur);
     HIPCHK(h, launch_force(h->cfg.dtype, P, h->partials, h->nparts, h->result, h->stream));
-    HIPCHK(h, hipMemcpyAsync(force3, h->result, 3 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    const imx::ReadBack::Part part{force3, h->result, 3 * sizeof(double)};
+    HIPCHK(h, h->back.copy(&part, 1, h->device, h->stream));
     return IMEXLB_OK;
 }
 

@@ -22,6 +22,7 @@
 
 #include "../../include/imexlb.h"
 #include "fused.h"
+#include "readback.h"
 #include "window.h"
 #include "kernels.h"
 
@@ -146,6 +147,7 @@ struct imexlb_ensemble {
     std::vector<double *> tabs;          // TGV init tables per domain
     int32_t *dflags = nullptr;           // per-domain finite flags (imexlb_ensemble_status)
     double *dummy = nullptr;
+    ReadBack back;                       // reads of the members' fields
     int block = 256, cpt = 1, grid = 0, cus = 256;
     int64_t steps = 0, mom_step = -1, cells = 0, device_bytes = 0;
     hipGraphExec_t gexec = nullptr;
@@ -574,9 +576,11 @@ int imexlb_ensemble_get_moments(imexlb_ensemble *e, int d, double *p, double *u,
     ECHK(e, hipSetDevice(e->device));
     double *out[4] = {p, u, v, w};
     const size_t nb = (size_t)e->hp[2 * d].ncell * 8;
+    ReadBack::Part part[4];
+    int n = 0;
     for (int k = 0; k < 4; ++k)
-        if (out[k]) ECHK(e, hipMemcpyAsync(out[k], e->mom[4 * d + k], nb, hipMemcpyDeviceToHost, e->stream));
-    ECHK(e, hipStreamSynchronize(e->stream));
+        if (out[k]) part[n++] = {out[k], e->mom[4 * d + k], nb};
+    ECHK(e, e->back.copy(part, n, e->device, e->stream));
     return IMEXLB_OK;
 }
 
@@ -592,8 +596,8 @@ int imexlb_ensemble_status(imexlb_ensemble *e, int32_t *finite, int32_t *unstabl
     for (int d = 0; d < e->n; ++d) nc[d] = e->hp[2 * d].ncell;
     ECHK(e, launch_finite_flags(e->mom.data(), nc.data(), e->n, e->dflags, e->stream));
     std::vector<int32_t> fl(e->n);
-    ECHK(e, hipMemcpyAsync(fl.data(), e->dflags, fl.size() * sizeof(int32_t), hipMemcpyDeviceToHost, e->stream));
-    ECHK(e, hipStreamSynchronize(e->stream));
+    const ReadBack::Part part{fl.data(), e->dflags, fl.size() * sizeof(int32_t)};
+    ECHK(e, e->back.copy(&part, 1, e->device, e->stream));
     int32_t bad = 0;
     for (int d = 0; d < e->n; ++d) {
         bad += fl[d] == 0;
