@@ -388,7 +388,7 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
     // structure of arrays (imexlb_config.stride_pad, addr_mode)
     h->geom = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
     if (c.stride_pad < 0 && c.addr_mode < 0) tile_geom((uint32_t)c.nx, (uint32_t)c.ny, h->elem, c.storage == IMEXLB_AA, h->geom);
-    h->block = c.block ? c.block : (h->geom.tl == 31 ? 256 : tile_block((uint64_t)c.nx * c.ny));
+    h->block = c.block ? c.block : (h->geom.tl == 31 ? 256 : tile_block((uint64_t)c.nx * c.ny, h->ncell));
     h->cpt = c.cells_per_thread ? c.cells_per_thread : 1;
     h->xcd = c.xcd_remap < 0 ? 1 : c.xcd_remap;
     h->ntl = c.nt_loads < 0 ? 1 : (c.nt_loads ? 1 : 0);
@@ -418,6 +418,8 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
         h->block = c.block ? c.block : 256;
         have = alloc_lattices();
     }
+    if (c.nt_loads < 0 && h->geom.tl != 31)
+        h->ntl = tile_nt_loads(h->lat_bytes, c.storage == IMEXLB_AA, h->elem) ? 1 : 0;
     if (!have) return bail(fail(h, IMEXLB_ENOMEM, "lattice of %zu bytes", h->lat_bytes));
     h->device_bytes += (int64_t)nlat * (int64_t)h->lat_bytes;
     for (int k = 0; k < 4; ++k) {

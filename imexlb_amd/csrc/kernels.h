@@ -155,14 +155,38 @@ inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, bool aa, LatGeom 
     return true;
 }
 
-// Threads per workgroup of the plane-tile kernels where the caller names
-// none: the largest of 256, 192, 128 and 64 that leaves at most a sixteenth of
-// the plane's threads idle, else the one that leaves the fewest.
-inline int tile_block(uint64_t plane)
+// The XCD-aware order of the plane-tile kernels (tile.h tile_block_of, with the
+// measurements): one run of the lattice per XCD (1) where the lattices of a
+// step fit the caches it hopes to find them in -- the 256 MB last-level cache
+// for AA, whose step writes what it reads, the L2s' 32 MB for pull -- else runs of
+// eight workgroups.
+constexpr int XCD_RUNS = 2;
+inline int tile_order(uint64_t lattice_bytes, bool aa)
 {
+    return (aa ? lattice_bytes : 2 * lattice_bytes) <= (uint64_t(aa ? 256 : 32) << 20) ? 1 : XCD_RUNS;
+}
+
+// Default for non-temporal loads (imexlb_config.nt_loads) over plane tiles: not
+// where an AA lattice stays in the caches and its elements are small (us per
+// step, non-temporal / plain: FP16 160^3 81.1 / 63.6, 128^3 39.8 / 34.6, 48^3 4.8 / 4.5; FP32
+// 64^3 8.4 / 7.9, but 96^3 30.6 / 31.6; FP64 64^3 20.5 / 20.7, 128^3 142 / 171).
+inline bool tile_nt_loads(uint64_t lattice_bytes, bool aa, uint64_t elem)
+{
+    return !aa || elem == 8 || lattice_bytes > (uint64_t(elem == 2 ? 256 : 64) << 20);
+}
+
+// Threads per workgroup of the plane-tile kernels where the caller names
+// none: 64 below 200000 cells, where the chip has more compute units than there are
+// larger workgroups (us per step, 64 / 256: TGV 24^3 FP64 AA 4.9 / 5.8, 32^3 5.7 / 6.3, 40^3
+// 7.4 / 9.0, 56^3 14.5 / 14.8, 64^3 20.3 / 20.3 and FP16 7.0 / 6.8); above, the largest of
+// 256, 128 and 64 that leaves at most a sixteenth of the plane's threads idle, else
+// the one that leaves the fewest.
+inline int tile_block(uint64_t plane, uint64_t cells)
+{
+    if (cells < 200000) return 64;
     int best = 256;
     uint64_t idle_best = ~uint64_t(0);
-    for (int b = 256; b >= 64; b -= 64) {
+    for (int b = 256; b >= 64; b /= 2) {
         const uint64_t idle = (plane + b - 1) / b * b - plane;
         if (idle * 16 <= plane) return b;
         if (idle < idle_best) {
@@ -212,7 +236,7 @@ struct FusedParams {
     double corr[Q];          // cavity: moving-lid term for a link crossing z = nz
     double feq_in[Q];        // channel: inlet equilibrium, stored convention
     uint32_t nblocks;        // grid size (for the XCD-aware block order)
-    int xcd_remap;           // 1: give each XCD one contiguous run of tiles
+    int xcd_remap;           // 1: give each XCD one contiguous run of tiles; plane tiles: tile_order
     int cpt;                 // cells per thread: 1, 2 (blockDim apart) or 3 (two adjacent
                              // x cells; periodic lattices with nx even, else 1)
     int ntl;                 // 1: non-temporal loads of unshared lines

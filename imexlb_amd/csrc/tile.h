@@ -246,21 +246,24 @@ __device__ __forceinline__ void tile_scatter(const FusedParams &P, const TileCtx
     }
 }
 
-// XCD-aware order of the workgroups over plane tiles: runs of eight consecutive
-// workgroups per XCD, the eight XCDs' runs side by side.  The lines that the
-// x-shifted rows of neighbouring workgroups share then mostly stay in one L2
-// while the chip sweeps one window of the lattice.  Step times in us, linear
-// / one run per XCD / runs of 8, block 256 (pull unless said): TGV 256^3 FP64 1292 /
-// 1218 / 1209, FP32 605 / 621 / 603, FP16 310 / 310 / 297, 301x203x157 FP32 337 / 367 / 342,
-// channel 512x256x256 FP16 640 / 702 / 637, cavity 128^3 FP64 AA 149.6 / 149.6 / 146.0.
-// Grids that the chip holds at once stay linear (cavity 64^3 AA, 1024
-// workgroups, linear / runs of 8: FP64 22.3 / 23.4, FP32 10.8 / 12.4, FP16 8.0 / 9.2;
-// 96^3, 3456 workgroups: 67.8 / 67.5, 33.8 / 33.2, 23.5 / 22.7).
-__device__ __forceinline__ uint32_t xcd_run(uint32_t b, uint32_t nb)
+// XCD-aware order of the workgroups over plane tiles (FusedParams::xcd_remap):
+// 1: one contiguous run of the lattice per XCD, which finds the lines it wrote
+// in the step before in its own L2 or, further out, still in the last-level
+// cache; XCD_RUNS: runs of eight consecutive workgroups per XCD, the eight
+// XCDs' runs side by side, so that the lines which the x-shifted rows of
+// neighbouring workgroups share mostly stay in one L2 while the chip sweeps one
+// window of the lattice.  tile_order chooses.  us per step, linear / one run /
+// runs of 8, block 256: pull TGV 256^3 FP64 1292 / 1218 / 1209, FP32 605 / 621 / 603, FP16
+// 310 / 310 / 297, 301x203x157 FP32 337 / 367 / 342, channel 512x256x256 FP16 640 / 702 /
+// 637, 96^3 FP32 34.8 / 37.4 / 34.7, 48^3 FP32 7.7 / 5.6 / 7.6; AA TGV 128^3 FP64 143.7 /
+// 144.7 / 141.9, 160^3 FP32 145 / 144 / 139, 128^3 FP32 67.6 / 65.7 / 67.3, 80^3 FP16 14.2 /
+// 10.8 / 13.0, 48^3 FP64 11.9 / 9.4 / 11.6.
+__device__ __forceinline__ uint32_t tile_block_of(const FusedParams &P, uint32_t b)
 {
     constexpr uint32_t RUN = 8, ALL = 8 * RUN;
+    if (P.xcd_remap == 1) return xcd_tile(b, P.nblocks);
     const uint32_t g = b / ALL, r = b % ALL;
-    return nb > 2048 && (g + 1) * ALL <= nb ? g * ALL + (r & 7u) * RUN + (r >> 3) : b;
+    return P.xcd_remap == XCD_RUNS && (g + 1) * ALL <= P.nblocks ? g * ALL + (r & 7u) * RUN + (r >> 3) : b;
 }
 
 // Before (structure of arrays, k_fused) and after, us per step, first
@@ -271,8 +274,7 @@ template <typename S, int BC, int PAT, int CPT, bool NTL>
 __global__ void __launch_bounds__(512) k_tiled(const FusedParams P)
 {
     using R = typename RealOf<S>::type;
-    uint32_t b = blockIdx.x;
-    if (P.xcd_remap) b = xcd_run(b, P.nblocks);
+    const uint32_t b = tile_block_of(P, blockIdx.x);
     const uint32_t z = P.divb.div(b);
     const uint32_t p0 = (b - z * P.bpp) * blockDim.x * CPT + threadIdx.x;
     const S *src[3];
@@ -354,8 +356,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
     constexpr bool F64 = std::is_same<S, double>::value;
     constexpr bool WALLS = BC == BC_CAVITY;
     __shared__ RowEdges<R> in, out;
-    uint32_t b = blockIdx.x;
-    if (P.xcd_remap) b = xcd_run(b, P.nblocks);
+    const uint32_t b = tile_block_of(P, blockIdx.x);
     const uint32_t nx = P.nx, ny = P.ny, nz = P.nz, plane = nx * ny;
     const uint32_t z = P.divb.div(b), lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), per_row = nx >> 6;
@@ -504,7 +505,9 @@ template <typename S>
 hipError_t launch_tiled(int bc, int pattern, const FusedParams &P0, int block, hipStream_t st)
 {
     FusedParams P = P0;
-    const uint32_t rows = tile_rows(P.nx, block, lattice_elems(P.geom, (uint32_t)P.nz) * sizeof(S), bc, sizeof(S));
+    const uint64_t bytes = lattice_elems(P.geom, (uint32_t)P.nz) * sizeof(S);
+    P.xcd_remap = P.xcd_remap ? tile_order(bytes, pattern != PAT_PULL) : 0;
+    const uint32_t rows = tile_rows(P.nx, block, bytes, bc, sizeof(S));
     if (pattern == PAT_AA_ODD && rows > 0) {
         P.bpp = ((uint32_t)P.ny + rows - 1) / rows;
         P.divb.init(P.bpp);
