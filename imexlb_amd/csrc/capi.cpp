@@ -203,6 +203,7 @@ static void fill_fused_params(imexlb_handle *h, FusedParams &P, int src, int dst
     P.dst = h->lat[dst];
     P.mask = h->mask;
     P.tau0 = c.tau0;
+    P.inv_den = div_reciprocal(c.tau0 + 0.5);
     P.omega_f = (float)(1.0 / (c.tau0 + 0.5));
     P.shift = h->shift;
     P.ush = h->ush;

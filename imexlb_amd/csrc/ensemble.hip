@@ -447,6 +447,7 @@ int imexlb_ensemble_create(const imexlb_domain *doms, int n, int dtype, int stor
             P.mom_v = e->mom[4 * d + 2];
             P.mom_w = e->mom[4 * d + 3];
             P.tau0 = D.tau0;
+            P.inv_den = div_reciprocal(D.tau0 + 0.5);
             P.omega_f = (float)(1.0 / (D.tau0 + 0.5));
             P.shift = dtype == IMEXLB_F64 ? 0.0 : D.rho0;
             if (dtype != IMEXLB_F64) storage_shift(P.shift, 0.0, P.sh);

@@ -169,8 +169,53 @@ __device__ __forceinline__ R edu_of(int i, R u, R v, R w)
     return acc;
 }
 
+// Division by a divisor known in advance, correctly rounded: the IEEE quotient
+// bit for bit, from its rounded reciprocal y = RN(1 / b) and fused
+// multiply-adds (P. W. Markstein, "Computation of elementary functions on the
+// IBM RISC System/6000 processor", IBM J. Res. Dev. 34(1), 1990, theorem on
+// division: if q is within one ulp of x / b and r = x - b q is exact,
+// RN(q + r y) = RN(x / b); N. Brisebarre, J.-M. Muller and S. K. Raina,
+// "Accelerating correctly rounded floating-point division when the divisor is
+// known in advance", IEEE Trans. Comput. 53(8), 2004).  RN(x y) is within one ulp
+// where |b y - 1| <= 2^-54, as for b = 3; for any other b it is within 1.5, and a
+// first correction brings it below one.  Nothing may underflow or overflow on
+// the way: div_safe.  The compiler's division is eleven operations, one of
+// them at a quarter of the rate; a cell has 54.
+__device__ __forceinline__ double div_by_3(double x)
+{
+    constexpr double y = 1.0 / 3.0;
+    const double q = x * y;
+    return __builtin_fma(-__builtin_fma(3.0, q, -x), y, q);
+}
+__device__ __forceinline__ double div_by(double x, double b, double y)
+{
+    double q = x * y;
+    q = __builtin_fma(-__builtin_fma(b, q, -x), y, q);
+    return __builtin_fma(-__builtin_fma(b, q, -x), y, q);
+}
+
+// Whether div_by_3 and div_by serve for a cell's populations: every |f| in
+// [2^-600, 2^401).  Then f / 3 is far from the limits, and f - feq is 0 or at least
+// 2^-760 in size: it is f itself, to a factor near 1, where |feq| < 2^-700, and a
+// multiple of the smaller one's ulp elsewhere.  The divisor is held to
+// [2^-10, 2^30] on the host (div_reciprocal).  Zeros fail too, and take the IEEE
+// division.
+__device__ __forceinline__ bool div_safe(const double (&f)[Q])
+{
+    constexpr uint32_t LO = (1023u - 600u) << 21, SPAN = (1001u << 21) - 1;
+    uint32_t m = 0;
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+        // exponent and leading fraction, without the sign
+        const uint32_t t = ((uint32_t)(__builtin_bit_cast(uint64_t, f[i]) >> 32) << 1) - LO;
+        m = m > t ? m : t;
+    }
+    return m <= SPAN;
+}
+
 // Moments in direction order 0..26 (lid_driven_cavity/src/lbm.cpp:329-347):
 // p = sum f/3, u = sum f e.  FP64 storage: exactly the oracle's sums.
+template <bool SAFE = false>
 __device__ __forceinline__ void moments_f64(const double (&f)[Q], double &pm, double &um, double &vm, double &wm)
 {
 #pragma clang fp contract(off)
@@ -180,7 +225,7 @@ __device__ __forceinline__ void moments_f64(const double (&f)[Q], double &pm, do
     wm = 0.0;
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-        pm = pm + f[i] / 3.0;
+        pm = pm + (SAFE ? div_by_3(f[i]) : f[i] / 3.0);
         if (EX[i] > 0) um = um + f[i];
         if (EX[i] < 0) um = um - f[i];
         if (EY[i] > 0) vm = vm + f[i];
@@ -192,7 +237,9 @@ __device__ __forceinline__ void moments_f64(const double (&f)[Q], double &pm, do
 
 // BGK relaxation in the reference's operation order (tgv/src/lbm.cpp:228-234):
 // feq = t p 3 + t (3 e.u + 4.5 (e.u)^2 - 1.5 u.u); f -= (f - feq) / (tau0 + 0.5).
-__device__ __forceinline__ void collide_f64(double (&f)[Q], double pm, double u, double v, double w, double tau0)
+template <bool SAFE>
+__device__ __forceinline__ void collide_f64(double (&f)[Q], double pm, double u, double v, double w, double tau0,
+                                            double inv_den)
 {
     // every product and sum rounds separately, whatever the translation
     // unit's contraction setting: the FP64 path is the oracle's arithmetic
@@ -208,7 +255,7 @@ __device__ __forceinline__ void collide_f64(double (&f)[Q], double pm, double u,
         const double edu = edu_of<double>(i, u, v, w);
         const double eu2 = edu * edu;
         const double feq = tp3[WCLASS[i]] + WVAL[WCLASS[i]] * (3.0 * edu + 4.5 * eu2 - u15);
-        f[i] = f[i] - (f[i] - feq) / den;
+        f[i] = f[i] - (SAFE ? div_by(f[i] - feq, den, inv_den) : (f[i] - feq) / den);
     }
 }
 
@@ -518,52 +565,63 @@ __device__ __forceinline__ void cell_gather(const FusedParams &P, const CellCtx 
     }
 }
 
+// Moments, boundary overrides and collision of an FP64 cell.
+template <int BC, bool SAFE>
+__device__ __forceinline__ void cell_collide_f64(const FusedParams &P, const CellCtx &k, double (&f)[Q],
+                                                 bool write_moments)
+{
+    const uint32_t c = k.c;
+    double pm, um, vm, wm;
+    moments_f64<SAFE>(f, pm, um, vm, wm);
+    if constexpr (BC == BC_FAITHFUL) {
+        if (P.faithful_sphere) {
+            // sphere/src/lbm.cpp:399-412: u, p *= usr; the inlet plane
+            // takes the parabolic profile in z, the outlet plane p = 0
+            const double m = P.mask[c] == 1 ? 0.0 : 1.0;
+            um = um * m;
+            vm = vm * m;
+            wm = wm * m;
+            pm = pm * m;
+            const int glz = P.nz, kz = (int)k.z;
+            const double gm = (double)(glz - 1);
+            const double uin = P.u0 * 4.0 * (double)kz * (double)(glz - 1 - kz) / (gm * gm);
+            um = k.x0 ? uin : um;
+            vm = k.x0 ? 0.0 : vm;
+            wm = k.x0 ? 0.0 : wm;
+            pm = k.x1 ? 0.0 : pm;
+        } else {
+            // the reference's lid: Update sets ua = 0.1 on the top fluid
+            // layer (lid_driven_cavity/src/lbm.cpp:343-344)
+            um = k.z1 ? 0.1 : um;
+        }
+    }
+    if (write_moments && k.live) {
+        *glb(P.mom_p + c) = pm;
+        *glb(P.mom_u + c) = um;
+        *glb(P.mom_v + c) = vm;
+        *glb(P.mom_w + c) = wm;
+    }
+    collide_f64<SAFE>(f, pm, um, vm, wm, P.tau0, P.inv_den);
+}
+
 template <typename S, int BC>
 __device__ __forceinline__ void cell_collide(const FusedParams &P, const CellCtx &k,
                                              typename RealOf<S>::type (&f)[Q], bool write_moments)
 {
     constexpr bool F64 = std::is_same<S, double>::value;
-    const uint32_t c = k.c;
     if constexpr (F64) {
-        double pm, um, vm, wm;
-        moments_f64(f, pm, um, vm, wm);
-        if constexpr (BC == BC_FAITHFUL) {
-            if (P.faithful_sphere) {
-                // sphere/src/lbm.cpp:399-412: u, p *= usr; the inlet plane
-                // takes the parabolic profile in z, the outlet plane p = 0
-                const double m = P.mask[c] == 1 ? 0.0 : 1.0;
-                um = um * m;
-                vm = vm * m;
-                wm = wm * m;
-                pm = pm * m;
-                const int glz = P.nz, kz = (int)k.z;
-                const double gm = (double)(glz - 1);
-                const double uin = P.u0 * 4.0 * (double)kz * (double)(glz - 1 - kz) / (gm * gm);
-                um = k.x0 ? uin : um;
-                vm = k.x0 ? 0.0 : vm;
-                wm = k.x0 ? 0.0 : wm;
-                pm = k.x1 ? 0.0 : pm;
-            } else {
-                // the reference's lid: Update sets ua = 0.1 on the top fluid
-                // layer (lid_driven_cavity/src/lbm.cpp:343-344)
-                um = k.z1 ? 0.1 : um;
-            }
-        }
-        if (write_moments) {
-            *glb(P.mom_p + c) = pm;
-            *glb(P.mom_u + c) = um;
-            *glb(P.mom_v + c) = vm;
-            *glb(P.mom_w + c) = wm;
-        }
-        collide_f64(f, pm, um, vm, wm, P.tau0);
+        // the choice between the divisions is tile_finish's: here it would cost
+        // a wavefront per SIMD (k_fused 120-146 registers, 166-196 with it)
+        cell_collide_f64<BC, false>(P, k, f, write_moments);
     } else {
+        const uint32_t c = k.c;
         double pd;
         float u, v, w;
         moments_lp(f, pd, u, v, w);
         if constexpr (BC == BC_CHANNEL) {
             // populations stored relative to the inflow equilibrium: the
             // moments above are the departure from the free stream (U, 0, 0)
-            if (write_moments) {
+            if (write_moments && k.live) {
                 *glb(P.mom_p + c) = (pd + P.shift) / 3.0;
                 *glb(P.mom_u + c) = (double)u + P.ush;
                 *glb(P.mom_v + c) = v;
@@ -571,7 +629,7 @@ __device__ __forceinline__ void cell_collide(const FusedParams &P, const CellCtx
             }
             collide_lp_stream(f, pd, u, v, w, P.omega_f, (float)P.ush);
         } else {
-            if (write_moments) {
+            if (write_moments && k.live) {
                 *glb(P.mom_p + c) = (pd + P.shift) / 3.0;
                 *glb(P.mom_u + c) = u;
                 *glb(P.mom_v + c) = v;
@@ -809,6 +867,7 @@ __global__ void __launch_bounds__(512) k_fused_pair(const FusedParams P)
 
     CellCtx k;
     k.c = c;
+    k.live = true;
     cell_collide<S, BC_PERIODIC>(P, k, f0, P.mom_p != nullptr);
     k.c = c + 1;
     cell_collide<S, BC_PERIODIC>(P, k, f1, P.mom_p != nullptr);

@@ -228,6 +228,7 @@ struct FusedParams {
     double *mom_p, *mom_u, *mom_v, *mom_w;  // written when mom_p != nullptr
     const uint8_t *mask;     // channel: 0 fluid, 1 solid, 2 fluid next to solid
     double tau0;             // f <- f - (f - feq) / (tau0 + 0.5)
+    double inv_den;          // FP64: div_reciprocal(tau0 + 0.5)
     float omega_f;           // 1 / (tau0 + 0.5) for the FP32 collision
     double shift;            // reduced precision: S, with sum_i s_i = S (p = (sum g + S) / 3)
     double ush;              // reduced-precision channel: the shift's free-stream x velocity U
@@ -315,6 +316,10 @@ inline void storage_shift(double S, double U, double out[Q])
         }
     }
 }
+
+// RN(1 / b) for a divisor the kernels may divide by through its reciprocal
+// (fused.h div_by), 0 for one beyond [2^-10, 2^30].
+inline double div_reciprocal(double b) { return b >= 0x1p-10 && b <= 0x1p30 ? 1.0 / b : 0.0; }
 
 // Launchers (defined next to their kernels).
 hipError_t launch_fused(int dtype, int bc, int pattern, const FusedParams &P, int block, hipStream_t st);
