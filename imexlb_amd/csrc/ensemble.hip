@@ -21,7 +21,7 @@
 #include <vector>
 
 #include "../../include/imexlb.h"
-#include "fused.h"
+#include "tile.h"
 #include "readback.h"
 #include "window.h"
 #include "kernels.h"
@@ -30,8 +30,9 @@ namespace imx {
 
 struct EnsParams {
     const FusedParams *doms;  // two entries per domain: [2 d + parity]
-    const uint2 *tiles;       // (domain, first cell)
+    const uint2 *tiles;       // (domain, first cell; plane tiles: workgroup of the domain)
     uint32_t t0, ntiles;      // this launch's tiles: [t0, ntiles)
+    int order;                // tile.h tile_block_of
     int parity;               // pull: which lattice of each pair is read
     int write_moments;
 };
@@ -73,56 +74,69 @@ __device__ __forceinline__ T read_const(const T *p)
 #endif
 }
 
-// Persistent over one boundary kind's run of the tile table (or one
-// workgroup per tile, grid 0): every workgroup exits after its last tile.  One kernel per boundary kind keeps
-// each at the registers of its own cell code (the periodic and cavity code in
-// one kernel held FP32 pull at 98 VGPRs and the AA odd step at 138, against
-// 68 and 108 for the periodic code alone).
-template <typename S, int BC, int PAT, int CPT>
+// Persistent over one run of the tile table (or one workgroup per tile, grid
+// 0): every workgroup exits after its last tile.  Members in plane tiles
+// (TILED: every plane of 512 cells or more) run tile.h's cells, periodic and cavity
+// in one launch, the choice being the workgroup's; members in arrays run
+// fused.h's, one launch per boundary kind (BC), since both kinds in one kernel
+// would hold the registers of the larger.  15 members of 32^3-96^3, us a step: FP32
+// pull 243 in arrays with 2048 persistent workgroups (the default before), 233 in
+// arrays with one workgroup per tile, 202 in tiles, 196 with one launch for both
+// kinds (218 persistent); FP64 pull 475 -> 389, FP16 AA 142 -> 113.
+template <typename S, int BC, int PAT, int CPT, bool TILED>
 __global__ void __launch_bounds__(512) k_ensemble(const EnsParams EP)
 {
     const bool wm = EP.write_moments != 0;
     const uint32_t count = EP.ntiles - EP.t0;
     for (uint32_t v = blockIdx.x; v < count; v += gridDim.x) {
         // XCD-aware order (v and blockIdx.x agree mod 8 when the grid is a
-        // multiple of 8, as the tuned grids are): each XCD walks one
-        // contiguous part of the run, so neighbouring tiles share its L2
-        const uint32_t t = EP.t0 + xcd_tile(v, count);
+        // multiple of 8, as the tuned grids are)
+        const uint32_t t = EP.t0 + (TILED ? tile_block_of(EP.order, v, count) : xcd_tile(v, count));
         const uint2 tl = read_const(EP.tiles + t);
-        const FusedParams P = read_const(EP.doms + 2 * tl.x + (uint32_t)EP.parity);
+        FusedParams P = read_const(EP.doms + 2 * tl.x + (uint32_t)EP.parity);
         // non-temporal loads of unshared lines (measured faster on every
         // storage type of the single-domain kernel)
-        tile_run<S, BC, PAT, CPT, true>(P, tl.y, wm);
+        if constexpr (TILED) {
+            if (!wm) P.mom_p = nullptr;
+            const uint32_t z = P.divb.div(tl.y);
+            const uint32_t p0 = (tl.y - z * P.bpp) * blockDim.x * CPT + threadIdx.x;
+            if (P.bc == BC_PERIODIC) tile_cells<S, BC_PERIODIC, PAT, CPT, true>(P, z, p0);
+            else tile_cells<S, BC_CAVITY, PAT, CPT, true>(P, z, p0);
+        } else {
+            tile_run<S, BC, PAT, CPT, true>(P, tl.y, wm);
+        }
     }
 }
 
-template <typename S, int BC, int CPT>
+template <typename S, int BC, int CPT, bool TILED>
 static hipError_t launch_ens_bc(int pattern, const EnsParams &EP, int grid, int block, hipStream_t st)
 {
     if (pattern == PAT_PULL)
-        hipLaunchKernelGGL((k_ensemble<S, BC, PAT_PULL, CPT>), dim3(grid), dim3(block), 0, st, EP);
+        hipLaunchKernelGGL((k_ensemble<S, BC, PAT_PULL, CPT, TILED>), dim3(grid), dim3(block), 0, st, EP);
     else if (pattern == PAT_AA_EVEN)
-        hipLaunchKernelGGL((k_ensemble<S, BC, PAT_AA_EVEN, CPT>), dim3(grid), dim3(block), 0, st, EP);
-    else hipLaunchKernelGGL((k_ensemble<S, BC, PAT_AA_ODD, CPT>), dim3(grid), dim3(block), 0, st, EP);
+        hipLaunchKernelGGL((k_ensemble<S, BC, PAT_AA_EVEN, CPT, TILED>), dim3(grid), dim3(block), 0, st, EP);
+    else hipLaunchKernelGGL((k_ensemble<S, BC, PAT_AA_ODD, CPT, TILED>), dim3(grid), dim3(block), 0, st, EP);
     return hipGetLastError();
 }
 
 template <typename S, int CPT>
-static hipError_t launch_ens_cpt(int bc, int pattern, const EnsParams &EP, int grid, int block, hipStream_t st)
+static hipError_t launch_ens_cpt(int bc, bool tiled, int pattern, const EnsParams &EP, int grid, int block,
+                                 hipStream_t st)
 {
-    if (bc == BC_PERIODIC) return launch_ens_bc<S, BC_PERIODIC, CPT>(pattern, EP, grid, block, st);
-    return launch_ens_bc<S, BC_CAVITY, CPT>(pattern, EP, grid, block, st);
+    if (tiled) return launch_ens_bc<S, BC_PERIODIC, CPT, true>(pattern, EP, grid, block, st);
+    if (bc == BC_PERIODIC) return launch_ens_bc<S, BC_PERIODIC, CPT, false>(pattern, EP, grid, block, st);
+    return launch_ens_bc<S, BC_CAVITY, CPT, false>(pattern, EP, grid, block, st);
 }
 
-static hipError_t launch_ensemble(int dtype, int cpt, int bc, int pattern, const EnsParams &EP, int grid,
+static hipError_t launch_ensemble(int dtype, int cpt, int bc, bool tiled, int pattern, const EnsParams &EP, int grid,
                                   int block, hipStream_t st)
 {
-    if (dtype == DT_F64) return cpt == 2 ? launch_ens_cpt<double, 2>(bc, pattern, EP, grid, block, st)
-                                         : launch_ens_cpt<double, 1>(bc, pattern, EP, grid, block, st);
-    if (dtype == DT_F32) return cpt == 2 ? launch_ens_cpt<float, 2>(bc, pattern, EP, grid, block, st)
-                                         : launch_ens_cpt<float, 1>(bc, pattern, EP, grid, block, st);
-    return cpt == 2 ? launch_ens_cpt<_Float16, 2>(bc, pattern, EP, grid, block, st)
-                    : launch_ens_cpt<_Float16, 1>(bc, pattern, EP, grid, block, st);
+    if (dtype == DT_F64) return cpt == 2 ? launch_ens_cpt<double, 2>(bc, tiled, pattern, EP, grid, block, st)
+                                         : launch_ens_cpt<double, 1>(bc, tiled, pattern, EP, grid, block, st);
+    if (dtype == DT_F32) return cpt == 2 ? launch_ens_cpt<float, 2>(bc, tiled, pattern, EP, grid, block, st)
+                                         : launch_ens_cpt<float, 1>(bc, tiled, pattern, EP, grid, block, st);
+    return cpt == 2 ? launch_ens_cpt<_Float16, 2>(bc, tiled, pattern, EP, grid, block, st)
+                    : launch_ens_cpt<_Float16, 1>(bc, tiled, pattern, EP, grid, block, st);
 }
 
 }  // namespace imx
@@ -135,8 +149,9 @@ struct imexlb_ensemble {
     std::vector<imexlb_domain> doms;
     std::vector<FusedParams> hp;         // host copy of the domain table
     FusedParams *dp = nullptr;           // device domain table
-    std::vector<uint2> tiles;            // periodic domains' tiles first, then the cavities'
-    uint32_t ntiles_periodic = 0;
+    // one run per boundary kind and layout (run_of), the periodic first
+    std::vector<uint2> tiles;
+    uint32_t bounds[4] = {0, 0, 0, 0};
     uint2 *dtiles = nullptr;
     void *pool = nullptr;                // every lattice, in one allocation
     ChunkedWindow win;                   // the address range pool lies in when a window search placed it
@@ -184,25 +199,39 @@ static void drop_graph(imexlb_ensemble *e)
     e->graph_parity = -1;
 }
 
+// The run of the tile table a member belongs to.
+static int run_of(const FusedParams &P) { return P.geom.tl != 31 ? 0 : P.bc == BC_PERIODIC ? 1 : 2; }
+
 static void build_tiles(imexlb_ensemble *e)
 {
     e->tiles.clear();
     const uint32_t tile = (uint32_t)e->block * (uint32_t)e->cpt;
-    // one run per boundary kind (periodic first), largest domains first
-    // within each, so the tail of each run is made of small work
+    // largest domains first within each run, so that its tail is made of
+    // small work
     std::vector<int> order(e->n);
     for (int d = 0; d < e->n; ++d) order[d] = d;
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
         const FusedParams &A = e->hp[2 * a], &B = e->hp[2 * b];
-        if ((A.bc == BC_PERIODIC) != (B.bc == BC_PERIODIC)) return A.bc == BC_PERIODIC;
+        if (run_of(A) != run_of(B)) return run_of(A) < run_of(B);
+        if (run_of(A) == 0 && A.bc != B.bc) return A.bc == BC_PERIODIC;
         return A.ncell > B.ncell;
     });
-    e->ntiles_periodic = 0;
-    for (int d : order)
-        for (uint32_t c = 0; c < e->hp[2 * d].ncell; c += tile) {
-            e->tiles.push_back(make_uint2((uint32_t)d, c));
-            if (e->hp[2 * d].bc == BC_PERIODIC) ++e->ntiles_periodic;
+    for (uint32_t &b : e->bounds) b = 0;
+    for (int d : order) {
+        const FusedParams &A = e->hp[2 * d];
+        const uint32_t plane = (uint32_t)A.nx * (uint32_t)A.ny;
+        if (A.geom.tl == 31) {
+            for (uint32_t c = 0; c < A.ncell; c += tile) e->tiles.push_back(make_uint2((uint32_t)d, c));
+        } else {
+            const uint32_t bpp = (plane + tile - 1) / tile;
+            for (int par = 0; par < 2; ++par) {
+                e->hp[2 * d + par].bpp = bpp;
+                e->hp[2 * d + par].divb.init(bpp);
+            }
+            for (uint32_t b = 0; b < bpp * (uint32_t)A.nz; ++b) e->tiles.push_back(make_uint2((uint32_t)d, b));
         }
+        for (int r = run_of(A) + 1; r < 4; ++r) e->bounds[r] = (uint32_t)e->tiles.size();
+    }
 }
 
 static int upload_tables(imexlb_ensemble *e)
@@ -250,16 +279,16 @@ static int launch_persistent(imexlb_ensemble *e, int pattern, int parity, bool w
     EP.tiles = e->dtiles;
     EP.parity = parity;
     EP.write_moments = wm ? 1 : 0;
-    // the periodic run, then the cavity run, back to back on the stream
-    const uint32_t bounds[3] = {0, e->ntiles_periodic, (uint32_t)e->tiles.size()};
-    const int kinds[2] = {BC_PERIODIC, BC_CAVITY};
-    for (int r = 0; r < 2; ++r) {
-        if (bounds[r + 1] == bounds[r]) continue;
-        EP.t0 = bounds[r];
-        EP.ntiles = bounds[r + 1];
-        const int count = (int)(bounds[r + 1] - bounds[r]);
+    EP.order = tile_order(e->pool_bytes / (e->storage == IMEXLB_PULL ? 2 : 1), e->storage == IMEXLB_AA);
+    // the runs, back to back on the stream
+    for (int r = 0; r < 3; ++r) {
+        if (e->bounds[r + 1] == e->bounds[r]) continue;
+        EP.t0 = e->bounds[r];
+        EP.ntiles = e->bounds[r + 1];
+        const int count = (int)(EP.ntiles - EP.t0);
         const int grid = e->grid == 0 ? count : std::min<int>(e->grid, count);
-        ECHK(e, launch_ensemble(e->dtype, e->cpt, kinds[r], pattern, EP, grid, e->block, e->stream));
+        ECHK(e, launch_ensemble(e->dtype, e->cpt, r == 2 ? BC_CAVITY : BC_PERIODIC, r == 0, pattern, EP, grid, e->block,
+                                e->stream));
     }
     return IMEXLB_OK;
 }
@@ -390,7 +419,6 @@ int imexlb_ensemble_create(const imexlb_domain *doms, int n, int dtype, int stor
     if (hipSetDevice(device) != hipSuccess || hipStreamCreate(&e->stream) != hipSuccess) return bail(IMEXLB_EHIP);
     int cus = 256;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && cus > 0) e->cus = cus;
-    e->grid = e->cus * 8;
     const size_t elem = dtype == IMEXLB_F64 ? 8 : (dtype == IMEXLB_F32 ? 4 : 2);
     e->hp.resize(2 * (size_t)n);
     e->lat.assign(2 * (size_t)n, nullptr);
@@ -398,22 +426,35 @@ int imexlb_ensemble_create(const imexlb_domain *doms, int n, int dtype, int stor
     // One pool for all lattices, each on a 4 KiB boundary: the step rate
     // depends on where a lattice's pages land, and a single allocation can be
     // swapped for a faster one as a whole (imexlb_ensemble_tune_placement).
-    // Population stride as in the single-domain engine: the cell count
-    // rounded up to 256 bytes plus the pad that staggers the 27 streams.
+    // Plane tiles or, for small planes or where only those fit, arrays with the
+    // population stride of the single-domain engine: the cell count rounded up
+    // to 256 bytes plus the pad that staggers the 27 streams.
     const int nl = storage == IMEXLB_PULL ? 2 : 1;
     std::vector<uint64_t> pstride(n);
+    std::vector<LatGeom> geom(n);
+    auto alloc_pool = [&](bool tiles) {
+        e->pool_bytes = 0;
+        for (int d = 0; d < n; ++d) {
+            geom[d] = soa_geom((uint32_t)doms[d].nx, (uint32_t)doms[d].ny, pstride[d]);
+            if (tiles) tile_geom((uint32_t)doms[d].nx, (uint32_t)doms[d].ny, elem, storage == IMEXLB_AA, geom[d]);
+            for (int k = 0; k < nl; ++k) {
+                e->lat_off[2 * d + k] = e->pool_bytes;
+                e->pool_bytes += ((size_t)lattice_elems(geom[d], (uint32_t)doms[d].nz) * elem + 4095) / 4096 * 4096;
+            }
+        }
+        if (hipMalloc(&e->pool, e->pool_bytes) == hipSuccess) return true;
+        (void)hipGetLastError();
+        e->pool = nullptr;
+        return false;
+    };
     for (int d = 0; d < n; ++d) {
         const uint64_t nc = (uint64_t)doms[d].nx * doms[d].ny * doms[d].nz, per = 256 / elem;
         pstride[d] = (nc + per - 1) / per * per + (uint64_t)IMEXLB_DEFAULT_PAD / elem;
         // the member kernels address a group of populations (16 bytes of
         // stride per cell, PopGroup) with 32-bit byte offsets
         if (pstride[d] * 16 > (1ull << 32)) return bail(IMEXLB_EINVAL);
-        for (int k = 0; k < nl; ++k) {
-            e->lat_off[2 * d + k] = e->pool_bytes;
-            e->pool_bytes += ((size_t)Q * pstride[d] * elem + 4095) / 4096 * 4096;
-        }
     }
-    if (hipMalloc(&e->pool, e->pool_bytes) != hipSuccess) return bail(IMEXLB_ENOMEM);
+    if (!alloc_pool(true) && !alloc_pool(false)) return bail(IMEXLB_ENOMEM);
     e->device_bytes += (int64_t)e->pool_bytes;
     for (int d = 0; d < n; ++d)
         for (int k = 0; k < nl; ++k) e->lat[2 * d + k] = (char *)e->pool + e->lat_off[2 * d + k];
@@ -435,7 +476,7 @@ int imexlb_ensemble_create(const imexlb_domain *doms, int n, int dtype, int stor
             P.nz = D.nz;
             P.ncell = nc;
             P.pstride = pstride[d];
-            P.geom = soa_geom((uint32_t)P.nx, (uint32_t)P.ny, pstride[d]);
+            P.geom = geom[d];
             if (storage == IMEXLB_PULL) {
                 P.src = e->lat[2 * d + par];
                 P.dst = e->lat[2 * d + 1 - par];

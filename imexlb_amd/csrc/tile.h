@@ -281,25 +281,20 @@ __device__ __forceinline__ void tile_finish(const FusedParams &P, const TileCtx 
 // 637, 96^3 FP32 34.8 / 37.4 / 34.7, 48^3 FP32 7.7 / 5.6 / 7.6; AA TGV 128^3 FP64 143.7 /
 // 144.7 / 141.9, 160^3 FP32 145 / 144 / 139, 128^3 FP32 67.6 / 65.7 / 67.3, 80^3 FP16 14.2 /
 // 10.8 / 13.0, 48^3 FP64 11.9 / 9.4 / 11.6.
-__device__ __forceinline__ uint32_t tile_block_of(const FusedParams &P, uint32_t b)
+__device__ __forceinline__ uint32_t tile_block_of(int order, uint32_t b, uint32_t nb)
 {
     constexpr uint32_t RUN = 8, ALL = 8 * RUN;
-    if (P.xcd_remap == 1) return xcd_tile(b, P.nblocks);
+    if (order == 1) return xcd_tile(b, nb);
     const uint32_t g = b / ALL, r = b % ALL;
-    return P.xcd_remap == XCD_RUNS && (g + 1) * ALL <= P.nblocks ? g * ALL + (r & 7u) * RUN + (r >> 3) : b;
+    return order == XCD_RUNS && (g + 1) * ALL <= nb ? g * ALL + (r & 7u) * RUN + (r >> 3) : b;
 }
 
-// Before (structure of arrays, k_fused) and after, us per step, first
-// allocations: TGV 256^3 FP64 pull 1342 -> 1209 (5.99 TB/s algorithmic), 301x203x157
-// FP32 pull 414 -> 342, channel 512x256x256 FP16 712 -> 637, the reference's sphere
-// 512x128x128 715 -> 642 with its boundary kernels, cavity 128^3 FP64 AA 153 -> 146.
+// CPT cells per thread, blockDim.x apart, of plane z from cell p0; the loads of
+// all are issued before any of them is collided.
 template <typename S, int BC, int PAT, int CPT, bool NTL>
-__global__ void __launch_bounds__(512) k_tiled(const FusedParams P)
+__device__ __forceinline__ void tile_cells(const FusedParams &P, uint32_t z, uint32_t p0)
 {
     using R = typename RealOf<S>::type;
-    const uint32_t b = tile_block_of(P, blockIdx.x);
-    const uint32_t z = P.divb.div(b);
-    const uint32_t p0 = (b - z * P.bpp) * blockDim.x * CPT + threadIdx.x;
     const S *src[3];
     S *dst[3];
     tile_planes<const S, BC>((const S *)P.src, P, z, src);
@@ -329,6 +324,18 @@ __global__ void __launch_bounds__(512) k_tiled(const FusedParams P)
     for (int r = 0; r < CPT; ++r) tile_gather<S, BC, PAT, NTL>(P, t[r], src, f[r]);
 #pragma unroll
     for (int r = 0; r < CPT; ++r) tile_finish<S, BC, PAT>(P, t[r], dst, f[r]);
+}
+
+// Before (structure of arrays, k_fused) and after, us per step, first
+// allocations: TGV 256^3 FP64 pull 1342 -> 1202 (6.03 TB/s algorithmic), 301x203x157
+// FP32 pull 414 -> 340, channel 512x256x256 FP16 712 -> 615, the reference's sphere
+// 512x128x128 715 -> 642 with its boundary kernels, cavity 128^3 FP64 AA 153 -> 136.
+template <typename S, int BC, int PAT, int CPT, bool NTL>
+__global__ void __launch_bounds__(512) k_tiled(const FusedParams P)
+{
+    const uint32_t b = tile_block_of(P.xcd_remap, blockIdx.x, P.nblocks);
+    const uint32_t z = P.divb.div(b);
+    tile_cells<S, BC, PAT, CPT, NTL>(P, z, (b - z * P.bpp) * blockDim.x * CPT + threadIdx.x);
 }
 
 // The value of the lane before (EXP 1) or after (EXP -1); the first (last)
@@ -371,7 +378,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
     constexpr bool F64 = std::is_same<S, double>::value;
     constexpr bool WALLS = BC == BC_CAVITY;
     __shared__ RowEdges<R> in, out;
-    const uint32_t b = tile_block_of(P, blockIdx.x);
+    const uint32_t b = tile_block_of(P.xcd_remap, blockIdx.x, P.nblocks);
     const uint32_t nx = P.nx, ny = P.ny, nz = P.nz, plane = nx * ny;
     const uint32_t z = P.divb.div(b), lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), per_row = nx >> 6;

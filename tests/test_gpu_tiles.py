@@ -83,3 +83,33 @@ def test_row_kernel_equals_arrays(case, mode, n, dtype):
     want = state(n, 5, addr_mode=2, **kw)
     for shape in (None, (512, 1, 0, 0)):
         same(state(n, 5, shape, **kw), want, f"launch {shape}")
+
+
+@pytest.mark.parametrize("dtype,storage", [("f64", "pull"), ("f64", "aa"), ("f32", "pull"), ("f16", "aa")])
+def test_ensemble_mixes_layouts(dtype, storage):
+    """Members in plane tiles and in arrays (planes below 512 cells), periodic
+    and cavity, ragged: each steps as the single domain does."""
+    from imexlb_amd import LBM, Ensemble
+    print(f"[case] ensemble layouts {dtype} {storage}", flush=True)
+    sizes = [(0, 20, 21, 7), (1, 45, 37, 5), (0, 33, 31, 6), (1, 12, 10, 9), (0, 64, 64, 3), (1, 129, 9, 4)]
+    doms = [dict(case_id=c, nx=x, ny=y, nz=z, tau0=0.05 + 0.01 * k, rho0=1.0, u0=0.05, lid_u=0.08)
+            for k, (c, x, y, z) in enumerate(sizes)]
+    want = []
+    for d in doms:
+        g = LBM(d["nx"], d["ny"], d["nz"], d["tau0"], u0=0.05, lid_u=0.08, case="cavity" if d["case_id"] else "tgv",
+                mode="config" if d["case_id"] else "faithful", dtype=dtype, storage=storage, addr_mode=2)
+        g.Initialize()
+        g.step(7)
+        want.append(g.moments())
+        g.close()
+    e = Ensemble(doms, dtype=dtype, storage=storage)
+    for launch in (None, (64, 1, 24), (192, 2, 0), (512, 1, 8)):
+        if launch:
+            e.set_launch(*launch)
+        for mode in ("persistent", "graph", "per_domain"):
+            e.Initialize()
+            e.step(7, mode=mode)
+            for k in range(len(doms)):
+                for name, a, b in zip("puvw", want[k], e.moments(k)):
+                    assert np.array_equal(a, b), f"member {k} {name}, launch {launch}, {mode}"
+    e.close()
