@@ -158,12 +158,12 @@ inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, bool aa, LatGeom 
 // The XCD-aware order of the plane-tile kernels (tile.h tile_block_of, with the
 // measurements): one run of the lattice per XCD (1) where the lattices of a
 // step fit the caches it hopes to find them in -- the 256 MB last-level cache
-// for AA, whose step writes what it reads, the L2s' 32 MB for pull -- else runs of
-// eight workgroups.
+// for AA, whose step writes what it reads, 48 MB for pull, somewhat beyond the
+// L2s' 32 MB -- else runs of eight workgroups.
 constexpr int XCD_RUNS = 2;
 inline int tile_order(uint64_t lattice_bytes, bool aa)
 {
-    return (aa ? lattice_bytes : 2 * lattice_bytes) <= (uint64_t(aa ? 256 : 32) << 20) ? 1 : XCD_RUNS;
+    return (aa ? lattice_bytes : 2 * lattice_bytes) <= (uint64_t(aa ? 256 : 48) << 20) ? 1 : XCD_RUNS;
 }
 
 // Default for non-temporal loads (imexlb_config.nt_loads) over plane tiles: not
