@@ -514,34 +514,41 @@ __device__ __forceinline__ GhostSrc faithful_src(const FusedParams &P, int q, in
     return g;
 }
 
+// The coordinates of cell r of the ring (ring_index backwards).
+__device__ __forceinline__ void ring_cell(const FusedParams &P, uint32_t r, int &i, int &j, int &k)
+{
+    if (r < 2 * P.ring_a) {
+        const bool high = r >= P.ring_a;
+        r -= high ? P.ring_a : 0;
+        i = high ? P.nx : -1;
+        k = (int)(r / (uint32_t)(P.ny + 2));
+        j = (int)(r - (uint32_t)k * (uint32_t)(P.ny + 2)) - 1;
+        k -= 1;
+        return;
+    }
+    r -= 2 * P.ring_a;
+    const bool yf = r < 2 * P.ring_b;
+    r -= yf ? 0 : 2 * P.ring_b;
+    const uint32_t n = yf ? P.ring_b : P.ring_c;
+    const bool high = r >= n;
+    r -= high ? n : 0;
+    const int row = (int)P.divx.div(r);
+    i = (int)(r - (uint32_t)row * (uint32_t)P.nx);
+    j = yf ? (high ? P.ny : -1) : row;
+    k = yf ? row - 1 : (high ? P.nz : -1);
+}
+
 // Initialize for the ring: every first-layer ghost cell takes its initial
 // populations (0 in the cavity).
 __global__ void k_faithful_ring_init(const FusedParams P)
 {
-    uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= P.ring_n) return;
-    const uint32_t rr = r;
     int i, j, k;
-    if (r < 2 * P.ring_a) {
-        i = r < P.ring_a ? -1 : P.nx;
-        r -= r < P.ring_a ? 0 : P.ring_a;
-        j = (int)(r % (P.ny + 2)) - 1;
-        k = (int)(r / (P.ny + 2)) - 1;
-    } else if ((r -= 2 * P.ring_a) < 2 * P.ring_b) {
-        j = r < P.ring_b ? -1 : P.ny;
-        r -= r < P.ring_b ? 0 : P.ring_b;
-        i = (int)(r % P.nx);
-        k = (int)(r / P.nx) - 1;
-    } else {
-        r -= 2 * P.ring_b;
-        k = r < P.ring_c ? -1 : P.nz;
-        r -= r < P.ring_c ? 0 : P.ring_c;
-        i = (int)(r % P.nx);
-        j = (int)(r / P.nx);
-    }
+    ring_cell(P, r, i, j, k);
 #pragma unroll
     for (int q = 0; q < Q; ++q)
-        P.ring[(uint64_t)q * P.ring_n + rr] = P.faithful_sphere ? faithful_sphere_f0(P, P.seed, q, i, j, k) : 0.0;
+        P.ring[(uint64_t)q * P.ring_n + r] = P.faithful_sphere ? faithful_sphere_f0(P, P.seed, q, i, j, k) : 0.0;
 }
 
 hipError_t launch_faithful_ring_init(const FusedParams &P, hipStream_t st)
@@ -550,94 +557,216 @@ hipError_t launch_faithful_ring_init(const FusedParams &P, hipStream_t st)
     return hipGetLastError();
 }
 
-// The one-rank unpack of lid_driven_cavity/src/mpi_view_transfer.cpp:617-688
-// writes receive buffers nothing filled (zeros) into the ghost planes
-// y = ny, z = nz, x = -1 and x = nx, all 27 populations: here their cells of
-// the first layer.  Of a cell's 27 entries only those a wall writes later in
-// the step (the directions pointing into the cavity across any of the cell's
-// ghost axes) ever hold anything but zero: Initialize zeroes the ring and
-// nothing else writes it.  Those are zeroed again here; the others already
-// are.  Thread t: the two x faces, then the plane y = ny (x in [0, nx)),
-// then the plane z = nz (x in [0, nx), y in [-1, ny]).
-__global__ void k_faithful_unpack(const FusedParams P)
+// "usrbc", sphere/src/lbm.cpp:350-356: a solid cell takes, for each
+// direction q whose neighbour x + e_q is fluid, f_bb(q)(x + 2 e_q), in place
+// in the post-collision lattice.  The reference's mask covers the ghost
+// cells too: where the ball reaches the first ghost layer (ny or nz within r
+// of its centre), a ghost neighbour can be solid, and its mask value is
+// recomputed here.  A source is never a target: between two solid voxels of a
+// ball the midpoint voxel is solid too, so that direction is not taken.  The
+// (cell, q) pairs are therefore independent: thread t of direction q
+// takes cell t of the box [lo, lo + n)^3 around the ball (clamped to the
+// cavity), so that the few thousand cells of the box fill 27 times as many
+// lanes.  Every thread loads (threads off the box from a valid cell) and only
+// solid cells store: no load sits under a divergent branch.
+__device__ __forceinline__ void faithful_usr(const FusedParams &P, int lo, int n, int q, int t)
 {
-    const uint32_t t0 = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t nyz = (uint32_t)(P.ny + 2) * (P.nz + 2), nxz = (uint32_t)P.nx * (P.nz + 2),
-                   nxy = (uint32_t)P.nx * (P.ny + 2);
-    uint32_t t = t0;
-    int i, j, k;
-    if (t < 2 * nyz) {
-        const uint32_t f = t / nyz, r = t - f * nyz;
-        i = f ? P.nx : -1;
-        k = (int)(r / (P.ny + 2)) - 1;
-        j = (int)(r % (P.ny + 2)) - 1;
-    } else if ((t -= 2 * nyz) < nxz) {
-        j = P.ny;
-        k = (int)(t / P.nx) - 1;
-        i = (int)(t % P.nx);
-    } else if ((t -= nxz) < nxy) {
-        k = P.nz;
-        j = (int)(t / P.nx) - 1;
-        i = (int)(t % P.nx);
+    int e[3], bq;
+    dir_of(q, e, bq);
+    const int ex = e[0], ey = e[1], ez = e[2];
+    const int tt = t < n * n * n ? t : 0;
+    const int x0 = lo + tt % n, y0 = lo + (tt / n) % n, z0 = lo + tt / (n * n);
+    const bool valid = (t < n * n * n) & (x0 < P.nx) & (y0 < P.ny) & (z0 < P.nz);
+    const int x = valid ? x0 : 0, y = valid ? y0 : 0, z = valid ? z0 : 0;
+    const uint32_t c = ((uint32_t)z * P.ny + y) * P.nx + x;
+    const int xi = x + ex, yi = y + ey, zi = z + ez;
+    const bool in = (xi >= 0) & (xi < P.nx) & (yi >= 0) & (yi < P.ny) & (zi >= 0) & (zi < P.nz);
+    const uint64_t mi = in ? ((uint64_t)zi * P.ny + yi) * P.nx + xi : (uint64_t)c;
+    const GhostSrc g = faithful_src(P, bq, x + 2 * ex, y + 2 * ey, z + 2 * ez);
+    const uint8_t mc = P.mask[c];
+    const uint8_t m = P.mask[mi];
+    double v = *g.p;
+    v = g.is_deep ? g.deep : v;
+    const bool solid = valid & (mc == 1);
+    const bool nb_solid = in ? m == 1 : faithful_sphere_solid(P.nx, xi, yi, zi);
+    if (solid & !nb_solid) ((double *)P.src)[P.geom.off(q, (uint32_t)z, (uint32_t)y * P.nx + x)] = v;
+}
+
+__global__ void k_faithful_usr(const FusedParams P, int lo, int n)
+{
+    faithful_usr(P, lo, n, blockIdx.y, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+// The boundary phase on the ring, in one launch.  The reference fills the ghost
+// cells in several passes, each reading what an earlier one wrote:
+//   cavity: the one-rank unpack of lid_driven_cavity/src/mpi_view_transfer.cpp:
+//     617-688 zeroes the planes x = -1, x = nx, y = ny and z = nz (it copies
+//     receive buffers that nothing filled), then the x, y and z walls
+//     (lid_driven_cavity/src/lbm.cpp:233-301) write, for every first-layer cell
+//     of their plane and direction q pointing into the cavity,
+//     f_q(cell) = f_bb(q)(cell + 2 e_q on the plane n - 2 or 1 of their axis; the
+//     top wall takes one e_y instead of two);
+//   sphere: the y and z walls, then the inlet copy f_q(-1, y, z) = f_q(0, y, z) and
+//     the outlet copy f_q(nx, y, z) = f_q(nx - 1, y + e_y, z + e_z)
+//     (sphere/src/lbm.cpp:277-347).
+// Here every entry that a pass writes finds its value by itself: the last pass
+// that writes it names a source, of which an earlier pass may be the last
+// writer, and so on -- at most three times, always between q and bb(q) -- down to a
+// cell of the lattice, a ghost cell deeper than the first layer, a zeroed
+// plane, or an entry that no pass before it wrote this step and that therefore
+// still holds the last step's value.  Those are read from the last step's ring,
+// so the two rings change places every step and no thread reads what another
+// writes.  Entries that no pass writes hold Initialize's values in both.
+//
+// It is bound by latency, not by what it moves: the launches, and per thread one
+// load of what another XCD wrote last.  us a step, a launch per pass before / now:
+// cavity 100^3 20 / 8 of a step of 92 / 84, sphere 512x128x128 45 / 20 of
+// 640 / 626; whole steps: sphere 72x24x24 27 / 11, cavity 24x16x24 19 / 10.
+
+// Workgroups of one face of each axis, of one direction of the edges' cells, and
+// of one direction of the box [lo, lo + n)^3 around the ball (0: not here).
+struct RingBlocks {
+    uint32_t x, y, z, edges, ball;
+    int lo, n;
+};
+
+// One entry of the ring on its way to its value: the cell, the direction there
+// (q, or bb(q) when turned) and how many of the step's passes come before.
+struct RingEntry {
+    int i, j, k, turned, before;
+};
+
+// Follows the entry through the last pass before `before` that writes it
+// (passes 0, 1, 2: the cavity's x, y, z walls; the sphere's y and z walls and
+// its inlet and outlet); false: none does.
+template <bool SPHERE>
+__device__ __forceinline__ bool ring_hop(const FusedParams &P, const int e[3], RingEntry &t)
+{
+    const int nx = P.nx, ny = P.ny, nz = P.nz, sg = t.turned ? -1 : 1;
+    const int ex = sg * e[0], ey = sg * e[1], ez = sg * e[2];
+    const bool first = t.i >= -1 && t.i <= nx && t.j >= -1 && t.j <= ny && t.k >= -1 && t.k <= nz;
+    // written by the pass of an axis: a first-layer ghost cell of that axis, the
+    // direction pointing inward there
+    const bool in_x = first && ((t.i < 0 && ex > 0) || (t.i >= nx && ex < 0));
+    const bool in_y = first && ((t.j < 0 && ey > 0) || (t.j >= ny && ey < 0));
+    const bool in_z = first && ((t.k < 0 && ez > 0) || (t.k >= nz && ez < 0));
+    const bool copy = SPHERE && in_x && t.before > 2;
+    const bool wz = !copy && in_z && t.before > (SPHERE ? 1 : 2);
+    const bool wy = !copy && !wz && in_y && t.before > (SPHERE ? 0 : 1);
+    const bool wx = !SPHERE && !wz && !wy && in_x && t.before > 0;
+    const bool wall = wx || wy || wz;
+    const bool out = copy && ex < 0;
+    const int sy = wz && !SPHERE && ez < 0 ? 1 : 2;  // the cavity's top wall
+    t.i = copy ? (out ? nx - 1 : 0) : wx ? (ex > 0 ? 1 : nx - 2) : wall ? t.i + 2 * ex : t.i;
+    t.j = out ? t.j + ey : wy ? (ey > 0 ? 1 : ny - 2) : wall ? t.j + sy * ey : t.j;
+    t.k = out ? t.k + ez : wz ? (ez > 0 ? 1 : nz - 2) : wall ? t.k + 2 * ez : t.k;
+    t.before = copy ? 2 : wz ? (SPHERE ? 1 : 2) : wy ? (SPHERE ? 0 : 1) : 0;
+    t.turned = wall ? !t.turned : t.turned;
+    return copy || wall;
+}
+
+// What the entry holds once no pass before it writes it.
+template <bool SPHERE>
+__device__ __forceinline__ double ring_value(const FusedParams &P, const double *last, int q, int bq, const int e[3],
+                                             const RingEntry &t)
+{
+    const int c = t.turned ? bq : q, cx = t.turned ? -e[0] : e[0];
+    const int64_t rc = ring_index(P, t.i, t.j, t.k);
+    const bool inside = rc == -2, deep = rc == -1;
+    // an interior cell on the planes that the fused pass copies beside the
+    // lattice, y fastest (one strided cell per row of the lattice otherwise)
+    const bool lo = SPHERE ? t.i == 0 && cx > 0 : t.i == 1 && cx < 0;
+    const bool hi = SPHERE ? t.i == P.nx - 1 && cx < 0 : t.i == P.nx - 2 && cx > 0;
+    const double *p = last + (uint64_t)c * P.ring_n + (uint64_t)(rc < 0 ? 0 : rc);
+    if (inside)
+        p = lo || hi ? P.stage + (((uint64_t)(lo ? 0 : 1) * P.nz + t.k) * P.ny + t.j) * STAGE_ROW + x_rank(c)
+                     : (const double *)P.src + P.geom.off(c, (uint32_t)t.k, (uint32_t)t.j * P.nx + t.i);
+    double v = *p;
+    if (SPHERE) {
+        if (deep) v = faithful_sphere_f0(P, P.seed, c, t.i, t.j, t.k);
+    } else if (!inside && (deep || t.i < 0 || t.i >= P.nx || t.j >= P.ny || t.k >= P.nz)) {
+        v = 0.0;  // never written, or zeroed by the unpack
+    }
+    return v;
+}
+
+// Workgroups: where the ball lies clear of what the passes read, its usrbc; then
+// the edges' cells, three directions of the 27 to a row (the long
+// ways start early); then per face its cells with one ghost coordinate, row y the
+// y-th of the nine directions entering there (the pass of that axis writes it, and
+// nearly always its source lies inside).
+template <bool SPHERE>
+__global__ void __launch_bounds__(256) k_faithful_ring(const FusedParams P, const double *last, RingBlocks nb)
+{
+    const int nx = P.nx, ny = P.ny, nz = P.nz;
+    uint32_t b = blockIdx.x;
+    if (SPHERE && b < 3 * nb.ball) {
+        faithful_usr(P, nb.lo, nb.n, 3 * (int)blockIdx.y + (int)(b % 3), (int)(b / 3 * 256 + threadIdx.x));
+        return;
+    }
+    b -= 3 * nb.ball;
+    if (b >= 3 * nb.edges) {
+        b -= 3 * nb.edges;
+        const int axis = b < 2 * nb.x ? 0 : b < 2 * (nb.x + nb.y) ? 1 : 2;
+        b -= axis == 0 ? 0 : axis == 1 ? 2 * nb.x : 2 * (nb.x + nb.y);
+        const uint32_t n = axis == 0 ? nb.x : axis == 1 ? nb.y : nb.z;
+        const bool high = b >= n;
+        const uint32_t t = (b - (high ? n : 0)) * 256 + threadIdx.x;
+        const uint32_t la = axis == 0 ? ny : nx, lb = axis == 2 ? ny : nz;
+        const uint32_t B = t / la, A = t - B * la;
+        if (B >= lb) return;
+        const int q = axis == 0 ? (high ? nth_dir<0, -1>(blockIdx.y) : nth_dir<0, 1>(blockIdx.y))
+                    : axis == 1 ? (high ? nth_dir<1, -1>(blockIdx.y) : nth_dir<1, 1>(blockIdx.y))
+                                : (high ? nth_dir<2, -1>(blockIdx.y) : nth_dir<2, 1>(blockIdx.y));
+        int e[3], bq;
+        dir_of(q, e, bq);
+        RingEntry w;
+        w.i = axis == 0 ? (high ? nx : -1) : (int)A;
+        w.j = axis == 1 ? (high ? ny : -1) : axis == 0 ? (int)A : (int)B;
+        w.k = axis == 2 ? (high ? nz : -1) : (int)B;
+        const uint64_t r = (uint64_t)ring_index(P, w.i, w.j, w.k);
+        const bool copy = SPHERE && axis == 0;
+        const int s = copy ? (high ? 1 : 0) : 2, sy = !SPHERE && axis == 2 && high ? 1 : s;
+        w.i = axis == 0 ? (high ? (copy ? nx - 1 : nx - 2) : (copy ? 0 : 1)) : w.i + s * e[0];
+        w.j = axis == 1 ? (high ? ny - 2 : 1) : w.j + sy * e[1];
+        w.k = axis == 2 ? (high ? nz - 2 : 1) : w.k + s * e[2];
+        w.turned = !copy;
+        w.before = SPHERE ? (axis + 2) % 3 : axis;
+        if (w.i < 0 || w.i >= nx || w.j < 0 || w.j >= ny || w.k < 0 || w.k >= nz) {
+            if (ring_hop<SPHERE>(P, e, w)) ring_hop<SPHERE>(P, e, w);
+        }
+        P.ring[(uint64_t)q * P.ring_n + r] = ring_value<SPHERE>(P, last, q, bq, e, w);
+        return;
+    }
+    const int q = 3 * (int)blockIdx.y + (int)(b % 3);
+    uint32_t t = b / 3 * 256 + threadIdx.x;
+    RingEntry w;
+    if (t < 4 * (uint32_t)(ny + 2)) {  // along y
+        const int l = (int)(t / (uint32_t)(ny + 2));
+        w.i = l & 1 ? nx : -1;
+        w.k = l & 2 ? nz : -1;
+        w.j = (int)t - l * (ny + 2) - 1;
+    } else if ((t -= 4 * (uint32_t)(ny + 2)) < 4 * (uint32_t)nz) {  // along z
+        const int l = (int)(t / (uint32_t)nz);
+        w.i = l & 1 ? nx : -1;
+        w.j = l & 2 ? ny : -1;
+        w.k = (int)t - l * nz;
+    } else if ((t -= 4 * (uint32_t)nz) < 4 * (uint32_t)nx) {  // along x
+        const int l = (int)(t / (uint32_t)nx);
+        w.j = l & 1 ? ny : -1;
+        w.k = l & 2 ? nz : -1;
+        w.i = (int)t - l * nx;
     } else {
         return;
     }
-    const uint64_t r = (uint64_t)ring_index(P, i, j, k);
-    // the inward direction across each ghost axis of the cell (0: not a
-    // ghost coordinate)
-    const int sx = i < 0 ? 1 : (i >= P.nx ? -1 : 0);
-    const int sy = j < 0 ? 1 : (j >= P.ny ? -1 : 0);
-    const int sz = k < 0 ? 1 : (k >= P.nz ? -1 : 0);
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const bool walled = (sx != 0 && EX[q] == sx) || (sy != 0 && EY[q] == sy) || (sz != 0 && EZ[q] == sz);
-        if (walled) P.ring[(uint64_t)q * P.ring_n + r] = 0.0;
-    }
-}
-
-// One wall of lid_driven_cavity/src/lbm.cpp:233-301: for the first-layer
-// cells (a, b) of the plane and every direction q pointing into the cavity,
-// f_q(plane) = f_bb(q)(src_plane, a + sa e_a, b + sb e_b).  The sources lie
-// in src_plane and the targets in plane, so no source is a target.
-// Thread t of row blockIdx.y: cell t of the plane, its blockIdx.y-th such q
-// (a row per direction: the pairs are independent, and nine times the lanes
-// hide the latency of the scattered loads).
-template <int AXIS, int SIGN>
-__device__ __forceinline__ void faithful_wall(const FusedParams &P, int plane, int src_plane, int sa, int sb)
-{
-    const int la = AXIS == 0 ? P.ny : P.nx, lb = AXIS == 2 ? P.ny : P.nz;
-    const int na = la + 2, nb = lb + 2;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= na * nb) return;
-    const int q = nth_dir<AXIS, SIGN>(blockIdx.y);
+    w.turned = 0;
+    w.before = 3;
+    const uint64_t r = (uint64_t)ring_index(P, w.i, w.j, w.k);
     int e[3], bq;
     dir_of(q, e, bq);
-    const int A = t % na - 1, B = t / na - 1;
-    int si, sj, sk, di, dj, dk;
-    if (AXIS == 0) {
-        si = src_plane; sj = A + sa * e[1]; sk = B + sb * e[2];
-        di = plane; dj = A; dk = B;
-    } else if (AXIS == 1) {
-        si = A + sa * e[0]; sj = src_plane; sk = B + sb * e[2];
-        di = A; dj = plane; dk = B;
-    } else {
-        si = A + sa * e[0]; sj = B + sb * e[1]; sk = src_plane;
-        di = A; dj = B; dk = plane;
-    }
-    double v;
-    if (AXIS == 0 && P.stage != nullptr && sj >= 0 && sj < P.ny && sk >= 0 && sk < P.nz) {
-        // an interior cell of plane 1 or nx - 2: from the copy the last fused
-        // pass wrote, y fastest (one strided cell per row of the lattice
-        // otherwise)
-        const int side = SIGN > 0 ? 0 : 1;
-        v = P.stage[(((uint64_t)side * P.nz + sk) * P.ny + sj) * STAGE_ROW + x_rank(bq)];
-    } else {
-        const GhostSrc g = faithful_src(P, bq, si, sj, sk);
-        v = *g.p;
-        v = g.is_deep ? g.deep : v;
-    }
-    const uint64_t r = (uint64_t)ring_index(P, di, dj, dk);
-    P.ring[(uint64_t)q * P.ring_n + r] = v;
+    if (!ring_hop<SPHERE>(P, e, w)) return;  // no pass writes this entry
+    if (ring_hop<SPHERE>(P, e, w)) ring_hop<SPHERE>(P, e, w);
+    P.ring[(uint64_t)q * P.ring_n + r] = ring_value<SPHERE>(P, last, q, bq, e, w);
 }
 
 // FusedParams::stage from the lattice P.src: thread t is entry t of the
@@ -671,119 +800,31 @@ hipError_t launch_faithful_stage_fill(const FusedParams &P, hipStream_t st)
     return hipGetLastError();
 }
 
-// The two walls of one axis in one launch: blockIdx.z = 0 the low wall
-// (plane -1, sources on plane 1), 1 the high wall (plane n, sources on plane
-// n - 2; its b-stride sb_high).  With n >= 2 both source planes lie inside the
-// domain on this axis, so neither wall reads what the other writes and their
-// order does not matter; the axes still follow the reference's order, since
-// a later axis reads edge cells an earlier one wrote.
-template <int AXIS>
-__global__ void k_faithful_walls(const FusedParams P, int sb_high)
+hipError_t launch_faithful_boundaries(const FusedParams &P, const double *last_ring, hipStream_t st)
 {
-    const int n = AXIS == 0 ? P.nx : AXIS == 1 ? P.ny : P.nz;
-    if (blockIdx.z == 0) faithful_wall<AXIS, 1>(P, -1, 1, 2, 2);
-    else faithful_wall<AXIS, -1>(P, n, n - 2, 2, sb_high);
-}
-
-// sphere/src/lbm.cpp:326-347: the inlet ghost plane takes the first
-// interior plane's populations with e_x > 0, the outlet ghost plane takes
-// f_q(nx - 1, y + e_y, z + e_z) for e_x < 0; first-layer cells only (the
-// sources lie on x = 0 or nx - 1, the targets on x = -1 or nx).  Thread t of
-// row blockIdx.y: cell t of the plane, its blockIdx.y-th such q.
-template <int OUTLET>
-__global__ void k_faithful_inlet_outlet(const FusedParams P)
-{
-    const int na = P.ny + 2, nb = P.nz + 2;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= na * nb) return;
-    const int q = OUTLET ? nth_dir<0, -1>(blockIdx.y) : nth_dir<0, 1>(blockIdx.y);
-    int e[3], bq;
-    dir_of(q, e, bq);
-    const int j = t % na - 1, k = t / na - 1;
-    const int sj = OUTLET ? j + e[1] : j, sk = OUTLET ? k + e[2] : k;
-    double v;
-    if (P.stage != nullptr && sj >= 0 && sj < P.ny && sk >= 0 && sk < P.nz) {
-        // an interior cell of plane 0 or nx - 1: from the copy the last fused
-        // pass wrote
-        v = P.stage[(((uint64_t)OUTLET * P.nz + sk) * P.ny + sj) * STAGE_ROW + x_rank(q)];
-    } else {
-        const GhostSrc g = faithful_src(P, q, OUTLET ? P.nx - 1 : 0, sj, sk);
-        v = *g.p;
-        v = g.is_deep ? g.deep : v;
-    }
-    const uint64_t r = (uint64_t)ring_index(P, OUTLET ? P.nx : -1, j, k);
-    P.ring[(uint64_t)q * P.ring_n + r] = v;
-}
-
-// "usrbc", sphere/src/lbm.cpp:350-356: a solid cell takes, for each
-// direction q whose neighbour x + e_q is fluid, f_bb(q)(x + 2 e_q), in place
-// in the post-collision lattice.  The reference's mask covers the ghost
-// cells too: where the ball reaches the first ghost layer (ny or nz within r
-// of its centre), a ghost neighbour can be solid, and its mask value is
-// recomputed here.  A source is never a target: between two solid voxels of a
-// ball the midpoint voxel is solid too, so that direction is not taken.  The
-// (cell, q) pairs are therefore independent: thread t of row q = blockIdx.y
-// takes cell t of the box [lo, lo + n)^3 around the ball (clamped to the
-// cavity), so that the few thousand cells of the box fill 27 times as many
-// lanes.  Every thread loads (threads off the box from a valid cell) and only
-// solid cells store: no load sits under a divergent branch.
-__global__ void k_faithful_usr(const FusedParams P, int lo, int n)
-{
-    const int q = blockIdx.y;
-    int ex = 0, ey = 0, ez = 0, bq = 0;
-#pragma unroll
-    for (int k = 0; k < Q; ++k)
-        if (k == q) {
-            ex = EX[k];
-            ey = EY[k];
-            ez = EZ[k];
-            bq = BB[k];
-        }
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int tt = t < n * n * n ? t : 0;
-    const int x0 = lo + tt % n, y0 = lo + (tt / n) % n, z0 = lo + tt / (n * n);
-    const bool valid = (t < n * n * n) & (x0 < P.nx) & (y0 < P.ny) & (z0 < P.nz);
-    const int x = valid ? x0 : 0, y = valid ? y0 : 0, z = valid ? z0 : 0;
-    const uint32_t c = ((uint32_t)z * P.ny + y) * P.nx + x;
-    const int xi = x + ex, yi = y + ey, zi = z + ez;
-    const bool in = (xi >= 0) & (xi < P.nx) & (yi >= 0) & (yi < P.ny) & (zi >= 0) & (zi < P.nz);
-    const uint64_t mi = in ? ((uint64_t)zi * P.ny + yi) * P.nx + xi : (uint64_t)c;
-    const GhostSrc g = faithful_src(P, bq, x + 2 * ex, y + 2 * ey, z + 2 * ez);
-    const uint8_t mc = P.mask[c];
-    const uint8_t m = P.mask[mi];
-    double v = *g.p;
-    v = g.is_deep ? g.deep : v;
-    const bool solid = valid & (mc == 1);
-    const bool nb_solid = in ? m == 1 : faithful_sphere_solid(P.nx, xi, yi, zi);
-    if (solid & !nb_solid) ((double *)P.src)[P.geom.off(q, (uint32_t)z, (uint32_t)y * P.nx + x)] = v;
-}
-
-hipError_t launch_faithful_boundaries(const FusedParams &P, hipStream_t st)
-{
-    const int nx = P.nx, ny = P.ny, nz = P.nz;
-    // nine rows of workgroups: one per direction entering the domain
-    auto grid = [](int la, int lb) { return dim3((unsigned)(((la + 2) * (lb + 2) + 255) / 256), 9); };
-    // the same, times the two walls of an axis
-    auto grid2 = [](int la, int lb) { return dim3((unsigned)(((la + 2) * (lb + 2) + 255) / 256), 9, 2); };
-    if (P.faithful_sphere) {
-        // bcf bcb bcd bcu, inlet, outlet, usrbc (sphere/src/lbm.cpp:277-356);
-        // one rank: the unpack has nothing to write
-        hipLaunchKernelGGL(k_faithful_walls<1>, grid2(nx, nz), dim3(256), 0, st, P, 2);
-        hipLaunchKernelGGL(k_faithful_walls<2>, grid2(nx, ny), dim3(256), 0, st, P, 2);
-        hipLaunchKernelGGL(k_faithful_inlet_outlet<0>, grid(ny, nz), dim3(256), 0, st, P);
-        hipLaunchKernelGGL(k_faithful_inlet_outlet<1>, grid(ny, nz), dim3(256), 0, st, P);
-        // the ball lies within [c - r, c + r] of its centre c on every axis
-        const int cc = (nx - 1) / 8, rr = (int)std::ceil((nx - 1) / 64.0);
-        const int lo = cc - rr < 0 ? 0 : cc - rr, n = cc + rr - lo + 1;
-        hipLaunchKernelGGL(k_faithful_usr, dim3((unsigned)((n * n * n + 255) / 256), Q), dim3(256), 0, st, P, lo, n);
+    auto blocks = [](int64_t n) { return (uint32_t)((n + 255) / 256); };
+    RingBlocks nb{blocks((int64_t)P.ny * P.nz), blocks((int64_t)P.nx * P.nz), blocks((int64_t)P.nx * P.ny),
+                  blocks(4ll * (P.nx + P.ny + 2 + P.nz)), 0, 0, 0};
+    dim3 grid(2 * (nb.x + nb.y + nb.z) + 3 * nb.edges, 9);
+    if (!P.faithful_sphere) {
+        hipLaunchKernelGGL(k_faithful_ring<false>, grid, dim3(256), 0, st, P, last_ring, nb);
         return hipGetLastError();
     }
-    const uint32_t nun = 2u * (P.ny + 2) * (P.nz + 2) + (uint32_t)P.nx * (P.nz + 2) + (uint32_t)P.nx * (P.ny + 2);
-    hipLaunchKernelGGL(k_faithful_unpack, dim3((nun + 255) / 256), dim3(256), 0, st, P);
-    // bcl bcr, bcf bcb, bcd bcu; the top wall reads j + e_y (:298)
-    hipLaunchKernelGGL(k_faithful_walls<0>, grid2(ny, nz), dim3(256), 0, st, P, 2);
-    hipLaunchKernelGGL(k_faithful_walls<1>, grid2(nx, nz), dim3(256), 0, st, P, 2);
-    hipLaunchKernelGGL(k_faithful_walls<2>, grid2(nx, ny), dim3(256), 0, st, P, 1);
+    // one rank: the unpack has nothing to write.  The ball lies within
+    // [c - r, c + r] of its centre c on every axis.  Where that box stays two
+    // cells off every face, usrbc reads no ghost cell and no pass reads a cell of
+    // the box (their sources lie on the two outermost planes of an axis): one
+    // launch does both.  Elsewhere usrbc follows in its own, as in the reference.
+    const int cc = (P.nx - 1) / 8, rr = (int)std::ceil((P.nx - 1) / 64.0);
+    nb.lo = cc - rr < 0 ? 0 : cc - rr;
+    nb.n = cc + rr - nb.lo + 1;
+    const int low = P.nx < P.ny ? P.nx : P.ny, least = low < P.nz ? low : P.nz;
+    const uint32_t ball = blocks((int64_t)nb.n * nb.n * nb.n);
+    const bool clear = nb.lo >= 2 && nb.lo + nb.n <= least - 2;
+    if (clear) nb.ball = ball;
+    grid.x += 3 * nb.ball;
+    hipLaunchKernelGGL(k_faithful_ring<true>, grid, dim3(256), 0, st, P, last_ring, nb);
+    if (!clear) hipLaunchKernelGGL(k_faithful_usr, dim3(ball, Q), dim3(256), 0, st, P, nb.lo, nb.n);
     return hipGetLastError();
 }
 

@@ -47,7 +47,9 @@ struct imexlb_handle {
     double corr[Q] = {};
     double feq_in[Q] = {};
     double *tgv_tab = nullptr;
-    double *ring = nullptr;  // faithful cavity: the first ghost layer (FusedParams::ring)
+    // faithful mode: the first ghost layer (FusedParams::ring); ring[cur] is the
+    // last step's, the other one the step's before (aux.hip k_faithful_ring)
+    double *ring[2] = {nullptr, nullptr};
     double *stage = nullptr; // faithful mode: what the x-face boundary kernels read (FusedParams::stage)
     uint32_t ring_a = 0, ring_b = 0, ring_c = 0;
     int block = 256, cpt = 1, xcd = 1, ntl = 0;
@@ -218,9 +220,9 @@ static void fill_fused_params(imexlb_handle *h, FusedParams &P, int src, int dst
     P.am_max = c.addr_mode < 0 ? 2 : c.addr_mode;
     P.divx.init(c.nx);
     P.divy.init(c.ny);
-    P.ring = h->ring;
+    P.ring = h->ring[dst];
     P.stage = h->stage;
-    if (h->ring) P.ring_rel = ((intptr_t)h->ring - (intptr_t)h->lat[src]) / (intptr_t)sizeof(double);
+    if (P.ring) P.ring_rel = ((intptr_t)P.ring - (intptr_t)h->lat[src]) / (intptr_t)sizeof(double);
     P.ring_a = h->ring_a;
     P.ring_b = h->ring_b;
     P.ring_c = h->ring_c;
@@ -270,9 +272,9 @@ static int fused_step(imexlb_handle *h, bool write_moments)
         P.mom_v = h->mom[2];
         P.mom_w = h->mom[3];
     }
-    // the faithful cavity's unpack and walls fill the ghost ring from the
-    // post-collision lattice first, as the reference's Streaming does
-    if (bc_of(c) == BC_FAITHFUL) HIPCHK(h, launch_faithful_boundaries(P, h->stream));
+    // faithful mode: the ghost ring is filled from the post-collision lattice
+    // first, as the reference's Streaming does
+    if (bc_of(c) == BC_FAITHFUL) HIPCHK(h, launch_faithful_boundaries(P, h->ring[h->cur], h->stream));
     HIPCHK(h, launch_fused(c.dtype, bc_of(c), pattern, P, h->block, h->stream));
     if (c.storage == IMEXLB_PULL) h->cur = 1 - h->cur;
     h->steps++;
@@ -438,8 +440,10 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
         h->ring_b = (uint32_t)c.nx * (uint32_t)(c.nz + 2);
         h->ring_c = (uint32_t)c.nx * (uint32_t)c.ny;
         const size_t rb = (size_t)Q * 2 * (h->ring_a + h->ring_b + h->ring_c) * 8;
-        if (hipMalloc(&h->ring, rb) != hipSuccess) return bail(fail(h, IMEXLB_ENOMEM, "ghost ring"));
-        h->device_bytes += (int64_t)rb;
+        for (auto &p : h->ring) {
+            if (hipMalloc(&p, rb) != hipSuccess) return bail(fail(h, IMEXLB_ENOMEM, "ghost ring"));
+            h->device_bytes += (int64_t)rb;
+        }
         const size_t sb = (size_t)2 * STAGE_ROW * c.ny * c.nz * 8;
         if (hipMalloc(&h->stage, sb) != hipSuccess) return bail(fail(h, IMEXLB_ENOMEM, "x-face stage"));
         h->device_bytes += (int64_t)sb;
@@ -543,7 +547,8 @@ int imexlb_destroy(imexlb_handle *h)
     if (h->partials) hipFree(h->partials);
     if (h->result) hipFree(h->result);
     if (h->tgv_tab) hipFree(h->tgv_tab);
-    if (h->ring) hipFree(h->ring);
+    for (auto &p : h->ring)
+        if (p) hipFree(p);
     if (h->stage) hipFree(h->stage);
     if (h->ph) phased_destroy(h->ph);
     if (h->gexec) hipGraphExecDestroy(h->gexec);
@@ -588,8 +593,10 @@ int imexlb_initialize(imexlb_handle *h)
     P.divx.init(c.nx);
     P.divy.init(c.ny);
     HIPCHK(h, launch_init(c.dtype, P, h->stream));
-    if (h->ring) {  // the first ghost layer starts from the initial fields too
+    if (h->ring[0]) {  // the first ghost layer starts from the initial fields too
         FusedParams F;
+        fill_fused_params(h, F, 0, 1);
+        HIPCHK(h, launch_faithful_ring_init(F, h->stream));
         fill_fused_params(h, F, 0, 0);
         HIPCHK(h, launch_faithful_ring_init(F, h->stream));
         if (h->stage) HIPCHK(h, launch_faithful_stage_fill(F, h->stream));
@@ -828,7 +835,7 @@ static const char CK_MAGIC_RING[8] = {'I', 'M', 'X', 'L', 'B', 'C', 'R', '1'};
 
 static size_t ring_doubles(const imexlb_handle *h)
 {
-    return h->ring ? (size_t)Q * 2 * (h->ring_a + h->ring_b + h->ring_c) : 0;
+    return h->ring[0] ? (size_t)Q * 2 * (h->ring_a + h->ring_b + h->ring_c) : 0;
 }
 
 int imexlb_checkpoint_write(imexlb_handle *h, const char *path)
@@ -845,14 +852,14 @@ int imexlb_checkpoint_write(imexlb_handle *h, const char *path)
     std::vector<double> f(n);
     rc = h->ph ? phased_get_state(h->ph, f.data(), h->err) : imexlb_get_f(h, f.data());
     if (rc) return rc;
-    if (h->ring) {
-        const imx::ReadBack::Part part{f.data() + nf, h->ring, ring_doubles(h) * 8};
+    if (h->ring[0]) {
+        const imx::ReadBack::Part part{f.data() + nf, h->ring[h->cur], ring_doubles(h) * 8};
         HIPCHK(h, h->back.copy(&part, 1, h->device, h->stream));
     }
     FILE *fp = std::fopen(path, "wb");
     if (!fp) return fail(h, IMEXLB_EIO, "cannot open %s", path);
     const int64_t steps = h->steps;
-    const char *magic = h->ph ? CK_MAGIC_PHASED : (h->ring ? CK_MAGIC_RING : CK_MAGIC);
+    const char *magic = h->ph ? CK_MAGIC_PHASED : (h->ring[0] ? CK_MAGIC_RING : CK_MAGIC);
     bool ok = std::fwrite(magic, 1, 8, fp) == 8 &&
               std::fwrite(&h->cfg, sizeof h->cfg, 1, fp) == 1 && std::fwrite(&steps, 8, 1, fp) == 1 &&
               std::fwrite(f.data(), 8, n, fp) == n;
@@ -877,7 +884,7 @@ int imexlb_checkpoint_read(imexlb_handle *h, const char *path)
     std::vector<double> f(n);
     bool ok = std::fread(magic, 1, 8, fp) == 8 && std::fread(&c, sizeof c, 1, fp) == 1 &&
               std::fread(&steps, 8, 1, fp) == 1;
-    const char *want = h->ph ? CK_MAGIC_PHASED : (h->ring ? CK_MAGIC_RING : CK_MAGIC);
+    const char *want = h->ph ? CK_MAGIC_PHASED : (h->ring[0] ? CK_MAGIC_RING : CK_MAGIC);
     if (ok && std::memcmp(magic, want, 8) != 0) {
         std::fclose(fp);
         const bool known = std::memcmp(magic, CK_MAGIC, 8) == 0 || std::memcmp(magic, CK_MAGIC_PHASED, 8) == 0 ||
@@ -923,8 +930,10 @@ int imexlb_checkpoint_read(imexlb_handle *h, const char *path)
         h->phase_collided = false;
         return phased_set_state(h->ph, f.data(), h->err);
     }
-    if (h->ring) {
-        HIPCHK(h, hipMemcpyAsync(h->ring, f.data() + nf, ring_doubles(h) * 8, hipMemcpyHostToDevice, h->stream));
+    if (h->ring[0]) {
+        // both: what no boundary pass writes is the same in the two
+        for (double *p : h->ring)
+            HIPCHK(h, hipMemcpyAsync(p, f.data() + nf, ring_doubles(h) * 8, hipMemcpyHostToDevice, h->stream));
         HIPCHK(h, hipStreamSynchronize(h->stream));
     }
     return imexlb_set_f(h, f.data());

@@ -280,9 +280,9 @@ __host__ __device__ __forceinline__ int64_t ring_index(const FusedParams &P, int
     return deep ? -1 : (xf ? rx : (yf ? ry : (zf ? rz : -2)));
 }
 
-// The faithful cavity's unpack and wall kernels on the ring (aux.hip):
-// Streaming's boundary phase, before the fused pass.
-hipError_t launch_faithful_boundaries(const FusedParams &P, hipStream_t st);
+// Streaming's boundary phase on the ring (aux.hip k_faithful_ring), before the
+// fused pass: P.ring from the lattice P.src and the last step's ring.
+hipError_t launch_faithful_boundaries(const FusedParams &P, const double *last_ring, hipStream_t st);
 // Initialize's values for the ring (0 in the cavity)
 hipError_t launch_faithful_ring_init(const FusedParams &P, hipStream_t st);
 // fills FusedParams::stage from the lattice P.src (after Initialize, set_f)

@@ -56,20 +56,21 @@ constexpr EzPos EZ_POS = ez_pos();
 
 // The d-th direction, in index order, of the nine with e_AXIS * SIGN > 0
 // (d < 9), and a direction's velocity and opposite, for kernels that give each
-// direction its own row of workgroups.
+// direction its own row of workgroups: packed into 64-bit constants, since a
+// search over the 27 directions costs such a kernel more than its work.
+constexpr uint64_t nth_table(int axis, int sign)
+{
+    uint64_t t = 0;
+    int n = 0;
+    for (int k = 0; k < Q; ++k)
+        if ((axis == 0 ? EX[k] : axis == 1 ? EY[k] : EZ[k]) * sign > 0) t |= (uint64_t)k << (5 * n++);
+    return t;
+}
 template <int AXIS, int SIGN>
 IMX_HD inline int nth_dir(int d)
 {
-    int q = 0, cnt = 0;
-#pragma unroll
-    for (int k = 0; k < Q; ++k) {
-        const int e = AXIS == 0 ? EX[k] : AXIS == 1 ? EY[k] : EZ[k];
-        if (e * SIGN > 0) {
-            if (cnt == d) q = k;
-            ++cnt;
-        }
-    }
-    return q;
+    constexpr uint64_t t = nth_table(AXIS, SIGN);
+    return (int)(t >> (5 * d)) & 31;
 }
 // The nine directions with e_x = +1 and with e_x = -1, in index order
 // (nth_dir<0, 1> and nth_dir<0, -1>), as tables: kernels that index a
@@ -98,23 +99,47 @@ static_assert(xdir_tables_ok(), "XDIR_P / XDIR_M must list the e_x = +1 / -1 dir
 
 // The rank of direction q among the nine with its e_x (e_x != 0): the d
 // with nth_dir<0, EX[q]>(d) == q.
-IMX_HD constexpr int x_rank(int q)
+constexpr uint64_t x_rank_table()
 {
-    int r = 0;
-    for (int k = 0; k < q; ++k) r += EX[k] == EX[q] ? 1 : 0;
-    return r;
+    uint64_t t = 0;
+    for (int r = 0; r < 9; ++r) t |= (uint64_t)r << (4 * ((XDIR_P[r] - 1) / 2));
+    return t;
 }
+constexpr bool x_dirs_pair_up()
+{
+    for (int r = 0; r < 9; ++r)
+        if (XDIR_P[r] % 2 != 1 || XDIR_M[r] != XDIR_P[r] + 1) return false;
+    return true;
+}
+static_assert(x_dirs_pair_up(), "x_rank takes the pair's number");
+IMX_HD inline int x_rank(int q)
+{
+    constexpr uint64_t t = x_rank_table();
+    return (int)(t >> (4 * ((q - 1) / 2))) & 15;
+}
+
+// Direction q and its opposite for a q known only at run time: two bits per
+// direction in one constant per axis.
+constexpr uint64_t dir_table(const int (&e)[Q])
+{
+    uint64_t t = 0;
+    for (int k = 0; k < Q; ++k) t |= (uint64_t)(e[k] + 1) << (2 * k);
+    return t;
+}
+constexpr bool opposites_pair_up()
+{
+    for (int k = 1; k < Q; ++k)
+        if (BB[k] != ((k - 1) ^ 1) + 1) return false;
+    return BB[0] == 0;
+}
+static_assert(opposites_pair_up(), "dir_of takes bb(q) from q");
 IMX_HD inline void dir_of(int q, int (&e)[3], int &bq)
 {
-    e[0] = e[1] = e[2] = bq = 0;
-#pragma unroll
-    for (int k = 0; k < Q; ++k)
-        if (k == q) {
-            e[0] = EX[k];
-            e[1] = EY[k];
-            e[2] = EZ[k];
-            bq = BB[k];
-        }
+    constexpr uint64_t tx = dir_table(EX), ty = dir_table(EY), tz = dir_table(EZ);
+    e[0] = (int)((tx >> (2 * q)) & 3) - 1;
+    e[1] = (int)((ty >> (2 * q)) & 3) - 1;
+    e[2] = (int)((tz >> (2 * q)) & 3) - 1;
+    bq = q ? ((q - 1) ^ 1) + 1 : 0;
 }
 
 }  // namespace imx
