@@ -828,4 +828,40 @@ hipError_t launch_faithful_boundaries(const FusedParams &P, const double *last_r
     return hipGetLastError();
 }
 
+// Device arrays into pinned host memory (CopyOut), 16 bytes per thread and pass,
+// straight over the link, whose 50 to 55 GB/s bound it (4 MiB 76 us); a read of a few
+// hundred KiB is bound by the launch and the wait, hence one launch for all four.
+__global__ void __launch_bounds__(256) k_copy_out(const CopyOut C)
+{
+    typedef uint32_t Unit __attribute__((ext_vector_type(4)));
+    for (uint64_t u = (uint64_t)blockIdx.x * 256 + threadIdx.x; u < C.at[4]; u += (uint64_t)gridDim.x * 256) {
+        const int k = (u >= C.at[1]) + (u >= C.at[2]) + (u >= C.at[3]);
+        const char *base = k == 0 ? C.src[0] : k == 1 ? C.src[1] : k == 2 ? C.src[2] : C.src[3];
+        const uint64_t bytes = k == 0 ? C.bytes[0] : k == 1 ? C.bytes[1] : k == 2 ? C.bytes[2] : C.bytes[3];
+        const uint64_t first = k == 0 ? C.at[0] : k == 1 ? C.at[1] : k == 2 ? C.at[2] : C.at[3];
+        const uint64_t o = (u - first) * 16;
+        const char *const s = base + o;
+        char *const d = C.dst + u * 16;
+        if (o + 16 <= bytes && (uintptr_t)base % 8 == 0) {
+            if ((uintptr_t)base % 16 == 0) {
+                __builtin_nontemporal_store(__builtin_nontemporal_load((const Unit *)s), (Unit *)d);
+            } else {
+                const uint64_t a = ((const uint64_t *)s)[0], b = ((const uint64_t *)s)[1];
+                const Unit v = {(uint32_t)a, (uint32_t)(a >> 32), (uint32_t)b, (uint32_t)(b >> 32)};
+                __builtin_nontemporal_store(v, (Unit *)d);
+            }
+        } else {
+            for (uint64_t b = 0; b < 16 && o + b < bytes; ++b) d[b] = s[b];
+        }
+    }
+}
+
+hipError_t launch_copy_out(const CopyOut &C, hipStream_t st)
+{
+    const uint64_t blocks = (C.at[4] + 255) / 256;
+    if (blocks == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_copy_out, dim3((unsigned)(blocks < 512 ? blocks : 512)), dim3(256), 0, st, C);
+    return hipGetLastError();
+}
+
 }  // namespace imx

@@ -280,6 +280,17 @@ __host__ __device__ __forceinline__ int64_t ring_index(const FusedParams &P, int
     return deep ? -1 : (xf ? rx : (yf ? ry : (zf ? rz : -2)));
 }
 
+// Up to four device arrays, one after the other from dst on (pinned host
+// memory), each from the next 16-byte unit; at[k] is array k's first unit, at[n] the
+// number of units.
+struct CopyOut {
+    const char *src[4];
+    uint64_t bytes[4];
+    uint64_t at[5];
+    char *dst;
+};
+hipError_t launch_copy_out(const CopyOut &C, hipStream_t st);
+
 // Streaming's boundary phase on the ring (aux.hip k_faithful_ring), before the
 // fused pass: P.ring from the lattice P.src and the last step's ring.
 hipError_t launch_faithful_boundaries(const FusedParams &P, const double *last_ring, hipStream_t st);

@@ -3,13 +3,14 @@
 // hipMemcpyAsync into pageable memory goes through the runtime's own staging
 // buffer, one megabyte and one host thread at a time, and the thread also takes
 // the page faults of a fresh array: 10 GB/s for 2-4 GB of fields, and 115 us a call for
-// 256 KiB.  Here the device copies into pinned slots at the link's rate (50 GB/s
-// in 4 MiB pieces, 38 in 1 MiB) while a few threads move finished slots on
-// (4 GB of fields: 41-46 GB/s with four threads and 4 MiB pieces, 24-27 with
-// two, no more with eight); a small read is one wait and one memcpy.  Read of
-// the four fields, ms, before / after: TGV 512^3 416 / 94, 256^3 52.6 / 12.6, channel
-// 512x256x256 103 / 24, cavity 128^3 7.8 / 2.4, TGV 32^3 0.20 / 0.10, 15 ensemble members
-// 27.4 / 11.6.
+// 256 KiB.  Here the device copies into pinned slots by a kernel of its own
+// (aux.hip k_copy_out; hipMemcpyAsync leaves 11 us between copies) while a few threads
+// move finished slots on: GB/s for 512 MB / 4 GB of fields 37 / 44 with four
+// threads, 42 / 46.5 with six, no more with eight.  A small read is one launch for
+// all its arrays, one wait and one memcpy: TGV 32^3 fields 95 -> 71 us and diagnostics
+// 31 -> 22 against one hipMemcpyAsync each.  Read of the four fields, ms, before any of
+// this / after: TGV 512^3 416 / 93, 256^3 52.6 / 12.7, channel 512x256x256 103 / 24,
+// cavity 128^3 7.8 / 2.3, TGV 32^3 0.20 / 0.07, 15 ensemble members 27.4 / 11.6.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -19,6 +20,8 @@
 #include <cstring>
 #include <thread>
 #include <vector>
+
+#include "kernels.h"
 
 namespace imx {
 
@@ -74,7 +77,7 @@ class ReadBack {
   private:
     static constexpr size_t MIB = size_t(1) << 20;
     static constexpr size_t SMALL = 2 * MIB;  // below, starting threads costs what they save
-    static constexpr int THREADS = 4, SLOTS = 2 * THREADS;
+    static constexpr int THREADS = 6, SLOTS = 2 * THREADS;
 
     static bool known(const void *p)
     {
@@ -82,6 +85,22 @@ class ReadBack {
         const bool ok = hipPointerGetAttributes(&a, p) == hipSuccess;
         if (!ok) (void)hipGetLastError();
         return ok && a.type != hipMemoryTypeUnregistered;
+    }
+
+    // The room of `bytes` in pinned memory: whole 16-byte units.
+    static size_t held(size_t bytes) { return (bytes + 15) / 16 * 16; }
+
+    // Up to four parts into pinned memory, one launch.
+    static hipError_t copy_out(const Part *parts, int n, char *pinned, hipStream_t st)
+    {
+        CopyOut c{};
+        for (int k = 0; k < 4; ++k) {
+            c.src[k] = k < n ? (const char *)parts[k].src : nullptr;
+            c.bytes[k] = k < n ? parts[k].bytes : 0;
+            c.at[k + 1] = c.at[k] + held(c.bytes[k]) / 16;
+        }
+        hipError_t e = hipHostGetDevicePointer((void **)&c.dst, pinned, 0);
+        return e == hipSuccess ? launch_copy_out(c, st) : e;
     }
 
     // Pinned memory of at least `bytes`; false (and none held) if there is none.
@@ -101,22 +120,20 @@ class ReadBack {
 
     hipError_t copy_small(const Part *parts, int n, size_t total, hipStream_t st)
     {
-        if (!hold(std::max<size_t>(total, 4096))) return hipErrorNotReady;
+        if (!hold(std::max<size_t>(total + 16 * (size_t)n, 4096))) return hipErrorNotReady;
         size_t at = 0;
-        for (int k = 0; k < n; ++k) {
-            const hipError_t e = hipMemcpyAsync(pin_ + at, parts[k].src, parts[k].bytes, hipMemcpyDeviceToHost, st);
-            if (e != hipSuccess) {
-                (void)hipStreamSynchronize(st);
-                return e;
-            }
-            at += parts[k].bytes;
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < n && e == hipSuccess; k += 4) {
+            const int m = std::min(4, n - k);
+            e = copy_out(parts + k, m, pin_ + at, st);
+            for (int i = k; i < k + m; ++i) at += held(parts[i].bytes);
         }
-        const hipError_t e = hipStreamSynchronize(st);
-        if (e != hipSuccess) return e;
+        const hipError_t w = hipStreamSynchronize(st);
+        if (e != hipSuccess || w != hipSuccess) return e != hipSuccess ? e : w;
         at = 0;
         for (int k = 0; k < n; ++k) {
             std::memcpy(parts[k].dst, pin_ + at, parts[k].bytes);
-            at += parts[k].bytes;
+            at += held(parts[k].bytes);
         }
         return hipSuccess;
     }
@@ -173,7 +190,7 @@ class ReadBack {
             while (freed[k % SLOTS].load(std::memory_order_acquire) < k / SLOTS && failed.load() == (int)hipSuccess)
                 std::this_thread::yield();
             if (failed.load() != (int)hipSuccess) break;
-            e = hipMemcpyAsync(pin_ + (size_t)(k % SLOTS) * piece, work[k].src, work[k].bytes, hipMemcpyDeviceToHost, st);
+            e = copy_out(&work[k], 1, pin_ + (size_t)(k % SLOTS) * piece, st);
             if (e == hipSuccess) e = hipEventRecord(ev_[k % SLOTS], st);
             if (e == hipSuccess) queued.store(k + 1, std::memory_order_release);
             else failed.store((int)e);

@@ -60,3 +60,15 @@ def test_single_fields_and_pinned_memory(n):
     g.close()
     del pinned
     assert hip.hipHostFree(p) == 0
+
+
+# fields that end inside a 16-byte unit, and that start inside one in pinned
+# memory's order: one kernel copies all four
+@pytest.mark.parametrize("n", [(3, 3, 3), (5, 7, 3), (41, 39, 37)])
+def test_fields_of_odd_cell_counts(n):
+    print(f"[case] read-back odd {n}", flush=True)
+    g, o = make(n)
+    for a, b in zip(o.moments(), g.moments()):
+        assert np.array_equal(a, b)
+    assert np.array_equal(o.get_f(), g.get_f())
+    g.close()
