@@ -829,7 +829,7 @@ hipError_t launch_faithful_boundaries(const FusedParams &P, const double *last_r
 }
 
 // Device arrays into pinned host memory (CopyOut), 16 bytes per thread and pass,
-// straight over the link, whose 50 to 55 GB/s bound it (4 MiB 76 us); a read of a few
+// straight over the link, whose 54 GB/s bound it (2 MiB 39 us); a read of a few
 // hundred KiB is bound by the launch and the wait, hence one launch for all four.
 __global__ void __launch_bounds__(256) k_copy_out(const CopyOut C)
 {
