@@ -19,19 +19,24 @@ __device__ __forceinline__ double feq_f64(int i, double p, double u, double v, d
     return WVAL[WCLASS[i]] * p * 3.0 + WVAL[WCLASS[i]] * (3.0 * edu + 4.5 * eu2 - 1.5 * udu);
 }
 
-// Population f of direction i (weight class of slot `slot`, which is i or
-// bb(i)) of cell p of plane z in the stored convention, g = f - s with s the
-// direction's shift.
+// Population f in the stored convention, g = f - s with s the direction's
+// shift, of the weight class of slot `slot` (i or bb(i)).
+template <typename S>
+__device__ __forceinline__ S stored(int slot, double f, double s)
+{
+    if constexpr (std::is_same<S, double>::value)
+        return f;
+    else if constexpr (std::is_same<S, float>::value)
+        return (float)(f - s);
+    else
+        return (_Float16)((float)(f - s) * H_SCALE[WCLASS[slot]]);
+}
+
+// The same into cell c of plane z.
 template <typename S>
 __device__ __forceinline__ void put(S *lat, const LatGeom &g, int slot, uint32_t z, uint32_t c, double f, double s)
 {
-    S *p = lat + g.off(g.pos(slot), z, c);
-    if constexpr (std::is_same<S, double>::value)
-        *p = f;
-    else if constexpr (std::is_same<S, float>::value)
-        *p = (float)(f - s);
-    else
-        *p = (_Float16)((float)(f - s) * H_SCALE[WCLASS[slot]]);
+    lat[g.off(g.pos(slot), z, c)] = stored<S>(slot, f, s);
 }
 
 template <typename S>
@@ -49,15 +54,23 @@ __device__ __forceinline__ double get(const S *lat, const LatGeom &g, int slot, 
 // Initial state = f0 = feq(p, u) of the analytic fields.  The reference's
 // first Collision relaxes f0 towards the feq of the same fields, which is f0
 // itself, so f0 is also the first post-collision state.
+//
+// Bound by its stores.  Workgroups stay within a plane, so that their lines are
+// whole in a plane tile, and each XCD writes one run of the lattice.  us, cells in
+// storage order over the whole lattice / this: TGV 301x203x157 FP32 340 / 235, 256^3
+// FP64 832 / 675, 512^3 FP64 6700 / 5400, FP16 3590 / 2450, cavity 100^3 62 / 58;
+// non-temporal stores 198, 626, 5490, 2440, 68.  The solid cells of the other
+// lattice are written here rather than by a copy of the whole: Initialize of the sphere
+// 512x128x128 1198 -> 383, channel 512x256x256 FP16 1490 -> 510.
 template <typename S>
 __global__ void k_init(const InitParams P)
 {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= P.ncell) return;
-    const uint32_t t = P.divx.div(c);
-    const uint32_t x = c - t * P.nx;
-    const uint32_t z = P.divy.div(t);
-    const uint32_t y = t - z * P.ny;
+    const uint32_t b = xcd_tile(blockIdx.x, gridDim.x);
+    const uint32_t z = P.divb.div(b), plane = (uint32_t)P.nx * P.ny;
+    const uint32_t pc = (b - z * P.bpp) * blockDim.x + threadIdx.x;
+    if (pc >= plane) return;
+    const uint32_t y = P.divx.div(pc), x = pc - y * P.nx;
+    const uint32_t c = z * plane + pc;
     double u, v, w, p;
     if (P.kind == 0) {
         // tgv/src/lbm.cpp:197-204 with per-axis sin/cos tables
@@ -92,17 +105,19 @@ __global__ void k_init(const InitParams P)
         w = 0.0;
         p = P.p0;
     }
-    S *lat = (S *)P.dst;
+    const bool solid = P.mask && P.mask[c] == 1;
+    const uint64_t at = P.geom.off(0, z, pc);
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
-        const double f = feq_f64(i, p, u, v, w);
-        put<S>(lat, P.geom, P.layout == 1 ? BB[i] : i, z, y * P.nx + x, f, P.sh[i]);
+        const uint64_t o = at + (uint64_t)P.geom.pos(P.layout == 1 ? BB[i] : i) * P.geom.is;
+        const S f = stored<S>(i, feq_f64(i, p, u, v, w), P.sh[i]);
+        ((S *)P.dst)[o] = f;
+        if (solid && P.other) ((S *)P.other)[o] = f;
     }
     // the fields themselves are the moments of step 0, as the reference's
     // Initialize leaves them in p, ua, va, wa; a solid cell reports a fluid at
     // rest with p = 0, as every later step leaves it
     if (P.mom[0]) {
-        const bool solid = P.mask && P.mask[c] == 1;
         P.mom[0][c] = solid ? 0.0 : p;
         P.mom[1][c] = u;
         P.mom[2][c] = v;
@@ -110,9 +125,11 @@ __global__ void k_init(const InitParams P)
     }
 }
 
-hipError_t launch_init(int dtype, const InitParams &P, hipStream_t st)
+hipError_t launch_init(int dtype, InitParams P, hipStream_t st)
 {
-    dim3 blk(256), grid((P.ncell + 255) / 256);
+    P.bpp = ((uint32_t)P.nx * P.ny + 255) / 256;
+    P.divb.init(P.bpp);
+    dim3 blk(256), grid(P.bpp * (uint32_t)P.nz);
     if (dtype == DT_F64) hipLaunchKernelGGL(k_init<double>, grid, blk, 0, st, P);
     else if (dtype == DT_F32) hipLaunchKernelGGL(k_init<float>, grid, blk, 0, st, P);
     else hipLaunchKernelGGL(k_init<_Float16>, grid, blk, 0, st, P);

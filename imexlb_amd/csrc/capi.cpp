@@ -578,6 +578,8 @@ int imexlb_initialize(imexlb_handle *h)
     P.ncell = h->ncell;
     P.geom = h->geom;
     P.dst = h->lat[0];
+    // solid cells are never written by the step: both lattices get them here
+    P.other = c.storage == IMEXLB_PULL && c.case_id == IMEXLB_CASE_SPHERE ? h->lat[1] : nullptr;
     P.layout = c.storage == IMEXLB_AA ? 1 : 0;
     P.kind = c.case_id == IMEXLB_CASE_TGV ? 0 : (bc_of(c) == BC_FAITHFUL && c.case_id == IMEXLB_CASE_SPHERE ? 2 : 1);
     P.seed = c.seed;
@@ -602,11 +604,6 @@ int imexlb_initialize(imexlb_handle *h)
         if (h->stage) HIPCHK(h, launch_faithful_stage_fill(F, h->stream));
     }
     h->cur = 0;
-    if (c.storage == IMEXLB_PULL && c.case_id == IMEXLB_CASE_SPHERE) {
-        // solid cells are never written by the step; give both lattices the
-        // same initial contents
-        HIPCHK(h, hipMemcpyAsync(h->lat[1], h->lat[0], h->lat_bytes, hipMemcpyDeviceToDevice, h->stream));
-    }
     h->steps = 0;
     h->mom_step = 0;  // k_init wrote the initial fields
     h->initialized = true;

@@ -340,6 +340,8 @@ struct InitParams {
     uint32_t ncell;
     LatGeom geom;
     void *dst;               // lattice written (stored convention)
+    void *other;             // pull with solid cells: the other lattice, where
+                             // only they are written (no step does); or null
     int layout;              // 0 natural (pull), 1 swapped (AA after an even step)
     int kind;                // 0 TGV from the per-axis tables, 1 uniform (u0,0,0)/p0, masked,
                              // 2 the faithful sphere (parabolic inlet profile, seeded perturbation)
@@ -351,8 +353,10 @@ struct InitParams {
     double *mom[4];          // p, u, v, w of the initial fields (solid cells: 0);
                              // null: not written
     FastDiv divx, divy;
+    uint32_t bpp;            // workgroups of a plane (set by launch_init)
+    FastDiv divb;
 };
-hipError_t launch_init(int dtype, const InitParams &P, hipStream_t st);
+hipError_t launch_init(int dtype, InitParams P, hipStream_t st);
 
 // Copy between the stored lattice (any dtype, pull or AA layout after step
 // count parity) and a natural-order FP64 array of post-collision populations.
