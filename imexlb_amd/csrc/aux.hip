@@ -61,7 +61,7 @@ __device__ __forceinline__ double get(const S *lat, const LatGeom &g, int slot, 
 // FP64 832 / 675, 512^3 FP64 6700 / 5400, FP16 3590 / 2450, cavity 100^3 62 / 58;
 // non-temporal stores 198, 626, 5490, 2440, 68.  The solid cells of the other
 // lattice are written here rather than by a copy of the whole: Initialize of the sphere
-// 512x128x128 1198 -> 383, channel 512x256x256 FP16 1490 -> 510.
+// 512x128x128 1198 -> 383, channel 512x256x256 FP16 1490 -> 640.
 template <typename S>
 __global__ void k_init(const InitParams P)
 {

@@ -391,7 +391,8 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
     // structure of arrays (imexlb_config.stride_pad, addr_mode)
     h->geom = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
     if (c.stride_pad < 0 && c.addr_mode < 0) tile_geom((uint32_t)c.nx, (uint32_t)c.ny, h->elem, c.storage == IMEXLB_AA, h->geom);
-    h->block = c.block ? c.block : (h->geom.tl == 31 ? 256 : tile_block((uint64_t)c.nx * c.ny, h->ncell));
+    h->block = c.block ? c.block : (h->geom.tl == 31 ? 256 : tile_block((uint64_t)c.nx * c.ny, h->ncell,
+                                                                              c.case_id == IMEXLB_CASE_SPHERE && c.dtype == IMEXLB_F16));
     h->cpt = c.cells_per_thread ? c.cells_per_thread : 1;
     h->xcd = c.xcd_remap < 0 ? 1 : c.xcd_remap;
     h->ntl = c.nt_loads < 0 ? 1 : (c.nt_loads ? 1 : 0);

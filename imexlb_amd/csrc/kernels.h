@@ -180,10 +180,16 @@ inline bool tile_nt_loads(uint64_t lattice_bytes, bool aa, uint64_t elem)
 // larger workgroups (us per step, 64 / 256: TGV 24^3 FP64 AA 4.9 / 5.8, 32^3 5.7 / 6.3, 40^3
 // 7.4 / 9.0, 56^3 14.5 / 14.8, 64^3 20.3 / 20.3 and FP16 7.0 / 6.8); above, the largest of
 // 256, 128 and 64 that leaves at most a sixteenth of the plane's threads idle, else
-// the one that leaves the fewest.
-inline int tile_block(uint64_t plane, uint64_t cells)
+// the one that leaves the fewest.  192 for the FP16 channel (`channel_f16`) once its two
+// lattices exceed the 256 MB last-level cache: us per step, 128 / 192 / 256, 512x256x256
+// 650 / 605 / 655, 448x288x184 443 / 426 / 430, 640x256x160 483 / 469 / 477, 512x256x128
+// 318 / 299 / 315, 678x246x190 600 / 577 / 589, 300x150x150 129 / 125 / 128, 384x192x192
+// 260 / 262 / 257, 224x128x128 72.4 / 70.8 / 72.6, but inside it 160x96x96 35.6 / 35.0 / 34.5; not for
+// the periodic box (256^3 297 / 301, but 384x256x256 466 / 449) nor FP32 (1248 / 1227).
+inline int tile_block(uint64_t plane, uint64_t cells, bool channel_f16)
 {
     if (cells < 200000) return 64;
+    if (channel_f16 && cells * Q * 2 * 2 > (uint64_t(256) << 20) && ((plane + 191) / 192 * 192 - plane) * 16 <= plane) return 192;
     int best = 256;
     uint64_t idle_best = ~uint64_t(0);
     for (int b = 256; b >= 64; b /= 2) {
