@@ -423,7 +423,7 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
         have = alloc_lattices();
     }
     if (c.nt_loads < 0 && h->geom.tl != 31)
-        h->ntl = tile_nt_loads(h->lat_bytes, c.storage == IMEXLB_AA, h->elem) ? 1 : 0;
+        h->ntl = tile_nt(h->lat_bytes, c.storage == IMEXLB_AA, h->elem) ? 1 : 0;
     if (!have) return bail(fail(h, IMEXLB_ENOMEM, "lattice of %zu bytes", h->lat_bytes));
     h->device_bytes += (int64_t)nlat * (int64_t)h->lat_bytes;
     for (int k = 0; k < 4; ++k) {

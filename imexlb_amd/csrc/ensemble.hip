@@ -33,6 +33,7 @@ struct EnsParams {
     const uint2 *tiles;       // (domain, first cell; plane tiles: workgroup of the domain)
     uint32_t t0, ntiles;      // this launch's tiles: [t0, ntiles)
     int order;                // tile.h tile_block_of
+    bool nt;                  // kernels.h tile_nt
     int parity;               // pull: which lattice of each pair is read
     int write_moments;
 };
@@ -77,13 +78,14 @@ __device__ __forceinline__ T read_const(const T *p)
 // Persistent over one run of the tile table (or one workgroup per tile, grid
 // 0): every workgroup exits after its last tile.  Members in plane tiles
 // (TILED: every plane of 512 cells or more) run tile.h's cells, periodic and cavity
-// in one launch, the choice being the workgroup's; members in arrays run
+// in one launch, the choice being the workgroup's (NT: tile_nt of all of them);
+// members in arrays run
 // fused.h's, one launch per boundary kind (BC), since both kinds in one kernel
 // would hold the registers of the larger.  15 members of 32^3-96^3, us a step: FP32
 // pull 243 in arrays with 2048 persistent workgroups (the default before), 233 in
 // arrays with one workgroup per tile, 202 in tiles, 196 with one launch for both
 // kinds (218 persistent); FP64 pull 475 -> 389, FP16 AA 142 -> 113.
-template <typename S, int BC, int PAT, int CPT, bool TILED>
+template <typename S, int BC, int PAT, int CPT, bool TILED, bool NT>
 __global__ void __launch_bounds__(512) k_ensemble(const EnsParams EP)
 {
     const bool wm = EP.write_moments != 0;
@@ -94,28 +96,26 @@ __global__ void __launch_bounds__(512) k_ensemble(const EnsParams EP)
         const uint32_t t = EP.t0 + (TILED ? tile_block_of(EP.order, v, count) : xcd_tile(v, count));
         const uint2 tl = read_const(EP.tiles + t);
         FusedParams P = read_const(EP.doms + 2 * tl.x + (uint32_t)EP.parity);
-        // non-temporal loads of unshared lines (measured faster on every
-        // storage type of the single-domain kernel)
         if constexpr (TILED) {
             if (!wm) P.mom_p = nullptr;
             const uint32_t z = P.divb.div(tl.y);
             const uint32_t p0 = (tl.y - z * P.bpp) * blockDim.x * CPT + threadIdx.x;
-            if (P.bc == BC_PERIODIC) tile_cells<S, BC_PERIODIC, PAT, CPT, true>(P, z, p0);
-            else tile_cells<S, BC_CAVITY, PAT, CPT, true>(P, z, p0);
+            if (P.bc == BC_PERIODIC) tile_cells<S, BC_PERIODIC, PAT, CPT, NT>(P, z, p0);
+            else tile_cells<S, BC_CAVITY, PAT, CPT, NT>(P, z, p0);
         } else {
-            tile_run<S, BC, PAT, CPT, true>(P, tl.y, wm);
+            tile_run<S, BC, PAT, CPT, NT>(P, tl.y, wm);
         }
     }
 }
 
-template <typename S, int BC, int CPT, bool TILED>
+template <typename S, int BC, int CPT, bool TILED, bool NT>
 static hipError_t launch_ens_bc(int pattern, const EnsParams &EP, int grid, int block, hipStream_t st)
 {
     if (pattern == PAT_PULL)
-        hipLaunchKernelGGL((k_ensemble<S, BC, PAT_PULL, CPT, TILED>), dim3(grid), dim3(block), 0, st, EP);
+        hipLaunchKernelGGL((k_ensemble<S, BC, PAT_PULL, CPT, TILED, NT>), dim3(grid), dim3(block), 0, st, EP);
     else if (pattern == PAT_AA_EVEN)
-        hipLaunchKernelGGL((k_ensemble<S, BC, PAT_AA_EVEN, CPT, TILED>), dim3(grid), dim3(block), 0, st, EP);
-    else hipLaunchKernelGGL((k_ensemble<S, BC, PAT_AA_ODD, CPT, TILED>), dim3(grid), dim3(block), 0, st, EP);
+        hipLaunchKernelGGL((k_ensemble<S, BC, PAT_AA_EVEN, CPT, TILED, NT>), dim3(grid), dim3(block), 0, st, EP);
+    else hipLaunchKernelGGL((k_ensemble<S, BC, PAT_AA_ODD, CPT, TILED, NT>), dim3(grid), dim3(block), 0, st, EP);
     return hipGetLastError();
 }
 
@@ -123,9 +123,10 @@ template <typename S, int CPT>
 static hipError_t launch_ens_cpt(int bc, bool tiled, int pattern, const EnsParams &EP, int grid, int block,
                                  hipStream_t st)
 {
-    if (tiled) return launch_ens_bc<S, BC_PERIODIC, CPT, true>(pattern, EP, grid, block, st);
-    if (bc == BC_PERIODIC) return launch_ens_bc<S, BC_PERIODIC, CPT, false>(pattern, EP, grid, block, st);
-    return launch_ens_bc<S, BC_CAVITY, CPT, false>(pattern, EP, grid, block, st);
+    if (tiled && EP.nt) return launch_ens_bc<S, BC_PERIODIC, CPT, true, true>(pattern, EP, grid, block, st);
+    if (tiled) return launch_ens_bc<S, BC_PERIODIC, CPT, true, false>(pattern, EP, grid, block, st);
+    if (bc == BC_PERIODIC) return launch_ens_bc<S, BC_PERIODIC, CPT, false, true>(pattern, EP, grid, block, st);
+    return launch_ens_bc<S, BC_CAVITY, CPT, false, true>(pattern, EP, grid, block, st);
 }
 
 static hipError_t launch_ensemble(int dtype, int cpt, int bc, bool tiled, int pattern, const EnsParams &EP, int grid,
@@ -272,6 +273,13 @@ static int pattern_of(const imexlb_ensemble *e)
     return (e->steps % 2 == 0) ? PAT_AA_ODD : PAT_AA_EVEN;
 }
 
+// every member's lattice, and their accesses in plane tiles
+static uint64_t lattice_bytes(const imexlb_ensemble *e) { return e->pool_bytes / (e->storage == IMEXLB_PULL ? 2 : 1); }
+static bool nt_of(const imexlb_ensemble *e)
+{
+    return tile_nt(lattice_bytes(e), e->storage == IMEXLB_AA, e->dtype == IMEXLB_F64 ? 8 : e->dtype == IMEXLB_F32 ? 4 : 2);
+}
+
 static int launch_persistent(imexlb_ensemble *e, int pattern, int parity, bool wm)
 {
     EnsParams EP;
@@ -279,7 +287,8 @@ static int launch_persistent(imexlb_ensemble *e, int pattern, int parity, bool w
     EP.tiles = e->dtiles;
     EP.parity = parity;
     EP.write_moments = wm ? 1 : 0;
-    EP.order = tile_order(e->pool_bytes / (e->storage == IMEXLB_PULL ? 2 : 1), e->storage == IMEXLB_AA);
+    EP.order = tile_order(lattice_bytes(e), e->storage == IMEXLB_AA);
+    EP.nt = nt_of(e);
     // the runs, back to back on the stream
     for (int r = 0; r < 3; ++r) {
         if (e->bounds[r + 1] == e->bounds[r]) continue;
@@ -302,6 +311,7 @@ static int ens_step(imexlb_ensemble *e, bool per_domain, bool wm)
         for (int d = 0; d < e->n; ++d) {
             FusedParams P = e->hp[2 * d + parity];
             P.xcd_remap = 0;
+            if (P.geom.tl != 31) P.ntl = nt_of(e) ? 1 : 0;
             if (!wm) P.mom_p = P.mom_u = P.mom_v = P.mom_w = nullptr;
             ECHK(e, launch_fused(e->dtype, P.bc, pattern, P, e->block, e->stream));
         }

@@ -157,22 +157,29 @@ inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, bool aa, LatGeom 
 
 // The XCD-aware order of the plane-tile kernels (tile.h tile_block_of, with the
 // measurements): one run of the lattice per XCD (1) where the lattices of a
-// step fit the caches it hopes to find them in -- the 256 MB last-level cache
-// for AA, whose step writes what it reads, 48 MB for pull, somewhat beyond the
-// L2s' 32 MB -- else runs of eight workgroups.
+// step fit the 256 MB last-level cache, else runs of eight workgroups.
 constexpr int XCD_RUNS = 2;
+constexpr uint64_t LAST_LEVEL = uint64_t(256) << 20;
 inline int tile_order(uint64_t lattice_bytes, bool aa)
 {
-    return (aa ? lattice_bytes : 2 * lattice_bytes) <= (uint64_t(aa ? 256 : 48) << 20) ? 1 : XCD_RUNS;
+    return (aa ? lattice_bytes : 2 * lattice_bytes) <= LAST_LEVEL ? 1 : XCD_RUNS;
 }
 
-// Default for non-temporal loads (imexlb_config.nt_loads) over plane tiles: not
-// where an AA lattice stays in the caches and its elements are small (us per
-// step, non-temporal / plain: FP16 160^3 81.1 / 63.6, 128^3 39.8 / 34.6, 48^3 4.8 / 4.5; FP32
-// 64^3 8.4 / 7.9, but 96^3 30.6 / 31.6; FP64 64^3 20.5 / 20.7, 128^3 142 / 171).
-inline bool tile_nt_loads(uint64_t lattice_bytes, bool aa, uint64_t elem)
+// Default for non-temporal accesses (imexlb_config.nt_loads) over plane tiles: not
+// where the lattices of a step fit the 256 MB last-level cache, which keeps what
+// plain loads and stores bring in (an in-place pass over 64 to 256 MB: 6.4 TB/s
+// non-temporal, 6.6-7.1 plain; over 448 MB 6.4 and 5.7).  us per step,
+// non-temporal / plain: pull FP64 64^3 22.5 / 18.7, 80^3 41.8 / 34.9, FP32 96^3
+// 34.7 / 29.4, FP16 96^3 19.7 / 17.0, faithful cavity 80^3 48.0 / 41.6, but FP64 96^3 (382 MB)
+// 67.3 / 72.0; AA FP64 64^3 20.4 / 18.8, 96^3 59.6 / 56.1, 128^3 (453 MB) 138 / 161, FP32
+// 128^3 66.2 / 63.9, FP16 128^3 40.1 / 34.2.
+//
+// FP64 pull lattices of about the L2s' 32 MB stay non-temporal (32^3 5.34 / 5.31, 36^3
+// 5.79 / 6.09, 40^3 6.38 / 7.18, 44^3 8.21 / 8.95, 48^3 10.14 / 10.24, 52^3 14.7 / 12.1).
+inline bool tile_nt(uint64_t lattice_bytes, bool aa, uint64_t elem)
 {
-    return !aa || elem == 8 || lattice_bytes > (uint64_t(elem == 2 ? 256 : 64) << 20);
+    const uint64_t bytes = aa ? lattice_bytes : 2 * lattice_bytes, mib = uint64_t(1) << 20;
+    return bytes > LAST_LEVEL || (!aa && elem == 8 && bytes > 16 * mib && bytes <= 40 * mib);
 }
 
 // Threads per workgroup of the plane-tile kernels where the caller names
@@ -189,7 +196,7 @@ inline bool tile_nt_loads(uint64_t lattice_bytes, bool aa, uint64_t elem)
 inline int tile_block(uint64_t plane, uint64_t cells, bool channel_f16)
 {
     if (cells < 200000) return 64;
-    if (channel_f16 && cells * Q * 2 * 2 > (uint64_t(256) << 20) && ((plane + 191) / 192 * 192 - plane) * 16 <= plane) return 192;
+    if (channel_f16 && cells * Q * 2 * 2 > LAST_LEVEL && ((plane + 191) / 192 * 192 - plane) * 16 <= plane) return 192;
     int best = 256;
     uint64_t idle_best = ~uint64_t(0);
     for (int b = 256; b >= 64; b /= 2) {
@@ -246,7 +253,8 @@ struct FusedParams {
     int xcd_remap;           // 1: give each XCD one contiguous run of tiles; plane tiles: tile_order
     int cpt;                 // cells per thread: 1, 2 (blockDim apart) or 3 (two adjacent
                              // x cells; periodic lattices with nx even, else 1)
-    int ntl;                 // 1: non-temporal loads of unshared lines
+    int ntl;                 // 1: non-temporal loads of unshared lines; plane tiles:
+                             // and stores (0: plain)
     int am_max;              // widest-saving address mode allowed (AddrMode in fused.h)
     int bc;                  // boundary kind (read by the ensemble kernel)
     FastDiv divx, divy;

@@ -11,9 +11,6 @@
 
 #include "fused.h"
 
-#ifndef IMX_TILE_ODD_NT
-#define IMX_TILE_ODD_NT 1
-#endif
 namespace imx {
 
 struct TileCtx {
@@ -108,7 +105,7 @@ __device__ __forceinline__ void tile_planes(S *lat, const FusedParams &P, uint32
 
 // The 27 populations arriving at the cell (cell_gather's rules).  CLEAR: no
 // lane of the wavefront is beside the channel's ball.
-template <typename S, int BC, int PAT, bool NTL, bool CLEAR = true>
+template <typename S, int BC, int PAT, bool NT, bool CLEAR = true>
 __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx &t, const S *const (&pl)[3],
                                             typename RealOf<S>::type (&f)[Q])
 {
@@ -118,7 +115,7 @@ __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx 
 #pragma unroll
     for (int i = 0; i < Q; ++i) {
         if constexpr (PAT == PAT_AA_EVEN) {
-            f[i] = ld_ptr<S, NTL>(tile_ptr<PAT>(pl[1], P, i, t.o[1][1]), WCLASS[i]);
+            f[i] = ld_ptr<S, NT>(tile_ptr<PAT>(pl[1], P, i, t.o[1][1]), WCLASS[i]);
             if constexpr (BC == BC_CAVITY) {
                 if (EZ[i] < 0) {
                     R lid;
@@ -132,7 +129,7 @@ __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx 
             const S *const from = pl[1 - EZ[i]];
             const uint32_t o = t.o[1 - EY[i]][1 - EX[i]];
             // lines that no other wavefront reads are not kept
-            const bool nt = NTL && EX[i] == 0;
+            const bool nt = NT && EX[i] == 0;
             if constexpr (BC == BC_PERIODIC) {
                 const S *p = tile_ptr<PAT>(from, P, s, o);
                 f[i] = nt ? ld_ptr<S, true>(p, WCLASS[i]) : ld_ptr<S, false>(p, WCLASS[i]);
@@ -202,7 +199,7 @@ __device__ __forceinline__ void tile_gather(const FusedParams &P, const TileCtx 
     }
 }
 
-template <typename S, int BC, int PAT>
+template <typename S, int BC, int PAT, bool NT>
 __device__ __forceinline__ void tile_scatter(const FusedParams &P, const TileCtx &t, S *const (&pl)[3],
                                              const typename RealOf<S>::type (&f)[Q])
 {
@@ -223,7 +220,7 @@ __device__ __forceinline__ void tile_scatter(const FusedParams &P, const TileCtx
         if constexpr (BC == BC_FAITHFUL) stage_rows(P, k, f);
 #pragma unroll
         for (int i = 0; i < Q; ++i)
-            st_ptr<S>(tile_ptr<PAT>(pl[1], P, PAT == PAT_PULL ? i : BB[i], o9[1][1]), WCLASS[i], f[i]);
+            st_ptr<S, NT>(tile_ptr<PAT>(pl[1], P, PAT == PAT_PULL ? i : BB[i], o9[1][1]), WCLASS[i], f[i]);
     } else {
         // to slot i of x + e_i, or bounced back into slot bb(i) at x
 #pragma unroll
@@ -240,8 +237,7 @@ __device__ __forceinline__ void tile_scatter(const FusedParams &P, const TileCtx
             } else {
                 p = tile_ptr<PAT>(to, P, i, o);
             }
-            if (IMX_TILE_ODD_NT || EX[i] == 0) st_ptr<S, true>(p, WCLASS[i], f[i]);
-            else st_ptr<S, false>(p, WCLASS[i], f[i]);
+            st_ptr<S, NT>(p, WCLASS[i], f[i]);
         }
     }
 }
@@ -251,21 +247,21 @@ __device__ __forceinline__ void tile_scatter(const FusedParams &P, const TileCtx
 // 677 vector operations for a cell instead of 1055, us per step before /
 // after: cavity 128^3 AA 146.7 / 136.0, TGV 96^3 AA 63.6 / 59.2, 64^3 AA 21.4 / 20.0, 32^3 pull
 // 5.8 / 5.2, 256^3 pull 1211 / 1202 (HBM).
-template <typename S, int BC, int PAT>
+template <typename S, int BC, int PAT, bool NT>
 __device__ __forceinline__ void tile_finish(const FusedParams &P, const TileCtx &t, S *const (&dst)[3],
                                             typename RealOf<S>::type (&f)[Q])
 {
     if constexpr (std::is_same<S, double>::value) {
         if (P.inv_den == 0.0 || wave_any(!div_safe(f))) {
             cell_collide_f64<BC, false>(P, t.k, f, P.mom_p != nullptr);
-            if (t.k.live) tile_scatter<S, BC, PAT>(P, t, dst, f);
+            if (t.k.live) tile_scatter<S, BC, PAT, NT>(P, t, dst, f);
         } else {
             cell_collide_f64<BC, true>(P, t.k, f, P.mom_p != nullptr);
-            if (t.k.live) tile_scatter<S, BC, PAT>(P, t, dst, f);
+            if (t.k.live) tile_scatter<S, BC, PAT, NT>(P, t, dst, f);
         }
     } else {
         cell_collide<S, BC>(P, t.k, f, P.mom_p != nullptr);
-        if (t.k.live) tile_scatter<S, BC, PAT>(P, t, dst, f);
+        if (t.k.live) tile_scatter<S, BC, PAT, NT>(P, t, dst, f);
     }
 }
 
@@ -278,9 +274,10 @@ __device__ __forceinline__ void tile_finish(const FusedParams &P, const TileCtx 
 // window of the lattice.  tile_order chooses.  us per step, linear / one run /
 // runs of 8, block 256: pull TGV 256^3 FP64 1292 / 1218 / 1209, FP32 605 / 621 / 603, FP16
 // 310 / 310 / 297, 301x203x157 FP32 337 / 367 / 342, channel 512x256x256 FP16 640 / 702 /
-// 637, 96^3 FP32 34.8 / 37.4 / 34.7, 48^3 FP32 7.7 / 5.6 / 7.6; AA TGV 128^3 FP64 143.7 /
-// 144.7 / 141.9, 160^3 FP32 145 / 144 / 139, 128^3 FP32 67.6 / 65.7 / 67.3, 80^3 FP16 14.2 /
-// 10.8 / 13.0, 48^3 FP64 11.9 / 9.4 / 11.6.
+// 637; in the last-level cache, with plain stores, 80^3 FP64 36.2 / 33.8 / 35.1, 96^3
+// FP32 31.0 / 28.5 / 29.5, 48^3 FP32 9.9 / 5.4 / 8.2, 112^3 FP16 28.5 / 23.7 / 25.3; AA TGV
+// 160^3 FP32 145 / 144 / 139, 128^3 66.0 / 64.1 / 65.3, 96^3 FP64 59.1 / 56.2 / 57.7, 48^3 11.9 / 8.4 /
+// 10.9, 80^3 FP16 12.0 / 9.4 / 11.1.
 __device__ __forceinline__ uint32_t tile_block_of(int order, uint32_t b, uint32_t nb)
 {
     constexpr uint32_t RUN = 8, ALL = 8 * RUN;
@@ -291,7 +288,7 @@ __device__ __forceinline__ uint32_t tile_block_of(int order, uint32_t b, uint32_
 
 // CPT cells per thread, blockDim.x apart, of plane z from cell p0; the loads of
 // all are issued before any of them is collided.
-template <typename S, int BC, int PAT, int CPT, bool NTL>
+template <typename S, int BC, int PAT, int CPT, bool NT>
 __device__ __forceinline__ void tile_cells(const FusedParams &P, uint32_t z, uint32_t p0)
 {
     using R = typename RealOf<S>::type;
@@ -315,27 +312,27 @@ __device__ __forceinline__ void tile_cells(const FusedParams &P, uint32_t z, uin
     if (BC == BC_CHANNEL && wave_any(near)) {
 #pragma unroll
         for (int r = 0; r < CPT; ++r) {
-            tile_gather<S, BC, PAT, NTL, false>(P, t[r], src, f[r]);
-            tile_finish<S, BC, PAT>(P, t[r], dst, f[r]);
+            tile_gather<S, BC, PAT, NT, false>(P, t[r], src, f[r]);
+            tile_finish<S, BC, PAT, NT>(P, t[r], dst, f[r]);
         }
         return;
     }
 #pragma unroll
-    for (int r = 0; r < CPT; ++r) tile_gather<S, BC, PAT, NTL>(P, t[r], src, f[r]);
+    for (int r = 0; r < CPT; ++r) tile_gather<S, BC, PAT, NT>(P, t[r], src, f[r]);
 #pragma unroll
-    for (int r = 0; r < CPT; ++r) tile_finish<S, BC, PAT>(P, t[r], dst, f[r]);
+    for (int r = 0; r < CPT; ++r) tile_finish<S, BC, PAT, NT>(P, t[r], dst, f[r]);
 }
 
 // Before (structure of arrays, k_fused) and after, us per step, first
 // allocations: TGV 256^3 FP64 pull 1342 -> 1202 (6.03 TB/s algorithmic), 301x203x157
 // FP32 pull 414 -> 340, channel 512x256x256 FP16 712 -> 615, the reference's sphere
 // 512x128x128 715 -> 642 with its boundary kernels, cavity 128^3 FP64 AA 153 -> 136.
-template <typename S, int BC, int PAT, int CPT, bool NTL>
+template <typename S, int BC, int PAT, int CPT, bool NT>
 __global__ void __launch_bounds__(512) k_tiled(const FusedParams P)
 {
     const uint32_t b = tile_block_of(P.xcd_remap, blockIdx.x, P.nblocks);
     const uint32_t z = P.divb.div(b);
-    tile_cells<S, BC, PAT, CPT, NTL>(P, z, (b - z * P.bpp) * blockDim.x * CPT + threadIdx.x);
+    tile_cells<S, BC, PAT, CPT, NT>(P, z, (b - z * P.bpp) * blockDim.x * CPT + threadIdx.x);
 }
 
 // The value of the lane before (EXP 1) or after (EXP -1); the first (last)
@@ -371,7 +368,7 @@ struct RowEdges {
     R v[8][2][10];
 };
 
-template <typename S, int BC, bool NTL>
+template <typename S, int BC, bool NT>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k_tiled_rows(const FusedParams P)
 {
     using R = typename RealOf<S>::type;
@@ -412,7 +409,7 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
         // from slot bb(i) of x - e_i; where that row lies outside the cavity,
         // the cell's own slot i, not shifted
         const bool o = zo[1 - EZ[i]] || yo[1 - EY[i]];
-        f[i] = ld_ptr<S, NTL>(o ? at(1, 1, i, lane) : at(1 - EZ[i], 1 - EY[i], BB[i], lane), WCLASS[i]);
+        f[i] = ld_ptr<S, NT>(o ? at(1, 1, i, lane) : at(1 - EZ[i], 1 - EY[i], BB[i], lane), WCLASS[i]);
     }
     // cells at an x wall take their own slot i
     R wall[9];
@@ -467,7 +464,6 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
     CellCtx k;
     k.c = z * plane + y * nx + x;
     k.live = live;
-    k.live = live;
     // FP64 keeps the IEEE division: the choice of tile_finish takes 12 registers
     // more than four wavefronts per SIMD leave, and these lattices wait for HBM
     cell_collide<S, BC>(P, k, f, P.mom_p != nullptr);
@@ -501,11 +497,11 @@ __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4))) k
     }
 }
 
-template <typename S, int CPT, bool NTL>
+template <typename S, int CPT, bool NT>
 hipError_t launch_tiled_cpt(int bc, int pattern, const FusedParams &P, int block, hipStream_t st)
 {
     dim3 grid(P.nblocks), blk(block);
-#define IMX_L(B, PT) hipLaunchKernelGGL((k_tiled<S, B, PT, CPT, NTL>), grid, blk, 0, st, P)
+#define IMX_L(B, PT) hipLaunchKernelGGL((k_tiled<S, B, PT, CPT, NT>), grid, blk, 0, st, P)
     if (bc == BC_PERIODIC) {
         if (pattern == PAT_PULL) IMX_L(BC_PERIODIC, PAT_PULL);
         else if (pattern == PAT_AA_EVEN) IMX_L(BC_PERIODIC, PAT_AA_EVEN);
