@@ -446,7 +446,9 @@ int imexlb_ensemble_create(const imexlb_domain *doms, int n, int dtype, int stor
         e->pool_bytes = 0;
         for (int d = 0; d < n; ++d) {
             geom[d] = soa_geom((uint32_t)doms[d].nx, (uint32_t)doms[d].ny, pstride[d]);
-            if (tiles) tile_geom((uint32_t)doms[d].nx, (uint32_t)doms[d].ny, elem, storage == IMEXLB_AA, geom[d]);
+            // smaller planes would leave most of a workgroup of 256 idle
+            if (tiles && (uint64_t)doms[d].nx * doms[d].ny >= 512)
+                tile_geom((uint32_t)doms[d].nx, (uint32_t)doms[d].ny, elem, storage == IMEXLB_AA, geom[d]);
             for (int k = 0; k < nl; ++k) {
                 e->lat_off[2 * d + k] = e->pool_bytes;
                 e->pool_bytes += ((size_t)lattice_elems(geom[d], (uint32_t)doms[d].nz) * elem + 4095) / 4096 * 4096;

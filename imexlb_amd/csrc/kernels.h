@@ -136,13 +136,16 @@ inline uint64_t lattice_elems(const LatGeom &g, uint32_t nz)
 
 // Plane tiles for a lattice, where they serve: the largest tile of at most
 // 32 KiB per population (at least 64 cells) whose last tile leaves at most a
-// sixteenth of the plane unused.  Not for planes below 512 cells, whose
-// workgroups would be mostly idle (a workgroup never spans two planes), nor
-// where three planes exceed the 4 GiB that the kernels' 32-bit offsets reach.
+// sixteenth of the plane unused.  Not for planes below 64 cells, whose wavefronts
+// would be mostly idle (a workgroup never spans two planes), nor where three
+// planes exceed the 4 GiB that the kernels' 32-bit offsets reach.  us per step, arrays /
+// tiles: TGV 8^3 FP64 5.6 / 4.1, 16^3 5.86 / 4.17, FP32 4.12 / 3.19, FP16 AA 3.88 / 3.15, 9x13x30 FP64
+// 5.88 / 4.15, 22x18x22 6.03 / 4.32, faithful cavity 16^3 10.1 / 8.8, 12x12x3000 FP64 41.7 / 28.7 (but
+// 16x16x400 FP64 pull 9.5 / 9.9 and FP16 AA 12x12x3000 10.5 / 11.1).
 inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, bool aa, LatGeom &g)
 {
     const uint64_t plane = (uint64_t)nx * ny;
-    if (plane < 512) return false;
+    if (plane < 64) return false;
     uint32_t tl = 6;
     for (uint32_t t = 6; (elem << t) <= 32768; ++t) {
         const uint64_t n = ((plane - 1) >> t) + 1;

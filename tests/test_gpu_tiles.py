@@ -7,7 +7,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-# (32, 16): the smallest tiled plane; (45, 37), (129, 33): ragged rows and
+# (32, 16): one tile of 512 cells; (45, 37), (129, 33): ragged rows and
 # tiles; (64, 64), (128, 32): whole tiles; (700, 2) and (2, 300): one and many
 # rows per workgroup; (64, 9), (192, 7), (512, 3): rows of one, three and eight
 # wavefronts, with rows left over in the last workgroup
@@ -113,3 +113,34 @@ def test_ensemble_mixes_layouts(dtype, storage):
                 for name, a, b in zip("puvw", want[k], e.moments(k)):
                     assert np.array_equal(a, b), f"member {k} {name}, launch {launch}, {mode}"
     e.close()
+
+
+# (8, 8): the smallest tiled plane; (7, 9): the largest that is not; (13, 5),
+# (2, 33): one cell more than a wavefront; (9, 13), (16, 31): ragged
+SMALL_PLANES = [(8, 8, 3), (7, 9, 4), (13, 5, 6), (2, 33, 5), (9, 13, 2), (16, 31, 3)]
+
+
+@pytest.mark.parametrize("n", SMALL_PLANES)
+@pytest.mark.parametrize("case,mode,dtype,storage", [("tgv", "faithful", "f64", "pull"), ("tgv", "faithful", "f32", "aa"),
+                                                     ("cavity", "config", "f64", "aa"), ("cavity", "config", "f16", "pull"),
+                                                     ("cavity", "faithful", "f64", "pull")])
+def test_small_planes_equal_arrays(n, case, mode, dtype, storage):
+    print(f"[case] small planes {case} {mode} {n} {dtype} {storage}", flush=True)
+    kw = dict(case=case, mode=mode, dtype=dtype, storage=storage, tau=0.1)
+    for steps in (6, 7):
+        want = state(n, steps, addr_mode=2, **kw)
+        for shape in (None, (128, 2, 1, 0), (64, 1, 0, 1)):
+            same(state(n, steps, shape, **kw), want, f"{steps} steps, launch {shape}")
+
+
+# both accesses of plane tiles (nt_loads), on both sides of the rule that chooses
+@pytest.mark.parametrize("n,dtype,storage", [((40, 41, 39), "f64", "pull"), ((24, 40, 21), "f64", "aa"),
+                                             ((33, 31, 30), "f32", "pull"), ((64, 64, 9), "f16", "aa")])
+@pytest.mark.parametrize("case,mode", [("tgv", "faithful"), ("cavity", "config")])
+def test_plain_and_non_temporal_agree(n, dtype, storage, case, mode):
+    print(f"[case] accesses {case} {n} {dtype} {storage}", flush=True)
+    kw = dict(case=case, mode=mode, dtype=dtype, storage=storage)
+    want = state(n, 7, addr_mode=2, **kw)
+    for nt in (0, 1):
+        same(state(n, 7, (64, 1, 1, nt), **kw), want, f"nt {nt}")
+    same(state(n, 7, **kw), want, "default")
