@@ -38,6 +38,7 @@ struct imexlb_handle {
     int nparts = 1024;
     uint64_t pstride = 0;    // structure of arrays: elements between populations
     LatGeom geom{};          // the lattices' layout
+    size_t lat_held = 0;     // bytes allocated for each lattice outside a window
     size_t lat_bytes = 0;    // one lattice
     uint32_t ncell = 0;
     size_t elem = 8;
@@ -299,7 +300,7 @@ static void graph_key(const imexlb_handle *h, uint64_t (&key)[8])
     key[2] = (uint64_t)h->cur;
     key[3] = (uint64_t)(h->steps & 1);
     key[4] = (uint64_t)h->block;
-    key[5] = (uint64_t)h->cpt;
+    key[5] = (uint64_t)h->cpt | (uint64_t)h->geom.tl << 8;  // the shape and the layout
     key[6] = (uint64_t)h->xcd;
     key[7] = (uint64_t)h->ntl;
 }
@@ -425,6 +426,7 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
     if (c.nt_loads < 0 && h->geom.tl != 31)
         h->ntl = tile_nt(h->lat_bytes, c.storage == IMEXLB_AA, h->elem) ? 1 : 0;
     if (!have) return bail(fail(h, IMEXLB_ENOMEM, "lattice of %zu bytes", h->lat_bytes));
+    h->lat_held = h->lat_bytes;
     h->device_bytes += (int64_t)nlat * (int64_t)h->lat_bytes;
     for (int k = 0; k < 4; ++k) {
         if (hipMalloc(&h->mom[k], (size_t)h->ncell * 8) != hipSuccess)
@@ -1074,6 +1076,34 @@ int imexlb_set_launch(imexlb_handle *h, int block, int cpt, int xcd, int ntl)
     return IMEXLB_OK;
 }
 
+// What a placement search times at each place: the handle's layout, and for a
+// lattice in plane tiles beyond the last-level cache also arrays.  Tiles run at nearly
+// the same rate anywhere, arrays at most places slower but faster at the best
+// (TGV 512^3 AA FP64 over 96 GiB, GLUPS: tiles 13.9-14.1, arrays 12.1-14.7; FP32 28.0-28.4 and
+// 24.5-29.7; FP16 55.6-58.1 and 48.6-57.3), and a search looks for the best place.
+struct Layout {
+    LatGeom geom;
+    size_t lat_bytes;
+    int block, ntl;
+};
+static std::vector<Layout> layouts_of(const imexlb_handle *h)
+{
+    const imexlb_config &c = h->cfg;
+    std::vector<Layout> all{{h->geom, h->lat_bytes, h->block, h->ntl}};
+    if (h->geom.tl != 31 && tile_nt(h->lat_bytes, c.storage == IMEXLB_AA, h->elem)) {
+        const LatGeom g = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
+        all.push_back({g, (size_t)(lattice_elems(g, (uint32_t)c.nz) * h->elem), h->block == 192 ? 256 : h->block, h->ntl});
+    }
+    return all;
+}
+static void use_layout(imexlb_handle *h, const Layout &l)
+{
+    h->geom = l.geom;
+    h->lat_bytes = l.lat_bytes;
+    h->block = l.block;
+    h->ntl = l.ntl;
+}
+
 int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per_step, int32_t *chosen)
 {
     if (!h) return IMEXLB_EINVAL;
@@ -1083,7 +1113,10 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
     if (rc) return rc;
     if (steps < 2) steps = 2;
     steps += steps & 1;  // whole AA periods
-    const size_t lat_bytes = h->lat_bytes;
+    const std::vector<Layout> lay = layouts_of(h);
+    const size_t held = h->lat_held;  // by candidate 0
+    size_t most = 0;                  // by the others
+    for (const Layout &l : lay) most = std::max(most, l.lat_bytes);
     const int nlat = h->cfg.storage == IMEXLB_PULL ? 2 : 1;
     // candidate 0 is the current lattice, which may lie in a window
     imx::ChunkedWindow win0 = std::move(h->win);
@@ -1097,13 +1130,14 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
         if (!r) out /= (float)steps;
         return r;
     };
+    std::vector<int> of(trials, 0);  // each candidate's faster layout
     rc = time_current(ms[0]);
     for (int t = 1; !rc && t < trials; ++t) {
         size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < nlat * lat_bytes + (2ull << 30)) break;
+        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < nlat * most + (2ull << 30)) break;
         std::array<void *, 2> p{nullptr, nullptr};
         bool ok = true;
-        for (int k = 0; k < nlat && ok; ++k) ok = hipMalloc(&p[k], lat_bytes) == hipSuccess;
+        for (int k = 0; k < nlat && ok; ++k) ok = hipMalloc(&p[k], most) == hipSuccess;
         if (!ok) {
             (void)hipGetLastError();
             for (void *q : p)
@@ -1113,7 +1147,15 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
         cand.push_back(p);
         h->lat[0] = p[0];
         h->lat[1] = p[1];
-        rc = time_current(ms[t]);
+        for (int l = 0; !rc && l < (int)lay.size(); ++l) {
+            float m = 0;
+            use_layout(h, lay[l]);
+            rc = time_current(m);
+            if (l == 0 || m < ms[t]) {
+                ms[t] = m;
+                of[t] = l;
+            }
+        }
     }
     int best = 0;
     if (!rc)
@@ -1123,7 +1165,7 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
     for (int t = 0; t < (int)cand.size(); ++t) {
         if (t == best) continue;
         if (t == 0 && !win0.empty()) {
-            h->device_bytes -= (int64_t)win0.held() - (int64_t)(nlat * lat_bytes);
+            h->device_bytes -= (int64_t)win0.held() - (int64_t)(nlat * held);
             imx::window_destroy(win0);
             continue;
         }
@@ -1132,7 +1174,13 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
     }
     h->lat[0] = cand[best][0];
     h->lat[1] = cand[best][1];
-    if (best == 0) h->win = std::move(win0);
+    use_layout(h, lay[of[best]]);
+    if (best == 0) {
+        h->win = std::move(win0);
+    } else {
+        h->device_bytes += (int64_t)nlat * ((int64_t)most - (int64_t)held);
+        h->lat_held = most;
+    }
     const int rc2 = imexlb_initialize(h);
     if (rc) return rc;
     if (ms_per_step)
@@ -1157,9 +1205,11 @@ int imexlb_tune_placement_window(imexlb_handle *h, int64_t slack_bytes, int64_t 
     if (rc) return rc;
     if (steps < 2) steps = 2;
     steps += steps & 1;  // whole AA periods
-    const size_t lat_bytes = h->lat_bytes;
+    const std::vector<Layout> lay = layouts_of(h);
+    size_t most = 0;
+    for (const Layout &l : lay) most = std::max(most, l.lat_bytes);
     const int nlat = h->cfg.storage == IMEXLB_PULL ? 2 : 1;
-    const size_t total = (size_t)nlat * lat_bytes + (size_t)slack_bytes;
+    const size_t total = (size_t)nlat * most + (size_t)slack_bytes;
     size_t free_b = 0, total_b = 0;
     HIPCHK(h, hipMemGetInfo(&free_b, &total_b));
     if (free_b < total + (2ull << 30))
@@ -1174,16 +1224,28 @@ int imexlb_tune_placement_window(imexlb_handle *h, int64_t slack_bytes, int64_t 
     char *const big = w.base;
     void *old_lat[2] = {h->lat[0], h->lat[1]};
     std::vector<float> ms((size_t)npos, 0.0f);
-    for (int64_t k = 0; k < npos && !rc; ++k) {
+    std::vector<int> of((size_t)npos, 0);  // each position's faster layout
+    auto place = [&](int64_t k, int l) {
+        use_layout(h, lay[l]);
         h->lat[0] = (char *)big + k * step_bytes;
-        h->lat[1] = nlat == 2 ? (char *)h->lat[0] + lat_bytes : nullptr;
-        rc = imexlb_initialize(h);
-        if (!rc) rc = imexlb_step(h, 2, 0);
-        if (!rc) rc = imexlb_step_timed(h, steps, 0, &ms[k]);
-        if (!rc) ms[k] /= (float)steps;
-    }
+        h->lat[1] = nlat == 2 ? (char *)h->lat[0] + h->lat_bytes : nullptr;
+    };
+    for (int64_t k = 0; k < npos && !rc; ++k)
+        for (int l = 0; l < (int)lay.size() && !rc; ++l) {
+            float m = 0;
+            place(k, l);
+            rc = imexlb_initialize(h);
+            if (!rc) rc = imexlb_step(h, 2, 0);
+            if (!rc) rc = imexlb_step_timed(h, steps, 0, &m);
+            m /= (float)steps;
+            if (l == 0 || m < ms[k]) {
+                ms[k] = m;
+                of[k] = l;
+            }
+        }
     (void)hipStreamSynchronize(h->stream);
     if (rc) {  // keep the lattice the handle had
+        use_layout(h, lay[0]);
         h->lat[0] = old_lat[0];
         h->lat[1] = old_lat[1];
         imx::window_destroy(w);
@@ -1193,18 +1255,18 @@ int imexlb_tune_placement_window(imexlb_handle *h, int64_t slack_bytes, int64_t 
     int64_t best = 0;
     for (int64_t k = 1; k < npos; ++k)
         if (ms[k] < ms[best]) best = k;
-    h->lat[0] = (char *)big + best * step_bytes;
-    h->lat[1] = nlat == 2 ? (char *)h->lat[0] + lat_bytes : nullptr;
+    place(best, of[best]);
     if (!h->win.empty()) {
         h->device_bytes -= (int64_t)h->win.held();
         imx::window_destroy(h->win);
     } else {
-        h->device_bytes -= (int64_t)(nlat * lat_bytes);
+        h->device_bytes -= (int64_t)(nlat * h->lat_held);
         for (void *q : old_lat)
             if (q) hipFree(q);
     }
+    h->lat_held = h->lat_bytes;
     // the lattice stays on the pages it was timed on; the rest goes back
-    imx::window_keep(w, (size_t)(best * step_bytes), (size_t)nlat * lat_bytes);
+    imx::window_keep(w, (size_t)(best * step_bytes), (size_t)nlat * h->lat_bytes);
     h->device_bytes += (int64_t)w.held();
     h->win = std::move(w);
     if (ms_per_pos)

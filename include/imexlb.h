@@ -79,17 +79,22 @@ typedef struct imexlb_config {
     int32_t block;    /* threads per workgroup, 0 = default */
     int32_t cells_per_thread; /* 0 = default; 1, 2 (blockDim apart) or 3 (two
                                  adjacent x cells; periodic lattices with nx
-                                 even, one cell per thread elsewhere) */
+                                 even in arrays, see stride_pad; one cell per
+                                 thread elsewhere) */
     int32_t xcd_remap;        /* -1 = default, 0 off, 1 on */
     int32_t device;           /* HIP device ordinal */
-    int32_t stride_pad;       /* bytes added between populations, multiple of
-                                 256; -1 = default.  Keeps the 27 population
-                                 streams off a common power-of-two alignment */
+    int32_t stride_pad;       /* -1 = default.  With addr_mode -1 too: plane tiles
+                                 (each z plane a row of tiles, the 27 populations
+                                 of a tile together) for planes of 64 cells and
+                                 more.  Else one array per population with so
+                                 many bytes between them, a multiple of 256 */
     int32_t nt_loads;         /* -1 = default, 0/1: non-temporal loads of the
-                                 lines no other wavefront reads */
-    int32_t addr_mode;        /* fused kernels' addressing, the same results in
-                                 every mode: -1 = default (the most compact the
-                                 lattice allows), or at most 2 (a uniform base per
+                                 lines no other wavefront reads; in plane tiles 0
+                                 also makes the stores plain */
+    int32_t addr_mode;        /* fused kernels' addressing of arrays, the same
+                                 results in every mode: -1 = default (the most
+                                 compact the lattice allows; see stride_pad), or
+                                 at most 2 (a uniform base per
                                  group of populations; up to 2^28 cells per
                                  population), 1 (a base per population; up to
                                  4 GiB per population), 0 (64-bit offsets) */
@@ -271,9 +276,9 @@ int imexlb_tune_placement_window(imexlb_handle *h, int64_t slack_bytes, int64_t 
 
 /* ---- batched ensemble (no counterpart in the reference) ----------------
  * Many independent domains -- TGV boxes and config-mode cavities of uneven
- * size and Reynolds number -- advanced in lockstep by one persistent launch
- * per step over a table of tiles, optionally replayed from a captured HIP
- * graph.  Each member steps bit for bit as the fused engine steps it alone. */
+ * size and Reynolds number -- advanced in lockstep by one launch per step
+ * (one more per boundary kind for members with planes below 512 cells) over a
+ * table of tiles, optionally replayed from a captured HIP graph.  Each member steps bit for bit as the fused engine steps it alone. */
 typedef struct imexlb_domain {
     int32_t case_id;          /* IMEXLB_CASE_TGV or IMEXLB_CASE_CAVITY (config mode) */
     int32_t nx, ny, nz;
@@ -281,8 +286,8 @@ typedef struct imexlb_domain {
 } imexlb_domain;
 typedef struct imexlb_ensemble imexlb_ensemble;
 
-#define IMEXLB_ENS_PERSISTENT 0 /* one persistent launch per step */
-#define IMEXLB_ENS_GRAPH 1      /* persistent launches replayed from a HIP graph */
+#define IMEXLB_ENS_PERSISTENT 0 /* batched launches */
+#define IMEXLB_ENS_GRAPH 1      /* the same, replayed from a HIP graph */
 #define IMEXLB_ENS_PER_DOMAIN 2 /* one single-domain launch per domain per step */
 
 /* n domains drawn from seed: alternating TGV / cavity, edge in
@@ -307,8 +312,8 @@ int imexlb_ensemble_get_moments(imexlb_ensemble *e, int domain, double *p, doubl
 int imexlb_ensemble_status(imexlb_ensemble *e, int32_t *finite, int32_t *unstable);
 /* out[7]: cells, tiles, grid, block, cells per thread, device bytes, steps */
 int imexlb_ensemble_info(imexlb_ensemble *e, int64_t *out);
-/* grid: workgroups of each persistent launch (each walks every grid-th tile
- * of its run); 0 = one workgroup per tile. */
+/* grid: workgroups of each batched launch, which then walk every grid-th tile
+ * of its run; 0 (the default) = one workgroup per tile. */
 int imexlb_ensemble_set_launch(imexlb_ensemble *e, int block, int cells_per_thread, int grid);
 /* As imexlb_autotune, over block x cells per thread x grid (4 to 64
  * workgroups per CU, or one per tile), timed with graph replay; chosen[3] =

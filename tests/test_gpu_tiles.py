@@ -144,3 +144,28 @@ def test_plain_and_non_temporal_agree(n, dtype, storage, case, mode):
     for nt in (0, 1):
         same(state(n, 7, (64, 1, 1, nt), **kw), want, f"nt {nt}")
     same(state(n, 7, **kw), want, "default")
+
+
+# beyond the last-level cache a placement search times plane tiles and arrays
+@pytest.mark.parametrize("n,dtype,storage", [((96, 96, 90), "f64", "pull"), ((160, 128, 131), "f32", "aa")])
+def test_placement_searches_over_both_layouts_keep_results(n, dtype, storage):
+    from imexlb_amd import LBM
+    print(f"[case] searches {n} {dtype} {storage}", flush=True)
+    want = state(n, 7, dtype=dtype, storage=storage)
+    g = LBM(*n, 0.06, u0=0.05, dtype=dtype, storage=storage)
+    for search in (lambda: g.tune_placement_window(slack_gib=8 / 1024, step_gib=4 / 1024, steps=4),
+                   lambda: g.tune_placement(3, steps=4),
+                   lambda: g.tune_placement_window(slack_gib=4 / 1024, step_gib=4 / 1024, steps=4)):
+        kept, ms = search()
+        assert all(m > 0 for m in ms) and ms[kept] == min(ms)
+        g.Initialize()
+        g.step(7, 3)
+        same((g.get_f(), g.moments()), want, "after a search")
+    g.step(32, 32)  # a graph recorded on the kept layout
+    h = LBM(*n, 0.06, u0=0.05, dtype=dtype, storage=storage)
+    h.Initialize()
+    h.step(39, 39)
+    for a, b in zip(g.moments(), h.moments()):
+        assert np.array_equal(a, b)
+    g.close()
+    h.close()
