@@ -363,7 +363,7 @@ def main():
                      "traffic_source": traffic[2] if traffic else None,
                      "frac_of_measured_copy": achieved / gbps_copy,
                      "bytes_per_lup": bytes_lup, "launch": {k: info64[k] for k in ("block", "cells_per_thread", "xcd_remap", "nt_loads")},
-                     "kernel": "k_fused (FP64, periodic, "
+                     "kernel": "fused step: k_fused over arrays or k_tiled over plane tiles (FP64, periodic, "
                      + ("AA" if a.storage == "aa" else "pull") + ")",
                      "measured_copy_GBps": gbps_copy, "measured_copy_kernel": best_copy,
                      "bandwidth_probes_GBps": {k: round(v, 1) for k, v in probes.items()},
