@@ -325,8 +325,9 @@ __device__ __forceinline__ void tile_cells(const FusedParams &P, uint32_t z, uin
 
 // Before (structure of arrays, k_fused) and after, us per step, first
 // allocations: TGV 256^3 FP64 pull 1342 -> 1202 (6.03 TB/s algorithmic), 301x203x157
-// FP32 pull 414 -> 340, channel 512x256x256 FP16 712 -> 615, the reference's sphere
-// 512x128x128 715 -> 642 with its boundary kernels, cavity 128^3 FP64 AA 153 -> 136.
+// FP32 pull 414 -> 340, channel 512x256x256 FP16 712 -> 603, the reference's sphere
+// 512x128x128 715 -> 627 with its boundary launch, cavity 128^3 FP64 AA 153 -> 136, TGV 64^3
+// FP64 AA 21.0 -> 18.9.  NT: kernels.h tile_nt.
 template <typename S, int BC, int PAT, int CPT, bool NT>
 __global__ void __launch_bounds__(512) k_tiled(const FusedParams P)
 {
