@@ -55,8 +55,9 @@ __device__ __forceinline__ double get(const S *lat, const LatGeom &g, int slot, 
 // first Collision relaxes f0 towards the feq of the same fields, which is f0
 // itself, so f0 is also the first post-collision state.
 //
-// Bound by its stores.  Workgroups stay within a plane, so that their lines are
-// whole in a plane tile, and each XCD writes one run of the lattice.  us, cells in
+// Bound by its stores.  Over plane tiles workgroups stay within a plane, so that their
+// lines are whole in a tile; over arrays they follow the cells (init_block).  Each XCD
+// writes one run of the lattice.  us, cells in
 // storage order over the whole lattice / this: TGV 301x203x157 FP32 340 / 235, 256^3
 // FP64 832 / 675, 512^3 FP64 6700 / 5400, FP16 3590 / 2450, cavity 100^3 62 / 58;
 // non-temporal stores 198, 626, 5490, 2440, 68.  The solid cells of the other
@@ -66,11 +67,12 @@ template <typename S>
 __global__ void k_init(const InitParams P)
 {
     const uint32_t b = xcd_tile(blockIdx.x, gridDim.x);
-    const uint32_t z = P.divb.div(b), plane = (uint32_t)P.nx * P.ny;
-    const uint32_t pc = (b - z * P.bpp) * blockDim.x + threadIdx.x;
-    if (pc >= plane) return;
-    const uint32_t y = P.divx.div(pc), x = pc - y * P.nx;
-    const uint32_t c = z * plane + pc;
+    const uint32_t plane = (uint32_t)P.nx * P.ny, first = P.divb.div(b) * plane;  // (0 over arrays)
+    const uint32_t pc0 = (b - P.divb.div(b) * P.bpp) * blockDim.x + threadIdx.x;
+    const uint32_t c = first + pc0;
+    if (pc0 >= (P.geom.tl != 31 ? plane : P.ncell)) return;
+    const uint32_t row = P.divx.div(c), z = P.divy.div(row);
+    const uint32_t x = c - row * P.nx, y = row - z * P.ny, pc = c - z * plane;
     double u, v, w, p;
     if (P.kind == 0) {
         // tgv/src/lbm.cpp:197-204 with per-axis sin/cos tables
@@ -127,9 +129,10 @@ __global__ void k_init(const InitParams P)
 
 hipError_t launch_init(int dtype, InitParams P, hipStream_t st)
 {
-    P.bpp = ((uint32_t)P.nx * P.ny + 255) / 256;
+    const uint32_t plane = (uint32_t)P.nx * P.ny, block = init_block(P.geom, plane);
+    P.bpp = ((P.geom.tl != 31 ? plane : P.ncell) + block - 1) / block;
     P.divb.init(P.bpp);
-    dim3 blk(256), grid(P.bpp * (uint32_t)P.nz);
+    dim3 blk(block), grid(P.geom.tl != 31 ? P.bpp * (uint32_t)P.nz : P.bpp);
     if (dtype == DT_F64) hipLaunchKernelGGL(k_init<double>, grid, blk, 0, st, P);
     else if (dtype == DT_F32) hipLaunchKernelGGL(k_init<float>, grid, blk, 0, st, P);
     else hipLaunchKernelGGL(k_init<_Float16>, grid, blk, 0, st, P);

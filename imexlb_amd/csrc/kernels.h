@@ -373,6 +373,14 @@ struct InitParams {
     uint32_t bpp;            // workgroups of a plane (set by launch_init)
     FastDiv divb;
 };
+// Threads per workgroup of k_init: 256, over plane tiles no more than the plane's
+// wavefronts.  Threads then number less than twice the cells, below the 2^32
+// that HIP takes along one dimension of a launch (a subdomain has fewer than
+// 2^31 cells); whole workgroups of 256 for each plane reach it at 2^24 planes.
+inline uint32_t init_block(const LatGeom &g, uint32_t plane)
+{
+    return g.tl == 31 || plane > 192 ? 256u : (plane + 63) / 64 * 64;
+}
 hipError_t launch_init(int dtype, InitParams P, hipStream_t st);
 
 // Copy between the stored lattice (any dtype, pull or AA layout after step
