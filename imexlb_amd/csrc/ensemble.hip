@@ -289,13 +289,15 @@ static int launch_persistent(imexlb_ensemble *e, int pattern, int parity, bool w
     EP.write_moments = wm ? 1 : 0;
     EP.order = tile_order(lattice_bytes(e), e->storage == IMEXLB_AA);
     EP.nt = nt_of(e);
+    // HIP takes fewer than 2^32 work-items along one dimension of a launch
+    const int most = (int)(((uint64_t(1) << 32) - 1) / (uint64_t)e->block / 8 * 8);
     // the runs, back to back on the stream
     for (int r = 0; r < 3; ++r) {
         if (e->bounds[r + 1] == e->bounds[r]) continue;
         EP.t0 = e->bounds[r];
         EP.ntiles = e->bounds[r + 1];
         const int count = (int)(EP.ntiles - EP.t0);
-        const int grid = e->grid == 0 ? count : std::min<int>(e->grid, count);
+        const int grid = std::min(e->grid == 0 ? count : std::min<int>(e->grid, count), most);
         ECHK(e, launch_ensemble(e->dtype, e->cpt, r == 2 ? BC_CAVITY : BC_PERIODIC, r == 0, pattern, EP, grid, e->block,
                                 e->stream));
     }

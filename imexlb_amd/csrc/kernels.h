@@ -213,6 +213,16 @@ inline int tile_block(uint64_t plane, uint64_t cells, bool channel_f16)
     return best;
 }
 
+// Threads per workgroup that the plane-tile kernels run with for a requested
+// block: no more than the plane's wavefronts, since a workgroup stays within a plane.
+// Threads then number less than twice the cells, below the 2^32 that HIP takes
+// along one dimension of a launch (512 on planes of 64 cells: eight times).
+inline int tile_block_in_effect(uint64_t plane, int block)
+{
+    const uint64_t most = (plane + 63) / 64 * 64;
+    return (uint64_t)block > most ? (int)most : block;
+}
+
 // Rows per workgroup of the AA odd step's row kernel (tile.h k_tiled_rows)
 // for a requested block: as many whole rows as fit it, at least one; 0 where
 // the shifted form (k_tiled) serves better:

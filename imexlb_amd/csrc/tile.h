@@ -529,6 +529,8 @@ hipError_t launch_tiled(int bc, int pattern, const FusedParams &P0, int block, h
 {
     FusedParams P = P0;
     const uint64_t bytes = lattice_elems(P.geom, (uint32_t)P.nz) * sizeof(S);
+    const uint32_t plane = (uint32_t)P.nx * (uint32_t)P.ny;
+    block = tile_block_in_effect(plane, block);
     P.xcd_remap = P.xcd_remap ? tile_order(bytes, pattern != PAT_PULL) : 0;
     const uint32_t rows = tile_rows(P.nx, block, bytes, bc, sizeof(S));
     if (pattern == PAT_AA_ODD && rows > 0) {
@@ -548,7 +550,7 @@ hipError_t launch_tiled(int bc, int pattern, const FusedParams &P0, int block, h
         return hipGetLastError();
     }
     const int cpt = P.cpt == 2 ? 2 : 1;
-    const uint32_t plane = (uint32_t)P.nx * (uint32_t)P.ny, per = (uint32_t)block * (uint32_t)cpt;
+    const uint32_t per = (uint32_t)block * (uint32_t)cpt;
     P.bpp = (plane + per - 1) / per;
     P.divb.init(P.bpp);
     P.nblocks = P.bpp * (uint32_t)P.nz;

@@ -56,3 +56,42 @@ def test_initialize_of_long_thin_boxes(fake):
         assert "k_init" in name and grid * block < 2 * n[0] * n[1] * n[2] + 256, (n, grid, block)
         g.close()
     """)
+
+
+@pytest.mark.parametrize("shape", [(512, 1, 1, 1), (512, 2, 0, 0), (256, 1, 1, 0)])
+def test_wide_workgroups_on_small_planes(fake, shape):
+    """A workgroup as wide as the caller asks stays within its plane: what idles
+    doesn't count towards the 2^32 work-items that HIP takes."""
+    fake("""
+    shape = tuple(int(v) for v in sys.argv[2].split(","))
+    for n in [(8, 8, 1 << 23), (8, 8, 1 << 24), (10, 10, 21000000), (128, 2, 8388000)]:
+        g = LBM(*n, 0.1, dtype="f16", storage="aa")
+        g.set_launch(*shape)
+        g.Initialize()
+        launches()
+        g.step(2, 0)
+        for name, grid, block in launches():
+            assert grid * block < 2 * n[0] * n[1] * n[2] + 512, (n, name, grid, block)
+        g.close()
+    """, ",".join(map(str, shape)))
+
+
+def test_autotune_on_small_planes(fake):
+    fake("""
+    g = LBM(8, 8, 1 << 23, 0.1, dtype="f16", storage="aa")
+    g.autotune(steps=2)
+    """)
+
+
+def test_batched_launch_of_very_many_tiles(fake):
+    """Members whose tiles at one workgroup each exceed a launch: the grid stays
+    below it and walks them."""
+    fake("""
+    e = Ensemble([dict(case_id=0, nx=32, ny=17, nz=490000, tau0=0.1, rho0=1.0, u0=0.05, lid_u=0.0)] * 12,
+                 dtype="f16", storage="aa")
+    e.Initialize()
+    launches()
+    e.step(2, mode="persistent", moments_every=0)
+    got = launches()
+    assert len(got) == 2 and all(grid * block < 1 << 32 for _, grid, block in got), got
+    """)
