@@ -18,6 +18,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <mutex>
 #include <thread>
 #include <vector>
 
@@ -40,9 +41,11 @@ class ReadBack {
 
     // Copies the parts, ordered after the work queued on `st`, and returns when
     // all of them are in place.  A destination that the runtime knows (pinned,
-    // managed or device memory) is copied to directly.
+    // managed or device memory) is copied to directly.  Reads of several threads
+    // take turns: they share the slots (an uncontended lock costs some 20 ns).
     hipError_t copy(const Part *parts, int n, int device, hipStream_t st)
     {
+        std::lock_guard<std::mutex> turn(m_);
         size_t total = 0;
         bool plain = false;
         for (int k = 0; k < n; ++k) {
@@ -205,6 +208,7 @@ class ReadBack {
         return hipSuccess;
     }
 
+    std::mutex m_;
     char *pin_ = nullptr;  // at most SLOTS pieces of 2 MiB
     size_t cap_ = 0;
     hipEvent_t ev_[SLOTS] = {};

@@ -71,6 +71,15 @@ size_t fake_used() { return used; }
 size_t fake_most_pinned() { return most_pinned; }
 void fake_copy_delay(unsigned us) { copy_delay = us; }
 void fake_cost(const char *part, double ms) { costs.insert(costs.begin(), {part, ms}); }
+// every allocation of at most `bytes` holds a value of its own, in all its doubles
+void fake_paint(size_t bytes)
+{
+    std::lock_guard<std::mutex> l(m);
+    double v = 0;
+    for (auto &h : held)
+        if (++v, h.second <= bytes)
+            for (size_t k = 0; k < h.second / sizeof v; ++k) ((double *)h.first)[k] = v;
+}
 void fake_forget() { launches.clear(); }
 int fake_launches() { return (int)launches.size(); }
 const char *fake_name(int k) { return launches[k].name.c_str(); }

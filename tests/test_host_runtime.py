@@ -17,7 +17,7 @@ import ctypes, sys
 F = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
 F.fake_name.restype = ctypes.c_char_p
 F.fake_grid.restype = F.fake_block.restype = F.fake_used.restype = F.fake_most_pinned.restype = ctypes.c_size_t
-F.fake_room.argtypes = [ctypes.c_size_t]
+F.fake_room.argtypes = F.fake_paint.argtypes = [ctypes.c_size_t]
 F.fake_cost.argtypes = [ctypes.c_char_p, ctypes.c_double]
 import numpy as np
 from imexlb_amd import LBM, Ensemble
@@ -95,3 +95,41 @@ def test_batched_launch_of_very_many_tiles(fake):
     got = launches()
     assert len(got) == 2 and all(grid * block < 1 << 32 for _, grid, block in got), got
     """)
+
+
+@pytest.mark.parametrize("n", [(24, 20, 16), (80, 64, 64)])
+def test_reads_of_several_threads(fake, n):
+    """Threads that read fields of one handle at once, small and in pieces, each get
+    their own: a read only looks at the handle."""
+    fake("""
+    import threading
+    from imexlb_amd._lib import dptr, lib
+    n = tuple(int(v) for v in sys.argv[2].split(","))
+    g = LBM(*n, 0.1)
+    g.Initialize()
+    F.fake_paint(32 << 20)
+    F.fake_copy_delay(300)
+    want = [float(a.flat[0]) for a in g.moments()]
+    assert len(set(want)) == 4
+    none = ctypes.POINTER(ctypes.c_double)()
+    wrong = []
+
+    def read(k, rounds):
+        out = np.empty(g.shape)
+        for _ in range(rounds):
+            out[:] = -1
+            rc = lib().imexlb_get_moments(g.h, *[dptr(out) if i == k else none for i in range(4)])
+            if rc or (out != want[k]).any():
+                wrong.append(k)
+
+    def read_all():
+        if any((a != v).any() for a, v in zip(g.moments(), want)):
+            wrong.append("all")
+
+    ts = [threading.Thread(target=read, args=(k, 6)) for k in range(4)] + [threading.Thread(target=read_all) for _ in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not wrong, wrong
+    """, ",".join(map(str, n)))
