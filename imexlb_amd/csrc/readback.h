@@ -147,17 +147,18 @@ class ReadBack {
         // fields: 42 / 46 / 46 GB/s in 1 / 2 / 4 MiB pieces; the first read of a handle, which
         // allocates the slots, 256^3: 13.9 ms with 2 MiB, 16 with 4)
         const size_t piece = std::min(2 * MIB, std::max(MIB, (total / 32 + MIB - 1) / MIB * MIB));
-        if (!hold(piece * SLOTS)) return hipErrorNotReady;
-        for (hipEvent_t &e : ev_)
-            if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
-                (void)hipGetLastError();
-                return hipErrorNotReady;
-            }
         std::vector<Part> work;
         for (int k = 0; k < n; ++k)
             for (size_t o = 0; o < parts[k].bytes; o += piece)
                 work.push_back({(char *)parts[k].dst + o, (const char *)parts[k].src + o, std::min(piece, parts[k].bytes - o)});
-        const int pieces = (int)work.size();
+        const int pieces = (int)work.size(), slots = std::min(SLOTS, pieces);
+        // (pinning memory takes longer than copying into it: no slot that stays empty)
+        if (!hold(piece * (size_t)slots)) return hipErrorNotReady;
+        for (int k = 0; k < slots; ++k)
+            if (!ev_[k] && hipEventCreateWithFlags(&ev_[k], hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                return hipErrorNotReady;
+            }
         // wait for the steps here, not in every thread
         hipError_t e = hipStreamSynchronize(st);
         if (e != hipSuccess) return e;

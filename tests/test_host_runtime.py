@@ -133,3 +133,17 @@ def test_reads_of_several_threads(fake, n):
         t.join()
     assert not wrong, wrong
     """, ",".join(map(str, n)))
+
+
+@pytest.mark.parametrize("n,mib", [((16, 16, 16), 1), ((45, 37, 51), 4), ((64, 64, 64), 8), ((128, 128, 96), 24)])
+def test_a_read_pins_what_it_uses(fake, n, mib):
+    """The first read of a handle pins no more than its pieces, and at most 24 MiB."""
+    fake("""
+    n = tuple(int(v) for v in sys.argv[2].split(","))
+    g = LBM(*n, 0.1)
+    g.Initialize()
+    F.fake_paint(64 << 20)
+    for _ in range(2):
+        assert len({float(a.min()) for a in g.moments()} & {float(a.max()) for a in g.moments()}) == 4
+    assert F.fake_most_pinned() <= int(sys.argv[3]) << 20, F.fake_most_pinned()
+    """, ",".join(map(str, n)), mib)
