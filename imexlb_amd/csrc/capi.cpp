@@ -391,7 +391,11 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
     // plane tiles unless the caller asks for a stride or an address mode of the
     // structure of arrays (imexlb_config.stride_pad, addr_mode)
     h->geom = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
-    if (c.stride_pad < 0 && c.addr_mode < 0) tile_geom((uint32_t)c.nx, (uint32_t)c.ny, h->elem, c.storage == IMEXLB_AA, h->geom);
+    LatGeom tiles;
+    if (c.stride_pad < 0 && c.addr_mode < 0 &&
+        tile_geom((uint32_t)c.nx, (uint32_t)c.ny, h->elem, c.storage == IMEXLB_AA, tiles) &&
+        tiles_serve(tiles, (uint32_t)c.nx, (uint32_t)c.ny, (uint32_t)c.nz, h->elem, c.storage == IMEXLB_AA))
+        h->geom = tiles;
     h->block = c.block ? c.block : (h->geom.tl == 31 ? 256 : tile_block((uint64_t)c.nx * c.ny, h->ncell,
                                                                               c.case_id == IMEXLB_CASE_SPHERE && c.dtype == IMEXLB_F16));
     h->cpt = c.cells_per_thread ? c.cells_per_thread : 1;

@@ -134,20 +134,21 @@ inline uint64_t lattice_elems(const LatGeom &g, uint32_t nz)
     return g.tl == 31 ? (uint64_t)Q * g.is : (uint64_t)nz * g.zs;
 }
 
-// Plane tiles for a lattice, where they serve: the largest tile of at most
-// 32 KiB per population (at least 64 cells) whose last tile leaves at most a
-// sixteenth of the plane unused.  Not for planes below 64 cells, whose wavefronts
-// would be mostly idle (a workgroup never spans two planes), nor where three
-// planes exceed the 4 GiB that the kernels' 32-bit offsets reach.  us per step, arrays /
-// tiles: TGV 8^3 FP64 5.6 / 4.1, 16^3 5.86 / 4.17, FP32 4.12 / 3.19, FP16 AA 3.88 / 3.15, 9x13x30 FP64
-// 5.88 / 4.15, 22x18x22 6.03 / 4.32, faithful cavity 16^3 10.1 / 8.8, 12x12x3000 FP64 41.7 / 28.7 (but
-// 16x16x400 FP64 pull 9.5 / 9.9 and FP16 AA 12x12x3000 10.5 / 11.1).
+// Plane tiles for a lattice: the largest tile, of 128 bytes (a line) to 32 KiB per
+// population, whose last one leaves at most a sixteenth of the plane unused, else
+// tiles of a line.  Not for planes below 64 cells, whose wavefronts would be mostly
+// idle (a workgroup never spans two planes), nor where three planes exceed the 4 GiB
+// that the kernels' 32-bit offsets reach.  Tiles of a line instead of 64 cells take
+// a quarter (FP64) and a sixth (FP32) of the memory off planes of 10x13 and are as fast or
+// faster: us per step, 64 cells / a line, 12x12x69444 FP64 pull 751 / 731, FP32 AA 440 / 428, 12x12x13889
+// FP32 AA 83.6 / 64.0 (the lattice then fits the last-level cache).
 inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, bool aa, LatGeom &g)
 {
     const uint64_t plane = (uint64_t)nx * ny;
     if (plane < 64) return false;
-    uint32_t tl = 6;
-    for (uint32_t t = 6; (elem << t) <= 32768; ++t) {
+    const uint32_t line = elem == 8 ? 4 : elem == 4 ? 5 : 6;
+    uint32_t tl = line;
+    for (uint32_t t = line; (elem << t) <= 32768; ++t) {
         const uint64_t n = ((plane - 1) >> t) + 1;
         if (((n << t) - plane) * 16 <= plane) tl = t;
     }
@@ -158,11 +159,40 @@ inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, bool aa, LatGeom 
     return true;
 }
 
+// Whether a lattice that tile_geom lays out in tiles is better off in them than in
+// arrays.  A plane in tiles starts on a line and in a wavefront of its own, so
+// what its last line and its last wavefront hold beyond it is spent; arrays run
+// through the planes.  us per step, arrays / tiles:
+// - beyond the last-level cache the lines count.  Tiles of whole lines gain 9-10 %,
+//   so a twelfth of a plane is the most to spend: of 1e7 cells, 16x16 FP16 pull (none)
+//   231 / 213, 30x20 (a fifteenth) 221 / 214, 20x20 (an eighth) 209 / 223, 19x17 (a fifth)
+//   213 / 242, 10x13 (half) 239 / 304, 13x5 (all) 243 / 421, 12x12 FP64 (none) 850 / 731;
+// - in it tiles gain more, a fifth to a half: 2e6 cells FP16 pull 216 MB, 19x17 (a fifth)
+//   48.0 / 36.7, 12x12 (a third) 49.6 / 53.2, 9x8 (three quarters) 50.8 / 65.4; 4e5
+//   cells FP32 pull 86 MB, 9x8 (a third) 20.9 / 16.6, 10x13 (a quarter) 20.7 / 16.0;
+// - in the L2s (32 MB) the wavefronts count: none while each has a SIMD of its own
+//   (13x5x308 FP32 pull 4.23 / 3.97, 9x8x278 FP64 pull 6.22 / 6.21), few while all of
+//   them are resident, four to a SIMD (12x12x694 FP32 pull 6.31 / 5.41, 10x13x769 FP32 AA
+//   5.76 / 5.79, 9x8x1389 FP16 AA 4.97 / 6.01), more beyond (FP16 AA of 4e5 cells: 16x16
+//   10.2 / 10.0, 12x12 10.3 / 10.6, 10x13 10.5 / 11.7, 9x8 10.6 / 14.0).
+// At other sizes tiles serve: TGV 8^3 FP64 5.6 / 4.1, 16^3 5.86 / 4.17, FP32 4.12 / 3.19, FP16 AA
+// 3.88 / 3.15, 9x13x30 FP64 5.88 / 4.15, 22x18x22 6.03 / 4.32, faithful cavity 16^3 10.1 / 8.8.
+constexpr uint64_t LAST_LEVEL = uint64_t(256) << 20;
+inline bool tiles_serve(const LatGeom &g, uint32_t nx, uint32_t ny, uint32_t nz, uint64_t elem, bool aa)
+{
+    const uint64_t plane = (uint64_t)nx * ny, bytes = lattice_elems(g, nz) * elem * (aa ? 1 : 2);
+    const uint64_t spent = (plane * elem + 127) / 128 * 128 - plane * elem;
+    if (bytes > LAST_LEVEL) return spent * 12 <= plane * elem;
+    if (bytes > LAST_LEVEL / 2) return spent * 4 <= plane * elem;
+    const uint64_t waves = (plane + 63) / 64, idle = waves * 64 - plane, mib = uint64_t(1) << 20;
+    if (bytes > 32 * mib) return spent * 2 <= plane * elem && (bytes > 48 * mib || idle * 2 <= plane);
+    return waves * nz <= 1024 || idle * (waves * nz <= 4096 ? 2 : 4) <= plane;
+}
+
 // The XCD-aware order of the plane-tile kernels (tile.h tile_block_of, with the
 // measurements): one run of the lattice per XCD (1) where the lattices of a
 // step fit the 256 MB last-level cache, else runs of eight workgroups.
 constexpr int XCD_RUNS = 2;
-constexpr uint64_t LAST_LEVEL = uint64_t(256) << 20;
 inline int tile_order(uint64_t lattice_bytes, bool aa)
 {
     return (aa ? lattice_bytes : 2 * lattice_bytes) <= LAST_LEVEL ? 1 : XCD_RUNS;

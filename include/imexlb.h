@@ -85,8 +85,8 @@ typedef struct imexlb_config {
     int32_t device;           /* HIP device ordinal */
     int32_t stride_pad;       /* -1 = default.  With addr_mode -1 too: plane tiles
                                  (each z plane a row of tiles, the 27 populations
-                                 of a tile together) for planes of 64 cells and
-                                 more.  Else one array per population with so
+                                 of a tile together) where they serve: mostly,
+                                 for planes of 64 cells and more.  Else one array per population with so
                                  many bytes between them, a multiple of 256 */
     int32_t nt_loads;         /* -1 = default, 0/1: non-temporal loads of the
                                  lines no other wavefront reads; in plane tiles 0

@@ -147,3 +147,20 @@ def test_a_read_pins_what_it_uses(fake, n, mib):
         assert len({float(a.min()) for a in g.moments()} & {float(a.max()) for a in g.moments()}) == 4
     assert F.fake_most_pinned() <= int(sys.argv[3]) << 20, F.fake_most_pinned()
     """, ",".join(map(str, n)), mib)
+
+
+@pytest.mark.parametrize("n", [(13, 5, 153846), (9, 8, 138889), (10, 13, 76923), (12, 12, 69444), (23, 23, 18904)])
+@pytest.mark.parametrize("dtype,storage", [("f64", "pull"), ("f32", "aa"), ("f16", "pull")])
+def test_memory_of_boxes_of_small_planes(fake, n, dtype, storage):
+    """The default layout of a large box holds at most a twelfth more than arrays."""
+    fake("""
+    n = tuple(int(v) for v in sys.argv[2].split(","))
+    used = []
+    for am in (2, -1):
+        g = LBM(*n, 0.1, dtype=sys.argv[3], storage=sys.argv[4], addr_mode=am)
+        used.append(F.fake_used())
+        assert g.info()["device_bytes"] <= used[-1]
+        g.close()
+        assert F.fake_used() == 0
+    assert used[1] <= used[0] * 13 / 12, used
+    """, ",".join(map(str, n)), dtype, storage)
