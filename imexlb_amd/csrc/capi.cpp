@@ -341,6 +341,62 @@ static int ensure_graph(imexlb_handle *h)
     return IMEXLB_OK;
 }
 
+// A fused handle's device memory, in its layout.  On failure release() gives back what
+// there is.
+static int allocate(imexlb_handle *h)
+{
+    const imexlb_config &c = h->cfg;
+    const char *what = "";
+    auto take = [&](auto **p, size_t bytes, const char *name, bool counted) {
+        what = name;
+        if (hipMalloc((void **)p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            *p = nullptr;
+            return false;
+        }
+        if (counted) h->device_bytes += (int64_t)bytes;
+        return true;
+    };
+    const int nlat = c.storage == IMEXLB_PULL ? 2 : 1;
+    h->lat_held = h->lat_bytes = (size_t)(lattice_elems(h->geom, (uint32_t)c.nz) * h->elem);
+    bool ok = true;
+    for (int k = 0; k < nlat && ok; ++k)
+        if (!(ok = take(&h->lat[k], h->lat_bytes, "", true))) return fail(h, IMEXLB_ENOMEM, "lattice of %zu bytes", h->lat_bytes);
+    for (double *&p : h->mom) ok = ok && take(&p, (size_t)h->ncell * 8, "moments", true);
+    ok = ok && take(&h->partials, sizeof(double) * 4 * h->nparts, "reduction scratch", false) &&
+         take(&h->result, sizeof(double) * 4, "reduction scratch", false);
+    if (bc_of(c) == BC_FAITHFUL) {
+        h->ring_a = (uint32_t)(c.ny + 2) * (uint32_t)(c.nz + 2);
+        h->ring_b = (uint32_t)c.nx * (uint32_t)(c.nz + 2);
+        h->ring_c = (uint32_t)c.nx * (uint32_t)c.ny;
+        for (double *&p : h->ring)
+            ok = ok && take(&p, (size_t)Q * 2 * (h->ring_a + h->ring_b + h->ring_c) * 8, "ghost ring", true);
+        ok = ok && take(&h->stage, (size_t)2 * STAGE_ROW * c.ny * c.nz * 8, "x-face stage", true);
+    }
+    if (c.case_id == IMEXLB_CASE_SPHERE) ok = ok && take(&h->mask, h->ncell, "mask", true);
+    if (c.case_id == IMEXLB_CASE_TGV) ok = ok && take(&h->tgv_tab, 3 * ((size_t)c.nx + c.ny + c.nz) * 8, "tables", false);
+    return ok ? IMEXLB_OK : fail(h, IMEXLB_ENOMEM, "%s", what);
+}
+
+static void release(imexlb_handle *h)
+{
+    auto give = [](auto *&p) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+    };
+    if (!h->win.empty()) imx::window_destroy(h->win);
+    else
+        for (auto &p : h->lat) give(p);
+    for (auto &p : h->mom) give(p);
+    for (auto &p : h->ring) give(p);
+    give(h->mask);
+    give(h->partials);
+    give(h->result);
+    give(h->tgv_tab);
+    give(h->stage);
+    h->device_bytes = 0;
+}
+
 extern "C" {
 
 int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
@@ -408,53 +464,20 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
         if (c.case_id == IMEXLB_CASE_SPHERE && c.mode == IMEXLB_MODE_CONFIG) h->ush = c.u0;
         storage_shift(h->shift, h->ush, h->sh);
     }
-    const int nlat = c.storage == IMEXLB_PULL ? 2 : 1;
-    auto alloc_lattices = [&]() {
-        h->lat_bytes = (size_t)(lattice_elems(h->geom, (uint32_t)c.nz) * h->elem);
-        for (int k = 0; k < nlat; ++k)
-            if (hipMalloc(&h->lat[k], h->lat_bytes) != hipSuccess) {
-                (void)hipGetLastError();
-                for (auto &p : h->lat)
-                    if (p) hipFree(p);
-                h->lat[0] = h->lat[1] = nullptr;
-                return false;
-            }
-        return true;
-    };
-    bool have = alloc_lattices();
-    if (!have && h->geom.tl != 31) {  // tiles round the planes up: arrays may still fit
+    if (h->geom.tl != 31 && c.nt_loads < 0)
+        h->ntl = tile_nt(lattice_elems(h->geom, (uint32_t)c.nz) * h->elem, c.storage == IMEXLB_AA, h->elem) ? 1 : 0;
+    rc = allocate(h);
+    if (rc == IMEXLB_ENOMEM && h->geom.tl != 31) {  // tiles round the planes up: arrays may still fit
+        release(h);
         h->geom = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
         h->block = c.block ? c.block : 256;
-        have = alloc_lattices();
+        h->ntl = c.nt_loads < 0 ? 1 : (c.nt_loads ? 1 : 0);
+        rc = allocate(h);
     }
-    if (c.nt_loads < 0 && h->geom.tl != 31)
-        h->ntl = tile_nt(h->lat_bytes, c.storage == IMEXLB_AA, h->elem) ? 1 : 0;
-    if (!have) return bail(fail(h, IMEXLB_ENOMEM, "lattice of %zu bytes", h->lat_bytes));
-    h->lat_held = h->lat_bytes;
-    h->device_bytes += (int64_t)nlat * (int64_t)h->lat_bytes;
-    for (int k = 0; k < 4; ++k) {
-        if (hipMalloc(&h->mom[k], (size_t)h->ncell * 8) != hipSuccess)
-            return bail(fail(h, IMEXLB_ENOMEM, "moments"));
-        h->device_bytes += (int64_t)h->ncell * 8;
-        if (hipMemsetAsync(h->mom[k], 0, (size_t)h->ncell * 8, h->stream) != hipSuccess)
+    if (rc) return bail(rc);
+    for (double *p : h->mom)
+        if (hipMemsetAsync(p, 0, (size_t)h->ncell * 8, h->stream) != hipSuccess)
             return bail(fail(h, IMEXLB_EHIP, "memset"));
-    }
-    if (hipMalloc(&h->partials, sizeof(double) * 4 * h->nparts) != hipSuccess ||
-        hipMalloc(&h->result, sizeof(double) * 4) != hipSuccess)
-        return bail(fail(h, IMEXLB_ENOMEM, "reduction scratch"));
-    if (bc_of(c) == BC_FAITHFUL) {
-        h->ring_a = (uint32_t)(c.ny + 2) * (uint32_t)(c.nz + 2);
-        h->ring_b = (uint32_t)c.nx * (uint32_t)(c.nz + 2);
-        h->ring_c = (uint32_t)c.nx * (uint32_t)c.ny;
-        const size_t rb = (size_t)Q * 2 * (h->ring_a + h->ring_b + h->ring_c) * 8;
-        for (auto &p : h->ring) {
-            if (hipMalloc(&p, rb) != hipSuccess) return bail(fail(h, IMEXLB_ENOMEM, "ghost ring"));
-            h->device_bytes += (int64_t)rb;
-        }
-        const size_t sb = (size_t)2 * STAGE_ROW * c.ny * c.nz * 8;
-        if (hipMalloc(&h->stage, sb) != hipSuccess) return bail(fail(h, IMEXLB_ENOMEM, "x-face stage"));
-        h->device_bytes += (int64_t)sb;
-    }
 
     // boundary constants in the oracle's operation order
     const double cs2 = 1.0 / 3.0;
@@ -468,8 +491,6 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
             for (int y = 0; y < c.ny; ++y)
                 for (int x = 0; x < c.nx; ++x)
                     if (faithful_sphere_solid(c.nx, x, y, z)) m[((size_t)z * c.ny + y) * c.nx + x] = 1;
-        if (hipMalloc(&h->mask, h->ncell) != hipSuccess) return bail(fail(h, IMEXLB_ENOMEM, "mask"));
-        h->device_bytes += h->ncell;
         if (hipMemcpy(h->mask, m.data(), h->ncell, hipMemcpyHostToDevice) != hipSuccess)
             return bail(fail(h, IMEXLB_EHIP, "mask upload"));
     } else if (c.case_id == IMEXLB_CASE_SPHERE) {
@@ -513,8 +534,6 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
                         }
                     }
                 }
-        if (hipMalloc(&h->mask, h->ncell) != hipSuccess) return bail(fail(h, IMEXLB_ENOMEM, "mask"));
-        h->device_bytes += h->ncell;
         if (hipMemcpy(h->mask, m.data(), h->ncell, hipMemcpyHostToDevice) != hipSuccess)
             return bail(fail(h, IMEXLB_EHIP, "mask upload"));
     }
@@ -530,7 +549,6 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
             for (int k = 0; k < n; ++k) tab[o + 2 * n + k] = std::cos((double)k / (double)n * 2.0 * PI_REF * 2.0);
             o += 3 * (size_t)n;
         }
-        if (hipMalloc(&h->tgv_tab, tab.size() * 8) != hipSuccess) return bail(fail(h, IMEXLB_ENOMEM, "tables"));
         if (hipMemcpy(h->tgv_tab, tab.data(), tab.size() * 8, hipMemcpyHostToDevice) != hipSuccess)
             return bail(fail(h, IMEXLB_EHIP, "table upload"));
     }
@@ -544,19 +562,7 @@ int imexlb_destroy(imexlb_handle *h)
     if (!h) return IMEXLB_OK;
     hipSetDevice(h->device);
     if (h->stream) hipStreamSynchronize(h->stream);
-    if (!h->win.empty()) imx::window_destroy(h->win);
-    else
-        for (auto &p : h->lat)
-            if (p) hipFree(p);
-    for (auto &p : h->mom)
-        if (p) hipFree(p);
-    if (h->mask) hipFree(h->mask);
-    if (h->partials) hipFree(h->partials);
-    if (h->result) hipFree(h->result);
-    if (h->tgv_tab) hipFree(h->tgv_tab);
-    for (auto &p : h->ring)
-        if (p) hipFree(p);
-    if (h->stage) hipFree(h->stage);
+    release(h);
     if (h->ph) phased_destroy(h->ph);
     if (h->gexec) hipGraphExecDestroy(h->gexec);
     if (h->stream && h->own_stream) hipStreamDestroy(h->stream);

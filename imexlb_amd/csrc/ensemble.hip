@@ -444,7 +444,8 @@ int imexlb_ensemble_create(const imexlb_domain *doms, int n, int dtype, int stor
     const int nl = storage == IMEXLB_PULL ? 2 : 1;
     std::vector<uint64_t> pstride(n);
     std::vector<LatGeom> geom(n);
-    auto alloc_pool = [&](bool tiles) {
+    e->mom.assign(4 * (size_t)n, nullptr);
+    auto alloc = [&](bool tiles) {  // the pool and the members' fields
         e->pool_bytes = 0;
         for (int d = 0; d < n; ++d) {
             geom[d] = soa_geom((uint32_t)doms[d].nx, (uint32_t)doms[d].ny, pstride[d]);
@@ -456,9 +457,21 @@ int imexlb_ensemble_create(const imexlb_domain *doms, int n, int dtype, int stor
                 e->pool_bytes += ((size_t)lattice_elems(geom[d], (uint32_t)doms[d].nz) * elem + 4095) / 4096 * 4096;
             }
         }
-        if (hipMalloc(&e->pool, e->pool_bytes) == hipSuccess) return true;
+        bool ok = hipMalloc(&e->pool, e->pool_bytes) == hipSuccess;
+        if (!ok) e->pool = nullptr;
+        for (size_t k = 0; k < e->mom.size() && ok; ++k) {
+            const imexlb_domain &D = doms[k / 4];
+            ok = hipMalloc(&e->mom[k], (size_t)D.nx * D.ny * D.nz * 8) == hipSuccess;
+            if (!ok) e->mom[k] = nullptr;
+        }
+        if (ok) return true;
         (void)hipGetLastError();
+        if (e->pool) (void)hipFree(e->pool);
         e->pool = nullptr;
+        for (double *&p : e->mom) {
+            if (p) (void)hipFree(p);
+            p = nullptr;
+        }
         return false;
     };
     for (int d = 0; d < n; ++d) {
@@ -468,20 +481,16 @@ int imexlb_ensemble_create(const imexlb_domain *doms, int n, int dtype, int stor
         // stride per cell, PopGroup) with 32-bit byte offsets
         if (pstride[d] * 16 > (1ull << 32)) return bail(IMEXLB_EINVAL);
     }
-    if (!alloc_pool(true) && !alloc_pool(false)) return bail(IMEXLB_ENOMEM);
+    if (!alloc(true) && !alloc(false)) return bail(IMEXLB_ENOMEM);
     e->device_bytes += (int64_t)e->pool_bytes;
     for (int d = 0; d < n; ++d)
         for (int k = 0; k < nl; ++k) e->lat[2 * d + k] = (char *)e->pool + e->lat_off[2 * d + k];
-    e->mom.assign(4 * (size_t)n, nullptr);
     e->tabs.assign((size_t)n, nullptr);
     for (int d = 0; d < n; ++d) {
         const imexlb_domain &D = doms[d];
         const uint32_t nc = (uint32_t)((uint64_t)D.nx * D.ny * D.nz);
         e->cells += nc;
-        for (int k = 0; k < 4; ++k) {
-            if (hipMalloc(&e->mom[4 * d + k], (size_t)nc * 8) != hipSuccess) return bail(IMEXLB_ENOMEM);
-            e->device_bytes += (int64_t)nc * 8;
-        }
+        e->device_bytes += 4 * (int64_t)nc * 8;
         for (int par = 0; par < 2; ++par) {
             FusedParams &P = e->hp[2 * d + par];
             std::memset(&P, 0, sizeof P);

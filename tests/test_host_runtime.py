@@ -164,3 +164,69 @@ def test_memory_of_boxes_of_small_planes(fake, n, dtype, storage):
         assert F.fake_used() == 0
     assert used[1] <= used[0] * 13 / 12, used
     """, ",".join(map(str, n)), dtype, storage)
+
+
+# (case, mode, more): every allocation that follows the lattices
+LATER = [("tgv", "faithful", "{}"), ("cavity", "faithful", "{}"), ("sphere", "faithful", "{}"),
+         ("sphere", "config", "dict(sphere=(30.0, 20.0, 20.0, 5.0))")]
+
+
+@pytest.mark.parametrize("case,mode,more", LATER)
+def test_arrays_where_only_they_fit(fake, case, mode, more):
+    """A box whose arrays fit in the memory there is, and whose tiles do not, runs in
+    arrays, whichever allocation is the one that fails; a box that fits neither way is
+    refused and leaves nothing behind."""
+    fake("""
+    from imexlb_amd import ImexlbError
+    kw = dict(case=sys.argv[2], mode=sys.argv[3], **eval(sys.argv[4]))
+    n = (97, 41, 50)  # 3977 cells a plane: tiles hold 4096
+    used = {}
+    for am in (2, -1):
+        g = LBM(*n, 0.1, addr_mode=am, **kw)
+        used[am] = F.fake_used(), g.info()["device_bytes"]
+        g.close()
+    assert used[-1][0] > used[2][0] * 1.02
+    for room in np.linspace(used[2][0], used[-1][0], 40):
+        F.fake_room(int(room))
+        g = LBM(*n, 0.1, **kw)
+        assert g.info()["device_bytes"] == used[-1 if int(room) == used[-1][0] else 2][1]
+        g.Initialize()
+        g.step(2)
+        g.close()
+        assert F.fake_used() == 0
+    for room in np.linspace(0, used[2][0] - 1, 40):
+        F.fake_room(int(room))
+        try:
+            LBM(*n, 0.1, **kw)
+            assert False, room
+        except ImexlbError as e:
+            assert e.status == -3, e
+        assert F.fake_used() == 0
+    """, case, mode, more)
+
+
+def test_ensemble_in_arrays_where_only_they_fit(fake):
+    fake("""
+    from imexlb_amd import ImexlbError
+    doms = [dict(case_id=k % 2, nx=97, ny=41, nz=20 + k, tau0=0.1, rho0=1.0, u0=0.05, lid_u=0.1) for k in range(3)]
+    cells = sum(d["nx"] * d["ny"] * d["nz"] for d in doms)
+    arrays = cells * (2 * 27 + 4) * 8 + (1 << 20)
+    e = Ensemble(doms, dtype="f64")
+    tiles = F.fake_used()
+    e.close()
+    assert F.fake_used() == 0 and tiles > arrays, (F.fake_used(), tiles, arrays)
+    for room in np.linspace(arrays, tiles, 30):
+        F.fake_room(int(room))
+        e = Ensemble(doms, dtype="f64")
+        e.Initialize()
+        e.step(2)
+        e.close()
+        assert F.fake_used() == 0
+    F.fake_room(cells * 58 * 8)
+    try:
+        Ensemble(doms, dtype="f64")
+        assert False
+    except ImexlbError:
+        pass
+    assert F.fake_used() == 0
+    """)
