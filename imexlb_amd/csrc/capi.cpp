@@ -1009,7 +1009,8 @@ int imexlb_autotune(imexlb_handle *h, const char *cache_path, int steps, int32_t
     if (rc) return rc;
     const imexlb_config &c = h->cfg;
     char shape[96];
-    snprintf(shape, sizeof shape, "bc%d_%dx%dx%d", bc_of(c), c.nx, c.ny, c.nz);
+    // the two layouts run different kernels, whose shapes mean different things
+    snprintf(shape, sizeof shape, "bc%d_%dx%dx%d_%s", bc_of(c), c.nx, c.ny, c.nz, layout_name(h->geom));
     const std::string key = tune_key(h->device, "single", c.dtype, c.storage, shape);
     TuneChoice best{};
     if (!tune_cache_read(cache_path, key, best)) {

@@ -886,7 +886,10 @@ int imexlb_ensemble_autotune(imexlb_ensemble *e, const char *cache_path, int ste
     if (!e) return IMEXLB_EINVAL;
     ECHK(e, hipSetDevice(e->device));
     std::ostringstream shape;
-    shape << "ens" << e->n << "_cells" << e->cells;
+    // members in plane tiles run another kernel than those in arrays
+    int tiled = 0;
+    for (int d = 0; d < e->n; ++d) tiled += run_of(e->hp[2 * d]) == 0 ? 1 : 0;
+    shape << "ens" << e->n << "_cells" << e->cells << "_tiles" << tiled;
     const std::string key = tune_key(e->device, "ensemble", e->dtype, e->storage, shape.str());
     TuneChoice best{};
     if (!tune_cache_read(cache_path, key, best)) {

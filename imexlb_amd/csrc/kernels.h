@@ -128,6 +128,9 @@ inline LatGeom soa_geom(uint32_t nx, uint32_t ny, uint64_t pstride)
     return LatGeom{(uint64_t)nx * ny, pstride, 0, 31, 0};
 }
 
+// The layout in a tuner's cache key.
+inline const char *layout_name(const LatGeom &g) { return g.tl == 31 ? "arrays" : "tiles"; }
+
 // Elements of a lattice of nz planes.
 inline uint64_t lattice_elems(const LatGeom &g, uint32_t nz)
 {

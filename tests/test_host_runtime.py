@@ -230,3 +230,53 @@ def test_ensemble_in_arrays_where_only_they_fit(fake):
         pass
     assert F.fake_used() == 0
     """)
+
+
+def test_tuned_shapes_are_kept_by_layout(fake, tmp_path):
+    """A cached launch shape serves handles of the layout it was timed on: not the
+    other layout, and no line that names none is taken."""
+    fake("""
+    cache = sys.argv[2]
+
+    def tune(am, **kw):
+        g = LBM(66, 40, 30, 0.1, addr_mode=am, **kw)
+        launches()
+        c = g.autotune(cache, steps=2)
+        timed = any("k_fused" in name or "k_tiled" in name for name, _, _ in launches())
+        g.close()
+        return c, timed
+
+    F.fake_cost(b"k_fused_pair", 1e-3)  # two adjacent cells: faster, in arrays only
+    F.fake_cost(b"k_init", 0.0)
+    for p in (b"k_fusedI", b"k_tiled"):
+        F.fake_cost(p, 2e-3)
+    arrays, timed = tune(2)
+    assert timed and arrays[1] == 3, arrays
+    tiles, timed = tune(-1)
+    assert timed and tiles[1] != 3, tiles
+    assert tune(2) == (arrays, False) and tune(-1) == (tiles, False)
+    keys = [line.split('"')[3] for line in open(cache)]
+    assert len(set(keys)) == 2
+    # lines of before, which say nothing of the layout
+    with open(cache, "w") as f:
+        for k in keys:
+            f.write('{"key": "%s", "block": 448, "cpt": 1, "third": 0, "ntl": 0, "ms": 0.1}' % k.rsplit("_", 1)[0] + chr(10))
+    for am in (2, -1):
+        c, timed = tune(am)
+        assert timed and c[0] != 448, c
+    """, tmp_path / "cache.jsonl")
+
+
+def test_tuned_ensemble_shapes_are_kept_by_layout(fake, tmp_path):
+    """Two ensembles of equal counts, one of members in tiles and one in arrays."""
+    fake("""
+    cache = sys.argv[2]
+    for nx, ny, nz in ((32, 32, 16), (16, 16, 64)):
+        e = Ensemble([dict(case_id=0, nx=nx, ny=ny, nz=nz, tau0=0.1, rho0=1.0, u0=0.05, lid_u=0.1)] * 2)
+        e.Initialize()
+        for again in (False, True):
+            launches()
+            e.autotune(cache, steps=2)
+            assert any("k_ensemble" in name for name, _, _ in launches()) != again
+        e.close()
+    """, tmp_path / "cache.jsonl")
