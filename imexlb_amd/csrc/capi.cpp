@@ -341,6 +341,15 @@ static int ensure_graph(imexlb_handle *h)
     return IMEXLB_OK;
 }
 
+// Threads per workgroup of a layout where set_launch and the tuners name none.
+static int default_block(const imexlb_handle *h, const LatGeom &g)
+{
+    const imexlb_config &c = h->cfg;
+    if (c.block) return c.block;
+    if (g.tl == 31) return 256;
+    return tile_block((uint64_t)c.nx * c.ny, h->ncell, c.case_id == IMEXLB_CASE_SPHERE && c.dtype == IMEXLB_F16);
+}
+
 // A fused handle's device memory, in its layout.  On failure release() gives back what
 // there is.
 static int allocate(imexlb_handle *h)
@@ -452,8 +461,7 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
         tile_geom((uint32_t)c.nx, (uint32_t)c.ny, h->elem, c.storage == IMEXLB_AA, tiles) &&
         tiles_serve(tiles, (uint32_t)c.nx, (uint32_t)c.ny, (uint32_t)c.nz, h->elem, c.storage == IMEXLB_AA))
         h->geom = tiles;
-    h->block = c.block ? c.block : (h->geom.tl == 31 ? 256 : tile_block((uint64_t)c.nx * c.ny, h->ncell,
-                                                                              c.case_id == IMEXLB_CASE_SPHERE && c.dtype == IMEXLB_F16));
+    h->block = default_block(h, h->geom);
     h->cpt = c.cells_per_thread ? c.cells_per_thread : 1;
     h->xcd = c.xcd_remap < 0 ? 1 : c.xcd_remap;
     h->ntl = c.nt_loads < 0 ? 1 : (c.nt_loads ? 1 : 0);
@@ -470,7 +478,7 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
     if (rc == IMEXLB_ENOMEM && h->geom.tl != 31) {  // tiles round the planes up: arrays may still fit
         release(h);
         h->geom = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
-        h->block = c.block ? c.block : 256;
+        h->block = default_block(h, h->geom);
         h->ntl = c.nt_loads < 0 ? 1 : (c.nt_loads ? 1 : 0);
         rc = allocate(h);
     }
@@ -1027,7 +1035,10 @@ int imexlb_autotune(imexlb_handle *h, const char *cache_path, int steps, int32_t
             return r;
         };
         std::vector<TuneChoice> cand;
-        const int blocks[4] = {64, 128, 256, 512};
+        // the untuned shape is one of the candidates: no tuned handle is slower
+        std::vector<int> blocks{64, 128, 256, 512};
+        if (const int own = default_block(h, h->geom); std::find(blocks.begin(), blocks.end(), own) == blocks.end())
+            blocks.push_back(own);
         // cell pairs (3) only where their kernel runs (periodic, nx even,
         // grouped bases: address mode 2); elsewhere they would time the
         // one-cell kernel again

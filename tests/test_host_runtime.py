@@ -280,3 +280,26 @@ def test_tuned_ensemble_shapes_are_kept_by_layout(fake, tmp_path):
             assert any("k_ensemble" in name for name, _, _ in launches()) != again
         e.close()
     """, tmp_path / "cache.jsonl")
+
+
+@pytest.mark.parametrize("n,kw,block", [
+    ((512, 256, 256), dict(case="sphere", mode="config", sphere=(128.0, 128.0, 128.0, 20.0), dtype="f16"), 192),
+    ((128, 128, 128), dict(case="cavity", mode="config", storage="aa"), 256),
+    ((32, 32, 32), dict(), 64),
+    ((40, 40, 40), dict(block=448), 448)])
+def test_autotune_times_the_untuned_shape(fake, n, kw, block):
+    """Whatever shape a handle has by default is among those that the tuner times."""
+    fake("""
+    n, kw, block = eval(sys.argv[2])
+    g = LBM(*n, 0.1, **kw)
+    g.Initialize()
+    launches()
+    g.step(2, 0)
+    untuned = launches()[-1][2]
+    assert untuned == block, untuned
+    g.set_launch(320, 1, 1, 1)
+    launches()
+    g.autotune(steps=2)
+    timed = {b for name, _, b in launches() if "k_fused" in name or "k_tiled" in name}
+    assert {64, 128, 256, 512, block} <= timed, timed
+    """, repr((n, kw, block)))
