@@ -350,6 +350,14 @@ static int default_block(const imexlb_handle *h, const LatGeom &g)
     return tile_block((uint64_t)c.nx * c.ny, h->ncell, c.case_id == IMEXLB_CASE_SPHERE && c.dtype == IMEXLB_F16);
 }
 
+// Non-temporal accesses of a layout where set_launch and the tuners name none.
+static int default_ntl(const imexlb_handle *h, const LatGeom &g)
+{
+    const imexlb_config &c = h->cfg;
+    if (c.nt_loads >= 0) return c.nt_loads ? 1 : 0;
+    return g.tl == 31 || tile_nt(lattice_elems(g, (uint32_t)c.nz) * h->elem, c.storage == IMEXLB_AA, h->elem) ? 1 : 0;
+}
+
 // A fused handle's device memory, in its layout.  On failure release() gives back what
 // there is.
 static int allocate(imexlb_handle *h)
@@ -464,7 +472,7 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
     h->block = default_block(h, h->geom);
     h->cpt = c.cells_per_thread ? c.cells_per_thread : 1;
     h->xcd = c.xcd_remap < 0 ? 1 : c.xcd_remap;
-    h->ntl = c.nt_loads < 0 ? 1 : (c.nt_loads ? 1 : 0);
+    h->ntl = default_ntl(h, h->geom);
     // reduced precision stores g_i = f_i - s_i (storage_shift); FP64 stores f itself
     if (c.dtype != IMEXLB_F64) {
         h->shift = c.rho0;
@@ -472,14 +480,12 @@ int imexlb_create(const imexlb_config *cfg, imexlb_handle **out)
         if (c.case_id == IMEXLB_CASE_SPHERE && c.mode == IMEXLB_MODE_CONFIG) h->ush = c.u0;
         storage_shift(h->shift, h->ush, h->sh);
     }
-    if (h->geom.tl != 31 && c.nt_loads < 0)
-        h->ntl = tile_nt(lattice_elems(h->geom, (uint32_t)c.nz) * h->elem, c.storage == IMEXLB_AA, h->elem) ? 1 : 0;
     rc = allocate(h);
     if (rc == IMEXLB_ENOMEM && h->geom.tl != 31) {  // tiles round the planes up: arrays may still fit
         release(h);
         h->geom = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
         h->block = default_block(h, h->geom);
-        h->ntl = c.nt_loads < 0 ? 1 : (c.nt_loads ? 1 : 0);
+        h->ntl = default_ntl(h, h->geom);
         rc = allocate(h);
     }
     if (rc) return bail(rc);
@@ -1098,11 +1104,13 @@ int imexlb_set_launch(imexlb_handle *h, int block, int cpt, int xcd, int ntl)
     return IMEXLB_OK;
 }
 
-// What a placement search times at each place: the handle's layout, and for a
-// lattice in plane tiles beyond the last-level cache also arrays.  Tiles run at nearly
+// What a placement search times at each place: the handle's layout, and for
+// lattices beyond the last-level cache also the other one.  Tiles run at nearly
 // the same rate anywhere, arrays at most places slower but faster at the best
 // (TGV 512^3 AA FP64 over 96 GiB, GLUPS: tiles 13.9-14.1, arrays 12.1-14.7; FP32 28.0-28.4 and
 // 24.5-29.7; FP16 55.6-58.1 and 48.6-57.3), and a search looks for the best place.
+// The handle's own layout comes first; the other takes its defaults where the
+// handle has its own layout's.
 struct Layout {
     LatGeom geom;
     size_t lat_bytes;
@@ -1111,12 +1119,29 @@ struct Layout {
 static std::vector<Layout> layouts_of(const imexlb_handle *h)
 {
     const imexlb_config &c = h->cfg;
+    const bool aa = c.storage == IMEXLB_AA;
     std::vector<Layout> all{{h->geom, h->lat_bytes, h->block, h->ntl}};
-    if (h->geom.tl != 31 && tile_nt(h->lat_bytes, c.storage == IMEXLB_AA, h->elem)) {
-        const LatGeom g = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
-        all.push_back({g, (size_t)(lattice_elems(g, (uint32_t)c.nz) * h->elem), h->block == 192 ? 256 : h->block, h->ntl});
-    }
+    if (c.stride_pad >= 0 || c.addr_mode >= 0 || h->lat_bytes * (aa ? 1 : 2) <= LAST_LEVEL) return all;
+    LatGeom g = soa_geom((uint32_t)c.nx, (uint32_t)c.ny, h->pstride);
+    if (h->geom.tl == 31 && !tile_geom((uint32_t)c.nx, (uint32_t)c.ny, h->elem, aa, g)) return all;
+    all.push_back({g, (size_t)(lattice_elems(g, (uint32_t)c.nz) * h->elem),
+                   h->block == default_block(h, h->geom) ? default_block(h, g) : h->block,
+                   h->ntl == default_ntl(h, h->geom) ? default_ntl(h, g) : h->ntl});
     return all;
+}
+// Those whose lattices leave 2 GiB of `room` bytes free.
+static std::vector<Layout> layouts_in(const std::vector<Layout> &all, size_t nlat, size_t room)
+{
+    std::vector<Layout> fit;
+    for (const Layout &l : all)
+        if (room >= nlat * l.lat_bytes + (2ull << 30)) fit.push_back(l);
+    return fit;
+}
+static size_t most_bytes(const std::vector<Layout> &lay)
+{
+    size_t most = 0;
+    for (const Layout &l : lay) most = std::max(most, l.lat_bytes);
+    return most;
 }
 static void use_layout(imexlb_handle *h, const Layout &l)
 {
@@ -1137,8 +1162,6 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
     steps += steps & 1;  // whole AA periods
     const std::vector<Layout> lay = layouts_of(h);
     const size_t held = h->lat_held;  // by candidate 0
-    size_t most = 0;                  // by the others
-    for (const Layout &l : lay) most = std::max(most, l.lat_bytes);
     const int nlat = h->cfg.storage == IMEXLB_PULL ? 2 : 1;
     // candidate 0 is the current lattice, which may lie in a window
     imx::ChunkedWindow win0 = std::move(h->win);
@@ -1152,11 +1175,15 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
         if (!r) out /= (float)steps;
         return r;
     };
-    std::vector<int> of(trials, 0);  // each candidate's faster layout
+    std::vector<Layout> of(trials, lay[0]);  // each candidate's faster layout
+    std::vector<size_t> bytes(trials, held);
     rc = time_current(ms[0]);
     for (int t = 1; !rc && t < trials; ++t) {
         size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < nlat * most + (2ull << 30)) break;
+        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) break;
+        const std::vector<Layout> fit = layouts_in(lay, (size_t)nlat, free_b);
+        if (fit.empty()) break;
+        const size_t most = bytes[t] = most_bytes(fit);
         std::array<void *, 2> p{nullptr, nullptr};
         bool ok = true;
         for (int k = 0; k < nlat && ok; ++k) ok = hipMalloc(&p[k], most) == hipSuccess;
@@ -1169,13 +1196,13 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
         cand.push_back(p);
         h->lat[0] = p[0];
         h->lat[1] = p[1];
-        for (int l = 0; !rc && l < (int)lay.size(); ++l) {
+        for (size_t l = 0; !rc && l < fit.size(); ++l) {
             float m = 0;
-            use_layout(h, lay[l]);
+            use_layout(h, fit[l]);
             rc = time_current(m);
             if (l == 0 || m < ms[t]) {
                 ms[t] = m;
-                of[t] = l;
+                of[t] = fit[l];
             }
         }
     }
@@ -1196,12 +1223,12 @@ int imexlb_tune_placement(imexlb_handle *h, int trials, int steps, float *ms_per
     }
     h->lat[0] = cand[best][0];
     h->lat[1] = cand[best][1];
-    use_layout(h, lay[of[best]]);
+    use_layout(h, of[best]);
     if (best == 0) {
         h->win = std::move(win0);
     } else {
-        h->device_bytes += (int64_t)nlat * ((int64_t)most - (int64_t)held);
-        h->lat_held = most;
+        h->device_bytes += (int64_t)nlat * ((int64_t)bytes[best] - (int64_t)held);
+        h->lat_held = bytes[best];
     }
     const int rc2 = imexlb_initialize(h);
     if (rc) return rc;
@@ -1227,14 +1254,13 @@ int imexlb_tune_placement_window(imexlb_handle *h, int64_t slack_bytes, int64_t 
     if (rc) return rc;
     if (steps < 2) steps = 2;
     steps += steps & 1;  // whole AA periods
-    const std::vector<Layout> lay = layouts_of(h);
-    size_t most = 0;
-    for (const Layout &l : lay) most = std::max(most, l.lat_bytes);
     const int nlat = h->cfg.storage == IMEXLB_PULL ? 2 : 1;
-    const size_t total = (size_t)nlat * most + (size_t)slack_bytes;
     size_t free_b = 0, total_b = 0;
     HIPCHK(h, hipMemGetInfo(&free_b, &total_b));
-    if (free_b < total + (2ull << 30))
+    const std::vector<Layout> both = layouts_of(h),
+                              lay = layouts_in(both, (size_t)nlat, free_b - std::min(free_b, (size_t)slack_bytes));
+    const size_t total = (size_t)nlat * most_bytes(lay.empty() ? both : lay) + (size_t)slack_bytes;
+    if (lay.empty())
         return fail(h, IMEXLB_ENOMEM, "window of %zu bytes does not fit (%zu free)", total, free_b);
     // one address range in chunks of physical memory: the chunks the kept
     // offset does not use are given back after the search
@@ -1267,7 +1293,7 @@ int imexlb_tune_placement_window(imexlb_handle *h, int64_t slack_bytes, int64_t 
         }
     (void)hipStreamSynchronize(h->stream);
     if (rc) {  // keep the lattice the handle had
-        use_layout(h, lay[0]);
+        use_layout(h, both[0]);
         h->lat[0] = old_lat[0];
         h->lat[1] = old_lat[1];
         imx::window_destroy(w);

@@ -253,7 +253,9 @@ int imexlb_set_launch(imexlb_handle *h, int block, int cells_per_thread, int xcd
  * trials - 1 further lattices while device memory allows (2 GiB stay free),
  * keeping each candidate until the end so that every one has its own pages,
  * times `steps` steps on each with the current launch shape, keeps the
- * fastest and frees the others.  ms_per_step (may be NULL; `trials`
+ * fastest and frees the others.  With stride_pad and addr_mode -1, lattices
+ * beyond the 256 MB last-level cache are timed in plane tiles and in arrays at
+ * each place, and the faster layout is kept with it.  ms_per_step (may be NULL; `trials`
  * entries) receives each candidate's time per step, 0 where none was
  * allocated; *chosen (may be NULL) the index kept, 0 being the original.
  * The state is re-initialised.  Results do not depend on the placement.

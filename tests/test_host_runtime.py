@@ -303,3 +303,80 @@ def test_autotune_times_the_untuned_shape(fake, n, kw, block):
     timed = {b for name, _, b in launches() if "k_fused" in name or "k_tiled" in name}
     assert {64, 128, 256, 512, block} <= timed, timed
     """, repr((n, kw, block)))
+
+
+SEARCHES = {"trials": "g.tune_placement(3, steps=2)", "window": "g.tune_placement_window(4, 2, steps=2)"}
+
+
+@pytest.mark.parametrize("search", SEARCHES)
+def test_placement_searches_try_both_layouts_from_either(fake, search):
+    """A search times tiles and arrays at each place whichever the handle has, keeps the
+    faster one, and accounts for what it holds."""
+    fake("""
+    def faster(part):
+        for p in (b"k_fusedI", b"k_tiled"):
+            F.fake_cost(p, 1e-3 if p == part else 2e-3)
+
+    def kept():
+        launches()
+        g.Initialize()
+        g.step(2, 0)
+        return {name.split("I")[0].split("k_")[1] for name, _, _ in launches() if "k_init" not in name}
+
+    for storage in ("aa", "pull"):
+        g = LBM(200, 200, 100, 0.1, storage=storage)
+        assert kept() == {"tiled"}
+        own = g.info()["block"], g.info()["nt_loads"]
+        for part in (b"k_fusedI", b"k_tiled", b"k_fusedI", b"k_fusedI", b"k_tiled"):
+            faster(part)
+            SEARCH
+            assert kept() == {part.decode()[2:].split("I")[0]}, (storage, part)
+            i = g.info()
+            assert (i["block"], i["nt_loads"]) == (own if part == b"k_tiled" else (256, 1)), i
+            assert 0 <= F.fake_used() - i["device_bytes"] < 1 << 20
+        # the caller's own shape stays
+        g.set_launch(320, 1, 1, 0)
+        faster(b"k_fusedI")
+        SEARCH
+        assert g.info()["block"] == 320 and g.info()["nt_loads"] == 0
+        g.close()
+        assert F.fake_used() == 0
+    """.replace("SEARCH", SEARCHES[search]))
+
+
+@pytest.mark.parametrize("search", SEARCHES)
+def test_placement_searches_of_lattices_in_the_last_level_cache(fake, search):
+    """Their place in HBM hardly counts: the search times the handle's layout only."""
+    fake("""
+    for n in ((32, 32, 32), (40, 40, 40), (64, 64, 64)):
+        g = LBM(*n, 0.1)
+        launches()
+        SEARCH
+        assert not any("k_fused" in name for name, _, _ in launches()), n
+        g.close()
+    """.replace("SEARCH", SEARCHES[search]))
+
+
+@pytest.mark.parametrize("search", SEARCHES)
+def test_placement_searches_with_room_for_arrays_only(fake, search):
+    """Where a further lattice fits in arrays and not in tiles, arrays are searched, as
+    they were before there were tiles."""
+    fake("""
+    F.fake_cost(b"k_fusedI", 1e-3)
+    F.fake_cost(b"k_tiled", 2e-3)
+    n = (97, 41, 3000)
+    g = LBM(*n, 0.1, storage="aa", addr_mode=2)
+    arrays = g.info()["device_bytes"]
+    g.close()
+    g = LBM(*n, 0.1, storage="aa")
+    tiles = g.info()["device_bytes"]
+    assert tiles > arrays * 1.02
+    lattice = arrays - n[0] * n[1] * n[2] * 32
+    F.fake_room(F.fake_used() + lattice + (2 << 30) + (1 << 20) + SLACK)
+    SEARCH
+    assert g.info()["device_bytes"] < tiles + (2 << 30)
+    launches()
+    g.Initialize()
+    g.step(2, 0)
+    assert any("k_fused" in name for name, _, _ in launches())
+    """.replace("SEARCH", SEARCHES[search]).replace("SLACK", "(4 << 30) + (1 << 20)" if search == "window" else "0"))
