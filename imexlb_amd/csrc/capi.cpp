@@ -1008,7 +1008,7 @@ int imexlb_get_info(imexlb_handle *h, imexlb_info *info)
     info->block = h->block;
     info->xcd_remap = h->xcd;
     info->nt_loads = h->ntl;
-    info->addr_mode = h->ph ? -1 : fused_addr_mode(h->elem, h->pstride, c.addr_mode < 0 ? 2 : c.addr_mode);
+    info->addr_mode = h->ph || h->geom.tl != 31 ? -1 : fused_addr_mode(h->elem, h->pstride, c.addr_mode < 0 ? 2 : c.addr_mode);
     info->cells_per_thread = h->ph                  ? h->cpt
                              : h->geom.tl != 31 ? (h->cpt == 2 ? 2 : 1)
                                                 : fused_cells_per_thread(h->cpt, bc_of(c), (uint32_t)c.nx, info->addr_mode);

@@ -299,8 +299,9 @@ struct FusedParams {
     int xcd_remap;           // 1: give each XCD one contiguous run of tiles; plane tiles: tile_order
     int cpt;                 // cells per thread: 1, 2 (blockDim apart) or 3 (two adjacent
                              // x cells; periodic lattices with nx even, else 1)
-    int ntl;                 // 1: non-temporal loads of unshared lines; plane tiles:
-                             // and stores (0: plain)
+    int ntl;                 // 1: non-temporal loads of unshared lines; plane tiles: and
+                             // stores (0: plain; by whole rows stores are always
+                             // non-temporal)
     int am_max;              // widest-saving address mode allowed (AddrMode in fused.h)
     int bc;                  // boundary kind (read by the ensemble kernel)
     FastDiv divx, divy;

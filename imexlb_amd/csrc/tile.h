@@ -357,12 +357,15 @@ __device__ __forceinline__ double lane_shift(double v, double edge)
 
 // The AA odd step on rows that are whole wavefronts (nx a multiple of 64, at
 // most 512): a workgroup is one or more whole rows, every population moves in
-// x-aligned lines, loaded and stored non-temporally, and what crosses into a
-// neighbouring cell in x crosses between lanes (DPP; LDS between wavefronts)
-// instead of through shifted lines.  The shifted form loads a line twice and
+// x-aligned lines, and what crosses into a neighbouring cell in x crosses
+// between lanes (DPP; LDS between wavefronts) instead of through shifted lines.  The shifted form loads a line twice and
 // stores it in two parts, through L2: 5.2 TB/s against 5.9-6.1 for this
 // pattern without arithmetic (TGV 512^3, FP64).  As every row is one
 // wavefront's, its addresses are scalars and one lane offset serves all 27.
+// NT is the loads': stores are non-temporal in both forms (with plain loads too they are
+// faster, us per AA step, non-temporal / plain stores: 512^3 FP64 10490 / 10600, 448x256x256 FP64
+// 2338 / 2343, FP32 1207 / 1200, 512x512x256 FP16 1267 / 1272; non-temporal loads 9590, 2107,
+// 1077, 1161).
 template <typename R>
 struct RowEdges {
     // [wavefront][0: its last lane, e_x = 1; 1: its first lane, e_x = -1][XDIR_P / XDIR_M rank]

@@ -90,7 +90,8 @@ typedef struct imexlb_config {
                                  many bytes between them, a multiple of 256 */
     int32_t nt_loads;         /* -1 = default, 0/1: non-temporal loads of the
                                  lines no other wavefront reads; in plane tiles 0
-                                 also makes the stores plain */
+                                 also makes the stores plain (but for the AA odd
+                                 step by whole rows, which stores non-temporally) */
     int32_t addr_mode;        /* fused kernels' addressing of arrays, the same
                                  results in every mode: -1 = default (the most
                                  compact the lattice allows; see stride_pad), or
@@ -110,7 +111,8 @@ typedef struct imexlb_info {
     int32_t block, cells_per_thread, xcd_remap, nt_loads; /* launch shape; cells per
                                thread as the fused kernels run it (1 where the
                                lattice does not allow the requested 2 or 3) */
-    int32_t addr_mode;      /* the fused kernels' address mode; -1 phased engine */
+    int32_t addr_mode;      /* the address mode of a lattice in arrays; -1: in plane
+                               tiles, or the phased engine */
 } imexlb_info;
 
 /* Defaults: TGV, faithful, fused, FP64, pull, 64^3, tau0 = 0.0153, rho0 = 1,
@@ -235,7 +237,7 @@ int imexlb_bandwidth_probe(int device, int kind, size_t bytes, int reps, double 
 
 /* Launch-shape autotuner (no counterpart in the reference).  Times every
  * workgroup size x cells per thread (1, 2, and 3 where the lattice allows
- * cell pairs) x XCD tile order x load variant on this
+ * cell pairs: arrays, see stride_pad) x XCD tile order x load variant on this
  * handle for `steps` steps each, times the four fastest again (twice each,
  * interleaved, 2 x steps steps), keeps the fastest sum and appends it to the
  * JSON-lines cache at cache_path (NULL: no cache; a cache hit skips the
@@ -244,8 +246,10 @@ int imexlb_bandwidth_probe(int device, int kind, size_t bytes, int reps, double 
  * per thread, XCD order, non-temporal loads.  Fused engine only. */
 int imexlb_autotune(imexlb_handle *h, const char *cache_path, int steps, int32_t *chosen);
 /* Set the launch shape by hand (block 64..512 step 64, cells per thread 1|2|3
- * as imexlb_config.cells_per_thread, XCD order 0|1, non-temporal loads 0|1);
- * results do not depend on it. */
+ * as imexlb_config.cells_per_thread, XCD order 0|1, non-temporal loads 0|1 as
+ * imexlb_config.nt_loads); results do not depend on it.  imexlb_get_info names the
+ * cells per thread in effect: 3 needs arrays (an explicit addr_mode or stride_pad,
+ * or a placement search that kept them) and is 1 in plane tiles. */
 int imexlb_set_launch(imexlb_handle *h, int block, int cells_per_thread, int xcd_order, int nt_loads);
 /* Lattice placement search (no counterpart in the reference).  The step rate
  * of a lattice depends by several percent on where its pages land in HBM,

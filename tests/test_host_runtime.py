@@ -380,3 +380,18 @@ def test_placement_searches_with_room_for_arrays_only(fake, search):
     g.step(2, 0)
     assert any("k_fused" in name for name, _, _ in launches())
     """.replace("SEARCH", SEARCHES[search]).replace("SLACK", "(4 << 30) + (1 << 20)" if search == "window" else "0"))
+
+
+def test_info_names_the_layout(fake):
+    """imexlb_get_info: no address mode in plane tiles, where cells per thread 3 is 1."""
+    fake("""
+    for am, shape, want in ((-1, 1, (-1, 1)), (-1, 2, (-1, 2)), (-1, 3, (-1, 1)), (2, 3, (2, 3)), (1, 3, (1, 1))):
+        for how in ("config", "set_launch"):
+            g = LBM(48, 40, 32, 0.1, addr_mode=am, cells_per_thread=shape if how == "config" else 0)
+            if how == "set_launch":
+                g.set_launch(128, shape, 1, 1)
+            i = g.info()
+            assert (i["addr_mode"], i["cells_per_thread"]) == want, (am, shape, how, i)
+            g.close()
+    assert LBM(48, 40, 32, 0.1, stride_pad=256).info()["addr_mode"] == 2
+    """)
