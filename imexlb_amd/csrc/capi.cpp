@@ -192,6 +192,13 @@ static int validate(const imexlb_config *c)
     return IMEXLB_OK;
 }
 
+static int bc_of(const imexlb_config &c)
+{
+    if (c.case_id == IMEXLB_CASE_TGV) return BC_PERIODIC;
+    if (c.mode == IMEXLB_MODE_FAITHFUL) return BC_FAITHFUL;
+    return c.case_id == IMEXLB_CASE_CAVITY ? BC_CAVITY : BC_CHANNEL;
+}
+
 static void fill_fused_params(imexlb_handle *h, FusedParams &P, int src, int dst)
 {
     const imexlb_config &c = h->cfg;
@@ -206,7 +213,9 @@ static void fill_fused_params(imexlb_handle *h, FusedParams &P, int src, int dst
     P.dst = h->lat[dst];
     P.mask = h->mask;
     P.tau0 = c.tau0;
-    P.inv_den = div_reciprocal(c.tau0 + 0.5);
+    // (the faithful sphere's inlet speed stands in for a moment of populations that div_safe
+    // has looked at: it is held to their range, so that feq stays finite)
+    P.inv_den = bc_of(c) == BC_FAITHFUL && !(std::fabs(c.u0) <= 0x1p400) ? 0.0 : div_reciprocal(c.tau0 + 0.5);
     P.omega_f = (float)(1.0 / (c.tau0 + 0.5));
     P.shift = h->shift;
     P.ush = h->ush;
@@ -244,13 +253,6 @@ hipError_t launch_fused(int dtype, int bc, int pattern, const FusedParams &P, in
     return launch_fused_f16(bc, pattern, P, block, st);
 }
 }  // namespace imx
-
-static int bc_of(const imexlb_config &c)
-{
-    if (c.case_id == IMEXLB_CASE_TGV) return BC_PERIODIC;
-    if (c.mode == IMEXLB_MODE_FAITHFUL) return BC_FAITHFUL;
-    return c.case_id == IMEXLB_CASE_CAVITY ? BC_CAVITY : BC_CHANNEL;
-}
 
 // One fused step: step index k = h->steps + 1.
 static int fused_step(imexlb_handle *h, bool write_moments)
