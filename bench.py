@@ -157,6 +157,12 @@ def vel_l2(a, b):
     return (num / den) ** 0.5
 
 
+def traffic_key(n, storage, info):
+    """The FP64 workload's name in profiles/traffic.json: the arrays' kernels and the
+    plane tiles' move different amounts (imexlb_info.addr_mode is -1 in tiles)."""
+    return f"tgv{n}_{storage}_f64" + ("_tiles" if info["addr_mode"] == -1 else "")
+
+
 def traffic_from_profiles(workload):
     """HBM bytes per launch of the workload's kernel, from the calibrated
     FETCH_SIZE/WRITE_SIZE passes recorded under profiles/ (None if absent)."""
@@ -334,8 +340,7 @@ def main():
     gbps_copy = probes[best_copy]
     log(f"[bench] device copy {gbps_plain:.0f} GB/s plain, {gbps_copy:.0f} GB/s best ({best_copy}); probes "
         + ", ".join(f"{k} {v:.0f}" for k, v in probes.items()))
-    workload = f"tgv{n}_{a.storage}_f64"
-    traffic = traffic_from_profiles(workload)
+    traffic = traffic_from_profiles(traffic_key(n, a.storage, info64))
     cpu = None
     if not a.no_cpu:
         log("[bench] CPU baseline")
@@ -363,7 +368,8 @@ def main():
                      "traffic_source": traffic[2] if traffic else None,
                      "frac_of_measured_copy": achieved / gbps_copy,
                      "bytes_per_lup": bytes_lup, "launch": {k: info64[k] for k in ("block", "cells_per_thread", "xcd_remap", "nt_loads")},
-                     "kernel": "fused step: k_fused over arrays or k_tiled over plane tiles (FP64, periodic, "
+                     "kernel": ("fused step: k_tiled over plane tiles" if info64["addr_mode"] == -1 else
+                                "fused step: k_fused over arrays") + " (FP64, periodic, "
                      + ("AA" if a.storage == "aa" else "pull") + ")",
                      "measured_copy_GBps": gbps_copy, "measured_copy_kernel": best_copy,
                      "bandwidth_probes_GBps": {k: round(v, 1) for k, v in probes.items()},
