@@ -57,12 +57,11 @@ __device__ __forceinline__ double get(const S *lat, const LatGeom &g, int slot, 
 //
 // Bound by its stores.  Over plane tiles workgroups stay within a plane, so that their
 // lines are whole in a tile; over arrays they follow the cells (init_block).  Each XCD
-// writes one run of the lattice.  us, cells in
-// storage order over the whole lattice / this: TGV 301x203x157 FP32 340 / 235, 256^3
-// FP64 832 / 675, 512^3 FP64 6700 / 5400, FP16 3590 / 2450, cavity 100^3 62 / 58;
-// non-temporal stores 198, 626, 5490, 2440, 68.  The solid cells of the other
-// lattice are written here rather than by a copy of the whole: Initialize of the sphere
-// 512x128x128 1198 -> 383, channel 512x256x256 FP16 1490 -> 640.
+// writes one run of the lattice.  us, the kernel over arrays in the cells' order / this:
+// TGV 301x203x157 FP32 240 / 240, 256^3 FP64 735 / 690, 512^3 FP64 5840 / 5500, FP16 2400 / 2690,
+// cavity 100^3 33 / 33, sphere 512x128x128 377 / 372, channel 512x256x256 FP16 537 / 665 (10 % more or
+// less with the allocation).  The solid cells of the sphere's other lattice are written
+// here rather than by a copy of the whole, another 770 in both.
 template <typename S>
 __global__ void k_init(const InitParams P)
 {

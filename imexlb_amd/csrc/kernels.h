@@ -178,6 +178,10 @@ inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, bool aa, LatGeom 
 //   them are resident, four to a SIMD (12x12x694 FP32 pull 6.31 / 5.41, 10x13x769 FP32 AA
 //   5.76 / 5.79, 9x8x1389 FP16 AA 4.97 / 6.01), more beyond (FP16 AA of 4e5 cells: 16x16
 //   10.2 / 10.0, 12x12 10.3 / 10.6, 10x13 10.5 / 11.7, 9x8 10.6 / 14.0).
+// The rule leaves out, for want of a cause: FP64 pull of 36 to 46 MiB with a quarter
+// or more of the lanes idle (12x12x700 9.4 / 10.4) and the config cavity's AA beyond the
+// last-level cache with planes of 20x20, 24x24 and 40x40 (FP32 20x20x15000 242 / 257; 16x16
+// 240 / 220).
 // At other sizes tiles serve: TGV 8^3 FP64 5.6 / 4.1, 16^3 5.86 / 4.17, FP32 4.12 / 3.19, FP16 AA
 // 3.88 / 3.15, 9x13x30 FP64 5.88 / 4.15, 22x18x22 6.03 / 4.32, faithful cavity 16^3 10.1 / 8.8.
 constexpr uint64_t LAST_LEVEL = uint64_t(256) << 20;
@@ -210,8 +214,9 @@ inline int tile_order(uint64_t lattice_bytes, bool aa)
 // 67.3 / 72.0; AA FP64 64^3 20.4 / 18.8, 96^3 59.6 / 56.1, 128^3 (453 MB) 138 / 161, FP32
 // 128^3 66.2 / 63.9, FP16 128^3 40.1 / 34.2.
 //
-// FP64 pull lattices of about the L2s' 32 MB stay non-temporal (32^3 5.34 / 5.31, 36^3
-// 5.79 / 6.09, 40^3 6.38 / 7.18, 44^3 8.21 / 8.95, 48^3 10.14 / 10.24, 52^3 14.7 / 12.1).
+// FP64 pull lattices of about the L2s' 32 MB stay non-temporal: a bracket that the
+// measurements draw, whose cause (why it ends between 44^3 and 52^3, where the pair
+// leaves the L2s) is not known (32^3 5.34 / 5.31, 36^3 5.79 / 6.09, 40^3 6.38 / 7.18, 44^3 8.21 / 8.95, 48^3 10.14 / 10.24, 52^3 14.7 / 12.1).
 inline bool tile_nt(uint64_t lattice_bytes, bool aa, uint64_t elem)
 {
     const uint64_t bytes = aa ? lattice_bytes : 2 * lattice_bytes, mib = uint64_t(1) << 20;
@@ -223,7 +228,8 @@ inline bool tile_nt(uint64_t lattice_bytes, bool aa, uint64_t elem)
 // larger workgroups (us per step, 64 / 256: TGV 24^3 FP64 AA 4.9 / 5.8, 32^3 5.7 / 6.3, 40^3
 // 7.4 / 9.0, 56^3 14.5 / 14.8, 64^3 20.3 / 20.3 and FP16 7.0 / 6.8); above, the largest of
 // 256, 128 and 64 that leaves at most a sixteenth of the plane's threads idle, else
-// the one that leaves the fewest.  192 for the FP16 channel (`channel_f16`) once its two
+// the one that leaves the fewest.  192, from measurements alone (no cause is known), for
+// the FP16 channel (`channel_f16`) once its two
 // lattices exceed the 256 MB last-level cache: us per step, 128 / 192 / 256, 512x256x256
 // 650 / 605 / 655, 448x288x184 443 / 426 / 430, 640x256x160 483 / 469 / 477, 512x256x128
 // 318 / 299 / 315, 678x246x190 600 / 577 / 589, 300x150x150 129 / 125 / 128, 384x192x192
