@@ -177,7 +177,8 @@ inline bool tile_geom(uint32_t nx, uint32_t ny, uint64_t elem, bool aa, LatGeom 
 //   (13x5x308 FP32 pull 4.23 / 3.97, 9x8x278 FP64 pull 6.22 / 6.21), few while all of
 //   them are resident, four to a SIMD (12x12x694 FP32 pull 6.31 / 5.41, 10x13x769 FP32 AA
 //   5.76 / 5.79, 9x8x1389 FP16 AA 4.97 / 6.01), more beyond (FP16 AA of 4e5 cells: 16x16
-//   10.2 / 10.0, 12x12 10.3 / 10.6, 10x13 10.5 / 11.7, 9x8 10.6 / 14.0).
+//   10.2 / 10.0, 12x12 10.3 / 10.6, 10x13 10.5 / 11.7, 9x8 10.6 / 14.0); both count just
+//   beyond them (FP64 pull 43 MB, 13x5x1538 9.9 / 11.8, 9x8x1389 9.6 / 11.2).
 // The rule leaves out, for want of a cause: FP64 pull of 36 to 46 MiB with a quarter
 // or more of the lanes idle (12x12x700 9.4 / 10.4) and the config cavity's AA beyond the
 // last-level cache with planes of 20x20, 24x24 and 40x40 (FP32 20x20x15000 242 / 257; 16x16
